@@ -2,97 +2,39 @@
 // and per-row sorting.  These are not the hot path; they are written for
 // correctness with coalesced access and no host round trips.
 #include "dev_common.h"
+#include "scan.h"
 #include "tr_internal.h"
 
 namespace tr {
+
+namespace scan {
+
+__global__ __launch_bounds__(1024) void k_scan_tiles(int64_t *__restrict__ sums, int64_t ntiles) {
+    __shared__ int64_t tot[1024 / kWave];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    int64_t carry = 0;
+    for (int64_t base = 0; base < ntiles; base += 1024) {
+        const int64_t i = base + threadIdx.x;
+        const int64_t v = i < ntiles ? sums[i] : 0;
+        const int64_t inc = wave_incl_scan(v);
+        if (lane_id() == kWave - 1) tot[w] = inc;
+        __syncthreads();
+        int64_t off = carry;
+#pragma unroll
+        for (int u = 0; u < 1024 / kWave; ++u) {
+            off += u < w ? tot[u] : 0;
+            carry += tot[u];
+        }
+        if (i < ntiles) sums[i] = off + inc - v;
+        __syncthreads();
+    }
+}
+
+}  // namespace scan
+
 namespace {
 
 using namespace dev;
-
-constexpr int kScanThreads = 256;
-constexpr int kScanItems = 16;
-constexpr int kScanTile = kScanThreads * kScanItems;
-
-template <typename Tin>
-__global__ void k_scan_reduce(const Tin *__restrict__ in, int64_t n, int64_t *__restrict__ tile_sums) {
-    __shared__ int64_t wsum[kScanThreads / kWave];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    int64_t s = 0;
-    for (int t = 0; t < kScanItems; ++t) {
-        int64_t i = base + (int64_t)t * kScanThreads + threadIdx.x;
-        if (i < n) s += (int64_t)in[i];
-    }
-    s = wave_sum(s);
-    if (lane_id() == 0) wsum[threadIdx.x / kWave] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int64_t tot = 0;
-        for (int w = 0; w < kScanThreads / kWave; ++w) tot += wsum[w];
-        tile_sums[blockIdx.x] = tot;
-    }
-}
-
-// Exclusive scan of the tile sums in place, single block; writes the grand
-// total to *total.
-__global__ void k_scan_tiles(int64_t *__restrict__ sums, int64_t ntiles, int64_t *__restrict__ total) {
-    __shared__ int64_t wsum[kScanThreads / kWave];
-    __shared__ int64_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int64_t base = 0; base < ntiles; base += kScanThreads) {
-        int64_t i = base + threadIdx.x;
-        int64_t v = i < ntiles ? sums[i] : 0;
-        int64_t inc = wave_incl_scan(v);
-        if (lane_id() == kWave - 1) wsum[threadIdx.x / kWave] = inc;
-        __syncthreads();
-        int64_t off = carry;
-        for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) off += wsum[w];
-        if (i < ntiles) sums[i] = off + inc - v;
-        __syncthreads();
-        if (threadIdx.x == kScanThreads - 1) carry = off + inc;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *total = carry;
-}
-
-template <typename Tin>
-__global__ void k_scan_apply(const Tin *__restrict__ in, int64_t n, const int64_t *__restrict__ tile_off,
-                             int64_t *__restrict__ out) {
-    __shared__ int64_t wsum[kScanThreads / kWave];
-    __shared__ int64_t carry;
-    const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    if (threadIdx.x == 0) carry = tile_off[blockIdx.x];
-    __syncthreads();
-    for (int t = 0; t < kScanItems; ++t) {
-        int64_t i = base + (int64_t)t * kScanThreads + threadIdx.x;
-        int64_t v = i < n ? (int64_t)in[i] : 0;
-        int64_t inc = wave_incl_scan(v);
-        if (lane_id() == kWave - 1) wsum[threadIdx.x / kWave] = inc;
-        __syncthreads();
-        int64_t off = carry;
-        for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) off += wsum[w];
-        if (i < n) out[i] = off + inc - v;
-        __syncthreads();
-        if (threadIdx.x == kScanThreads - 1) carry = off + inc;
-        __syncthreads();
-    }
-}
-
-__global__ void k_store0_i64(int64_t *p) { *p = 0; }
-
-template <typename Tin>
-void scan_impl(tr_ctx *ctx, const Tin *in, int64_t *out, int64_t n, int64_t *tmp) {
-    // out[0..n] = exclusive prefix, out[n] = total
-    int64_t ntiles = (n + kScanTile - 1) / kScanTile;
-    if (ntiles == 0) {
-        TR_LAUNCH(ctx, "scan_empty", k_store0_i64, 1, 1, 0, out);
-        return;
-    }
-    int64_t *sums = tmp ? tmp : (int64_t *)scratch(ctx, S_SCAN_TMP, sizeof(int64_t) * (size_t)ntiles);
-    TR_LAUNCH(ctx, "scan_reduce", k_scan_reduce<Tin>, (uint32_t)ntiles, kScanThreads, 0, in, n, sums);
-    TR_LAUNCH(ctx, "scan_tiles", k_scan_tiles, 1, kScanThreads, 0, sums, ntiles, out + n);
-    TR_LAUNCH(ctx, "scan_apply", k_scan_apply<Tin>, (uint32_t)ntiles, kScanThreads, 0, in, n, sums, out);
-}
 
 // plain streaming copy, 16 bytes per lane per iteration (counter calibration)
 __global__ void k_copy16(const uint4 *__restrict__ src, uint4 *__restrict__ dst, int64_t n16) {
@@ -279,12 +221,12 @@ __global__ void k_sort_classify(const int32_t *__restrict__ ptr, int32_t m, int3
 
 }  // namespace
 
-size_t scan_tmp_bytes(int64_t n) { return sizeof(int64_t) * (size_t)((n + kScanTile - 1) / kScanTile + 1); }
+size_t scan_tmp_bytes(int64_t n) { return sizeof(int64_t) * (size_t)(scan::tiles(n) + 1); }
 void launch_exclusive_scan_i64(tr_ctx *ctx, const int64_t *in, int64_t *out, int64_t n, int64_t *tmp) {
-    scan_impl<int64_t>(ctx, in, out, n, tmp);
+    scan::launch(ctx, scan::ArrayIn<int64_t>{in}, out, n, tmp);
 }
 void launch_exclusive_scan_i32_to_i64(tr_ctx *ctx, const int32_t *in, int64_t *out, int64_t n, int64_t *tmp) {
-    scan_impl<int32_t>(ctx, in, out, n, tmp);
+    scan::launch(ctx, scan::ArrayIn<int32_t>{in}, out, n, tmp);
 }
 
 void launch_copy16(tr_ctx *ctx, void *dst, const void *src, size_t bytes) {
