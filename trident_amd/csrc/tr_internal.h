@@ -205,9 +205,25 @@ void launch_rowptr_i64_to_i32(tr_ctx *ctx, const int64_t *rp64, int32_t r0, int3
 void launch_bitmask_gen(tr_ctx *ctx, const int32_t *ptr, int32_t n, uint64_t *mask);
 void launch_bitmask_and(tr_ctx *ctx, const uint64_t *a, const uint64_t *b, int32_t words, uint64_t *out);
 int64_t compress(tr_ctx *ctx, const tr_csx_t *m, const uint64_t *mask, tr_csx_t *out);
-void launch_compress_fixed(tr_ctx *ctx, int32_t n, const int32_t *ptr, const int32_t *idx, const double *val,
-                           int64_t nnz_in, const uint64_t *mask, int32_t *kept_tmp, int64_t *np64, int64_t *scan_tmp,
-                           int32_t *optr, int32_t *oidx, double *oval);
+// One tile of an entry filter: keeps the entries of segments whose mask bit is
+// set, or (by_index) the entries whose index is set in a mask of nmask bits,
+// into arrays with room for cap entries.  A segment mask is bits or (bytes) a
+// byte per segment.  tile0: the job's first work unit in its launch.
+struct FilterJob {
+    const int32_t *ptr, *idx;
+    const double *val;
+    const uint64_t *mask;
+    int32_t *optr, *oidx;
+    double *oval;
+    int64_t nnz, cap;
+    int32_t n, nmask, by_index, bytes, tile0, pad;
+};
+constexpr int kFilterTile = 2048;  // segments plus entries per work unit
+int32_t filter_tiles(int32_t n, int64_t nnz);
+void launch_filter_count(tr_ctx *ctx, const FilterJob *jobs, int njobs, const FilterJob &one, int32_t ntiles,
+                         int32_t *counts, int64_t *first, int64_t *scan_tmp);
+void launch_filter_write(tr_ctx *ctx, const FilterJob *jobs, int njobs, const FilterJob &one, int32_t ntiles,
+                         const int64_t *first);
 
 // k_spgemm.hip
 void validate_operands(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B);
