@@ -1,5 +1,5 @@
-// Utility kernels of libtrident_hip: scans, CSR validation, transposition
-// and per-row sorting.  These are not the hot path; they are written for
+// Utility kernels of libtrident_hip: scans, CSR validation and
+// per-row sorting.  These are not the hot path; they are written for
 // correctness with coalesced access and no host round trips.
 #include "dev_common.h"
 #include "scan.h"
@@ -81,34 +81,6 @@ __global__ void k_validate_idx(const int32_t *__restrict__ idx, int64_t nnz, int
         }
     }
     if (flags) atomicOr(status, flags);
-}
-
-// ---- transpose ----
-__global__ void k_count_cols(const int32_t *__restrict__ idx, int64_t nnz, int32_t *__restrict__ cnt) {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; p < nnz; p += stride) atomicAdd(&cnt[idx[p]], 1);
-}
-
-__global__ void k_i64_to_i32(const int64_t *__restrict__ in, int64_t n, int32_t *__restrict__ out) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) out[i] = (int32_t)in[i];
-}
-
-// one wave per source segment; scatter entries to their destination
-// segments through per-segment cursors (order fixed afterwards by sorting)
-__global__ void k_transpose_scatter(const int32_t *__restrict__ ptr, const int32_t *__restrict__ idx,
-                                    const double *__restrict__ val, int32_t P, int32_t *__restrict__ cursor,
-                                    int32_t *__restrict__ oidx, double *__restrict__ oval) {
-    int32_t seg = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-    if (seg >= P) return;
-    for (int32_t p = ptr[seg] + lane_id(); p < ptr[seg + 1]; p += kWave) {
-        int32_t c = idx[p];
-        int32_t q = atomicAdd(&cursor[c], 1);
-        oidx[q] = seg;
-        oval[q] = val[p];
-    }
 }
 
 __global__ void k_rowptr_rebase(const int64_t *__restrict__ rp, int32_t r0, int32_t n, int32_t *__restrict__ o) {
@@ -297,29 +269,6 @@ void launch_sort_rows(tr_ctx *ctx, tr_csx_t *m) {
                       vcopy, lists + 2 * (int64_t)P + t, 1, g, g + N, N);
         }
     }
-}
-
-// out receives the segments of m's other dimension (for a CSR m: the CSR of
-// m^T); its descriptor and storage are prepared by the caller.
-void launch_transpose(tr_ctx *ctx, const tr_csx_t *m, tr_csx_t *out) {
-    const int32_t P = ptrdim(m), O = otherdim(m);
-    int32_t *cnt = (int32_t *)scratch(ctx, S_MISC, sizeof(int32_t) * ((size_t)O + 1));
-    TR_HIP(hipMemsetAsync(cnt, 0, sizeof(int32_t) * ((size_t)O + 1), ctx->stream));
-    if (m->nnz > 0) {
-        uint32_t g = (uint32_t)std::min<int64_t>((m->nnz + 255) / 256, 16384);
-        TR_LAUNCH(ctx, "transpose_count", k_count_cols, g, 256, 0, m->idx_vec, m->nnz, cnt);
-    }
-    int64_t *off = (int64_t *)scratch(ctx, S_ROWPTR64, sizeof(int64_t) * ((size_t)O + 1));
-    launch_exclusive_scan_i32_to_i64(ctx, cnt, off, O);
-    TR_LAUNCH(ctx, "i64_to_i32", k_i64_to_i32, div_up((uint64_t)O + 1, 256), 256, 0, off, (int64_t)O + 1,
-              out->ptr_vec);
-    // cursors start at the segment offsets
-    TR_HIP(hipMemcpyAsync(cnt, out->ptr_vec, sizeof(int32_t) * (size_t)O, hipMemcpyDeviceToDevice, ctx->stream));
-    if (m->nnz > 0) {
-        TR_LAUNCH(ctx, "transpose_scatter", k_transpose_scatter, div_up((uint64_t)P, 4), 256, 0, m->ptr_vec,
-                  m->idx_vec, m->val, P, cnt, out->idx_vec, out->val);
-    }
-    launch_sort_rows(ctx, out);
 }
 
 }  // namespace tr
