@@ -140,21 +140,6 @@ void *scratch(tr_ctx *ctx, int slot, size_t bytes) {
     return ctx->scratch_ptr[slot];
 }
 
-void *pinned(tr_ctx *ctx, size_t bytes) {
-    if (ctx->pinned_size < bytes) {
-        if (ctx->pinned) {
-            TR_HIP(hipStreamSynchronize(ctx->stream));
-            (void)hipHostFree(ctx->pinned);
-            ctx->pinned = nullptr;
-            ctx->pinned_size = 0;
-        }
-        size_t want = std::max<size_t>(bytes, 4096);
-        TR_HIP(hipHostMalloc(&ctx->pinned, want, hipHostMallocDefault));
-        ctx->pinned_size = want;
-    }
-    return ctx->pinned;
-}
-
 void read_array(tr_ctx *ctx, void *host, const void *dptr, size_t bytes) {
     if (bytes == 0) return;
     TR_HIP(hipMemcpyAsync(host, dptr, bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -241,17 +226,19 @@ void release_csx(tr_ctx *ctx, tr_csx_t *m) {
     std::memset(m, 0, sizeof(*m));
 }
 
-// Device validation of one operand; fails with TR_ERR_INVALID on a malformed
-// pointer or an out-of-range index (and on unsorted rows if need_sorted).
-static void require_valid(tr_ctx *ctx, const tr_csx_t *m, const char *what, bool need_sorted) {
-    int32_t *st = (int32_t *)scratch(ctx, S_PANELS, 64);
-    TR_HIP(hipMemsetAsync(st, 0, sizeof(int32_t), ctx->stream));
-    launch_validate(ctx, m, st);
-    int32_t hs = 0;
-    read_array(ctx, &hs, st, sizeof(hs));
+// Fails with TR_ERR_INVALID on what the checks of tile `what` found: a
+// malformed pointer, an out-of-range index (and unsorted segments if
+// need_sorted).
+static void require_status(int32_t hs, const char *what, bool need_sorted) {
     if (hs & 1) fail(TR_ERR_INVALID, std::string(what) + ": malformed pointer array");
     if (hs & 2) fail(TR_ERR_INVALID, std::string(what) + ": index out of range");
     if (need_sorted && (hs & 4)) fail(TR_ERR_INVALID, std::string(what) + ": unsorted or duplicate indices");
+}
+
+static void require_valid(tr_ctx *ctx, const tr_csx_t *m, const char *what, bool need_sorted) {
+    int32_t hs = 0;
+    check_tiles(ctx, &m, 1, &hs);
+    require_status(hs, what, need_sorted);
 }
 
 static bool ctx_owned(tr_ctx *ctx, const tr_csx_t *m) {
@@ -358,7 +345,9 @@ int tr_ctx_create(tr_ctx_t *out, int device, void *hip_stream) {
         hipDeviceProp_t prop;
         TR_HIP(hipGetDeviceProperties(&prop, device));
         ctx->cu_count = prop.multiProcessorCount;
-        (void)pinned(ctx, 4096);  // staging of scalar reads, so later calls need no host allocation
+        TR_HIP(hipHostMalloc(&ctx->pinned, kPinnedBytes, hipHostMallocDefault));
+        std::memset(ctx->pinned, 0, kPinnedBytes);
+        ctx->status = (uint8_t *)ctx->pinned + kPinnedValues;
         noalloc_init(device);     // device address of the allocation-free entry points' scratch
     });
     if (rc != TR_OK) {
@@ -441,12 +430,9 @@ static void require_add_operands(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t 
     check_csx(C, "C");
     TR_REQUIRE(A->majordim == TR_ROWS && C->majordim == TR_ROWS, w + ": operands must be CSR");
     TR_REQUIRE(A->nrows == C->nrows && A->ncols == C->ncols, w + ": shape mismatch");
-    int32_t *st = (int32_t *)scratch(ctx, S_PANELS, 64);
-    TR_HIP(hipMemsetAsync(st, 0, 2 * sizeof(int32_t), ctx->stream));
-    launch_validate(ctx, A, st);
-    launch_validate(ctx, C, st + 1);
+    const tr_csx_t *m[2] = {A, C};
     int32_t hs[2];
-    read_array(ctx, hs, st, sizeof(hs));
+    check_tiles(ctx, m, 2, hs);
     if ((hs[0] | hs[1]) & 3) fail(TR_ERR_INVALID, w + ": malformed CSR operand");
     if ((hs[0] | hs[1]) & 4) fail(TR_ERR_INVALID, w + ": operands need sorted unique columns");
 }
@@ -667,10 +653,7 @@ int tr_csx_validate(tr_ctx_t ctx, const tr_csx_t *M, int32_t *status) {
     return guarded(ctx, [&] {
         check_csx(M, "M");
         TR_REQUIRE(status != nullptr, "tr_csx_validate: null status");
-        int32_t *st = (int32_t *)scratch(ctx, S_PANELS, 64);
-        TR_HIP(hipMemsetAsync(st, 0, sizeof(int32_t), ctx->stream));
-        launch_validate(ctx, M, st);
-        read_array(ctx, status, st, sizeof(int32_t));
+        check_tiles(ctx, &M, 1, status);
     });
 }
 

@@ -17,6 +17,7 @@
 // list and output), then captures the same launch sequence, with every size
 // fixed, into a hipGraph; tr_batch_run replays it with no host round trip.
 // Inputs are borrowed and must not change shape between plan and run.
+#include "csr_units.h"
 #include "dev_common.h"
 #include "tr_internal.h"
 #include "spgemm_types.h"
@@ -280,7 +281,7 @@ void batch_compress_plan(tr_batch *b) {
         f.by_index = by_index ? 1 : 0;
         f.bytes = by_index ? 0 : 1;
         f.tile0 = (int32_t)tiles;
-        tiles += filter_tiles(m.nrows, m.nnz);
+        tiles += unit_count(m.nrows, m.nnz);
         TR_REQUIRE(tiles < INT32_MAX, "batch: too many compression work units");
         fj.push_back(f);
         mask_id.push_back(mask);
@@ -478,11 +479,9 @@ int tr::batch_create(tr_ctx_t ctx, int32_t ntasks, const tr_csx_t *A, const tr_c
                 check_csx(&C, "C_in");
                 TR_REQUIRE(C.majordim == TR_ROWS && C.nrows == b->A[t].nrows && C.ncols == b->B[t].ncols,
                            "tr_batch_create: accumulator shape mismatch");
-                int32_t *st = (int32_t *)scratch(ctx, S_TMP_CSX, 64);
-                TR_HIP(hipMemsetAsync(st, 0, sizeof(int32_t), ctx->stream));
-                launch_validate(ctx, &C, st);
+                const tr_csx_t *pc = &C;
                 int32_t hs = 0;
-                read_array(ctx, &hs, st, sizeof(hs));
+                check_tiles(ctx, &pc, 1, &hs);
                 TR_REQUIRE(hs == 0, "tr_batch_create: accumulator is not a sorted CSR");
             }
             max_m = std::max(max_m, b->A[t].nrows);
@@ -502,6 +501,8 @@ int tr::batch_create(tr_ctx_t ctx, int32_t ntasks, const tr_csx_t *A, const tr_c
             T = TaskDev{};
             T.m = a.nrows;
             T.n = bb.ncols;
+            T.k = a.ncols;
+            T.a_cap = a.nnz;
             if (compress_mode) {
                 BatchOperand &ac = b->Ac[t], &bc = b->Bc[t];
                 ac.optr = (int32_t *)b->own(sizeof(int32_t) * ((size_t)a.nrows + 1));

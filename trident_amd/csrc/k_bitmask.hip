@@ -10,8 +10,7 @@
 // a tile into units of equal segments plus entries; there is no per-entry
 // binary search over the pointer array and values and indices move in the
 // same pass.
-#include <algorithm>
-
+#include "csr_units.h"
 #include "dev_common.h"
 #include "tr_internal.h"
 
@@ -37,43 +36,21 @@ __global__ void k_bitmask_and(const uint64_t *__restrict__ a, const uint64_t *__
 // ---- entry filter ----
 // Keeps a subset of a tile's entries in their order: those of masked segments
 // (Compress; the B side of a stage) or those whose index is masked (the A
-// side).  A tile is cut into work units of kFilterTile steps of the merge of
-// its segment ends with its entries, so a unit has at most kFilterTile
-// segments and kFilterTile entries whatever the segment lengths are: one wave
-// per 64 segments, the split before, left the hub segments of an R-MAT to one
-// wave (2^18 segments, 4 M entries: 1110 us a tile; now 9 us to count, 23 us
-// to write 90 MB at about 4 TB/s).  A unit's kept
-// entries are 64-entry bit words in LDS, from which every entry's place and
-// every segment's new start are a popcount away.  Pass 1 counts per unit, a
-// scan over the units gives their first output entry, pass 2 writes.
-// Jobs of one launch come from a table, or as one job by value (njobs == 0).
-constexpr int kFilterThreads = 256;
-constexpr int kFilterWords = kFilterTile / 64;
-
-// Number of segment ends among the first d steps of the merge (segment r's
-// end comes before entry ptr[r + 1]), searched 64 probes at a time.  The
-// result lies in [max(0, d - nnz), min(d, n)] whatever ptr holds.
-__device__ __forceinline__ int32_t merge_rows(const int32_t *__restrict__ ptr, int32_t n, int64_t nnz, int64_t d) {
-    int64_t lo = d > nnz ? d - nnz : 0, hi = d < n ? d : n;
-    while (lo < hi) {
-        const int64_t step = (hi - lo + kWave - 1) / kWave;
-        const int64_t mid = lo + lane_id() * step;
-        const bool past = mid < hi && (int64_t)ptr[mid + 1] <= d - 1 - mid;
-        const int c = __popcll(ballot(past));
-        if (c == 0) break;
-        const int64_t up = lo + c * step;
-        lo = up - step + 1;
-        hi = up < hi ? up : hi;
-    }
-    return (int32_t)lo;
-}
+// side).  A workgroup takes one work unit (csr_units.h): one wave per 64
+// segments, the split before, left the hub segments of an R-MAT to one wave
+// (2^18 segments, 4 M entries: 1110 us a tile; now 9 us to count, 23 us to
+// write 90 MB at about 4 TB/s).  A unit's kept entries are 64-entry bit words
+// in LDS, from which every entry's place and every segment's new start are a
+// popcount away.  Pass 1 counts per unit, a scan over the units gives their
+// first output entry, pass 2 writes.  Jobs of one launch come from a table, or
+// as one job by value (njobs == 0).
 
 template <bool kWrite>
-__global__ __launch_bounds__(kFilterThreads) void k_filter(const FilterJob *__restrict__ jobs, int njobs,
+__global__ __launch_bounds__(kUnitThreads) void k_filter(const FilterJob *__restrict__ jobs, int njobs,
                                                            const FilterJob one, int32_t *__restrict__ counts,
                                                            const int64_t *__restrict__ first) {
-    __shared__ unsigned long long bits[kFilterWords];
-    __shared__ int32_t before[kFilterWords];
+    __shared__ unsigned long long bits[kUnitWords];
+    __shared__ int32_t before[kUnitWords];
     __shared__ int32_t split[2];
     const int tid = threadIdx.x, l = lane_id(), w = __builtin_amdgcn_readfirstlane(tid / kWave);
     int lo = 0, hi = njobs - 1;
@@ -84,20 +61,12 @@ __global__ __launch_bounds__(kFilterThreads) void k_filter(const FilterJob *__re
     }
     const FilterJob J = njobs ? jobs[lo] : one;
     const int32_t unit = (int32_t)blockIdx.x - J.tile0;
-    const int64_t steps = (int64_t)J.n + J.nnz;
-    const int64_t d0 = min((int64_t)unit * kFilterTile, steps), d1 = min(d0 + kFilterTile, steps);
-    if (w < 2) {
-        const int32_t i = merge_rows(J.ptr, J.n, J.nnz, w ? d1 : d0);
-        if (l == 0) split[w] = i;
-    }
-    if (tid < kFilterWords) bits[tid] = 0ull;
-    __syncthreads();
-    // segments whose end lies in the unit: [i0, i1); entries [j0, j0 + len)
-    const int32_t i0 = split[0], i1 = split[1];
-    const int64_t j0 = d0 - i0;
-    const int32_t len = (int32_t)(d1 - i1 - j0);
+    if (tid < kUnitWords) bits[tid] = 0ull;
+    const Unit U = find_unit(J.ptr, J.n, J.nnz, unit, split);
+    const int32_t i0 = U.i0, i1 = U.i1, len = U.len;
+    const int64_t j0 = U.j0;
     if (J.by_index) {
-        for (int u = w; u < kFilterWords; u += kFilterThreads / kWave) {
+        for (int u = w; u < kUnitWords; u += kUnitThreads / kWave) {
             const int32_t x = u * 64 + l;
             bool keep = false;
             if (x < len) {
@@ -109,7 +78,7 @@ __global__ __launch_bounds__(kFilterThreads) void k_filter(const FilterJob *__re
         }
     } else {
         // segment i1's end lies beyond the unit, some of its entries may not
-        for (int32_t i = i0 + tid; i <= i1 && i < J.n; i += kFilterThreads) {
+        for (int32_t i = i0 + tid; i <= i1 && i < J.n; i += kUnitThreads) {
             if (!(J.bytes ? ((const uint8_t *)J.mask)[i] : ((J.mask[i >> 6] >> (i & 63)) & 1ull))) continue;
             const int32_t x0 = (int32_t)max((int64_t)J.ptr[i] - j0, (int64_t)0);
             const int32_t x1 = (int32_t)min((int64_t)J.ptr[i + 1] - j0, (int64_t)len);
@@ -122,39 +91,39 @@ __global__ __launch_bounds__(kFilterThreads) void k_filter(const FilterJob *__re
     }
     __syncthreads();
     if (w == 0) {
-        const int32_t c = l < kFilterWords ? __popcll(bits[l]) : 0;
+        const int32_t c = l < kUnitWords ? __popcll(bits[l]) : 0;
         const int32_t inc = wave_incl_scan(c);
-        if (l < kFilterWords) before[l] = inc - c;
+        if (l < kUnitWords) before[l] = inc - c;
         if (!kWrite && l == kWave - 1) counts[blockIdx.x] = inc;
     }
     if constexpr (kWrite) {
         __syncthreads();
         const int64_t base = first[blockIdx.x] - first[J.tile0];
         auto place = [&](int32_t x) {  // kept entries of the unit before its entry x
-            if (x >= kFilterTile) return before[kFilterWords - 1] + __popcll(bits[kFilterWords - 1]);
+            if (x >= kUnit) return before[kUnitWords - 1] + __popcll(bits[kUnitWords - 1]);
             return before[x >> 6] + __popcll(bits[x >> 6] & ((1ull << (x & 63)) - 1ull));
         };
-        for (int32_t i = i0 + tid; i < i1; i += kFilterThreads) {
+        for (int32_t i = i0 + tid; i < i1; i += kUnitThreads) {
             const int64_t x = (int64_t)J.ptr[i + 1] - j0;
             J.optr[i + 1] = (int32_t)(base + place((int32_t)min(max(x, (int64_t)0), (int64_t)len)));
         }
         if (unit == 0 && tid == 0) J.optr[0] = 0;
-        if (before[kFilterWords - 1] + __popcll(bits[kFilterWords - 1]) == 0) return;  // block-uniform
+        if (before[kUnitWords - 1] + __popcll(bits[kUnitWords - 1]) == 0) return;  // block-uniform
         // all loads before the first store; a dropped entry's lane reads the
         // unit's first entry, which exists
-        constexpr int kPer = kFilterTile / kFilterThreads;
+        constexpr int kPer = kUnit / kUnitThreads;
         int32_t ci[kPer];
         double cv[kPer];
 #pragma unroll
         for (int t = 0; t < kPer; ++t) {
-            const int32_t x = t * kFilterThreads + tid;
+            const int32_t x = t * kUnitThreads + tid;
             const int64_t p = j0 + (((bits[x >> 6] >> (x & 63)) & 1ull) ? x : 0);
             ci[t] = J.idx[p];
             cv[t] = J.val[p];
         }
 #pragma unroll
         for (int t = 0; t < kPer; ++t) {
-            const int32_t x = t * kFilterThreads + tid;
+            const int32_t x = t * kUnitThreads + tid;
             if (!((bits[x >> 6] >> (x & 63)) & 1ull)) continue;
             const int64_t q = base + place(x);
             if (q < J.cap) {
@@ -177,22 +146,17 @@ void launch_bitmask_and(tr_ctx *ctx, const uint64_t *a, const uint64_t *b, int32
     TR_LAUNCH(ctx, "bitmask_and", k_bitmask_and, div_up((uint64_t)words, 256), 256, 0, a, b, words, out);
 }
 
-int32_t filter_tiles(int32_t n, int64_t nnz) {
-    const int64_t t = ((int64_t)n + nnz + kFilterTile - 1) / kFilterTile;
-    return (int32_t)std::max<int64_t>(t, 1);
-}
-
 // counts and first: one entry per work unit (first: one more)
 void launch_filter_count(tr_ctx *ctx, const FilterJob *jobs, int njobs, const FilterJob &one, int32_t ntiles,
                          int32_t *counts, int64_t *first, int64_t *scan_tmp) {
-    TR_LAUNCH(ctx, "filter_count", k_filter<false>, ntiles, kFilterThreads, 0, jobs, njobs, one, counts,
+    TR_LAUNCH(ctx, "filter_count", k_filter<false>, ntiles, kUnitThreads, 0, jobs, njobs, one, counts,
               (const int64_t *)nullptr);
     launch_exclusive_scan_i32_to_i64(ctx, counts, first, ntiles, scan_tmp);
 }
 
 void launch_filter_write(tr_ctx *ctx, const FilterJob *jobs, int njobs, const FilterJob &one, int32_t ntiles,
                          const int64_t *first) {
-    TR_LAUNCH(ctx, "filter_write", k_filter<true>, ntiles, kFilterThreads, 0, jobs, njobs, one, (int32_t *)nullptr,
+    TR_LAUNCH(ctx, "filter_write", k_filter<true>, ntiles, kUnitThreads, 0, jobs, njobs, one, (int32_t *)nullptr,
               first);
 }
 
@@ -204,7 +168,7 @@ int64_t compress(tr_ctx *ctx, const tr_csx_t *m, const uint64_t *mask, tr_csx_t 
     j.mask = mask;
     j.n = ptrdim(m);
     j.nnz = m->nnz;
-    const int32_t nt = filter_tiles(j.n, j.nnz);
+    const int32_t nt = (int32_t)unit_count(j.n, j.nnz);
     int32_t *counts = (int32_t *)scratch(ctx, S_MISC, sizeof(int32_t) * (size_t)nt);
     int64_t *first = (int64_t *)scratch(ctx, S_ROWPTR64, sizeof(int64_t) * ((size_t)nt + 1));
     launch_filter_count(ctx, nullptr, 0, j, nt, counts, first, nullptr);

@@ -3,9 +3,10 @@
 // Replaces LocalMatrix::spgemm / KokkosSparse::spgemm
 // (include/KokkosWrap.hpp:367-391, call at :375).  Pipeline:
 //
-//  1. row analysis   one wave per row: flops_i = sum_{k in A_i} nnz(B_k);
-//                    rows are binned by flops (empty / light classes by hash
-//                    table size / heavy).
+//  1. row analysis   flops_i = sum_{k in A_i} nnz(B_k), summed in equal units
+//                    of entries by the pass that also checks the operands
+//                    (k_check.hip); rows are binned by flops (empty / light
+//                    classes by hash table size / heavy).
 //  2. symbolic       light rows (flops <= the tuned cut): one wave per row, LDS
 //                    open-addressing hash of column keys;
 //                    heavy rows: one 1024-thread block per row, a bitmap of
@@ -276,81 +277,75 @@ __device__ __forceinline__ const Panel &find_panel(const Panel *__restrict__ pan
 }
 
 // ---------------------------------------------------------------- analysis
-// 256 global rows per block: a thread per row for short rows, the whole wave
-// for rows with more than 32 entries; class counters are aggregated in LDS
-// so there is one global atomic per class per block.
-constexpr int kRowsPerBlock = 256;
+// k_check.hip sums every row's multiplications; here a thread takes four global
+// rows and puts them into their classes.  Class counters are aggregated in LDS
+// so there is one global atomic per class per workgroup; they all meet in one
+// cache line, so a workgroup takes 1024 rows (256: 77 us on 2^19 rows, now
+// 23 us).
+constexpr int kRowsPerBlock = 1024;
+constexpr int kClassThreads = 256;
 
 __global__ void k_zero_counters(Counters *__restrict__ cnt) {
     if (threadIdx.x < sizeof(Counters) / 4) ((int32_t *)cnt)[threadIdx.x] = 0;
 }
 
-__global__ void k_zero_i64(int64_t *__restrict__ p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = 0;
+// start of a plain product: its one task, from the kernel's argument, and the
+// counters
+__global__ void k_put_task(TaskDev *__restrict__ dst, const TaskDev t, Counters *__restrict__ cnt) {
+    if (threadIdx.x < sizeof(Counters) / 4) ((int32_t *)cnt)[threadIdx.x] = 0;
+    if (threadIdx.x == 0) *dst = t;
 }
 
-__global__ __launch_bounds__(kRowsPerBlock) void k_row_flops(const TaskDev *__restrict__ tasks, int nt,
-                                                             int32_t rows_total, int64_t *__restrict__ flops,
-                                                             int32_t *__restrict__ lists,
-                                                             Counters *__restrict__ cnt, int32_t light_max) {
+__global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__restrict__ tasks, int nt,
+                                                            int32_t rows_total, const int64_t *__restrict__ flops,
+                                                            int64_t *__restrict__ rownnz,
+                                                            int32_t *__restrict__ lists, Counters *__restrict__ cnt,
+                                                            int32_t light_max) {
+    constexpr int kPer = kRowsPerBlock / kClassThreads;
     __shared__ int32_t s_cnt[kNumClasses], s_base[kNumClasses];
     __shared__ unsigned long long s_f, s_hf;
     const int tid = threadIdx.x, l = lane_id();
-    const int32_t g = blockIdx.x * kRowsPerBlock + tid;
+    const int32_t g0 = blockIdx.x * kRowsPerBlock + tid;
     if (tid < kNumClasses) s_cnt[tid] = 0;
     if (tid == 0) s_f = s_hf = 0ull;
     __syncthreads();
-    int32_t a0 = 0, a1 = 0, ncols = 0;
-    const int32_t *ai = nullptr, *bp = nullptr;
-    if (g < rows_total) {
-        const TaskDev &T = tasks[task_of(tasks, nt, g)];
-        const int32_t r = g - T.row_base;
-        a0 = T.ap[r];
-        a1 = T.ap[r + 1];
-        ai = T.ai;
-        bp = T.bp;
-        ncols = T.n;
-    }
-    int64_t f = 0;
-    if (a1 - a0 <= 32) {
-        for (int32_t p = a0; p < a1; ++p) {
-            const int32_t k = ai[p];
-            f += bp[k + 1] - bp[k];
+    int64_t f[kPer], sf = 0, shf = 0;
+    int32_t ncols[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int32_t g = g0 + u * kClassThreads;
+        f[u] = 0;
+        ncols[u] = 0;
+        if (g < rows_total) {
+            ncols[u] = tasks[task_of(tasks, nt, g)].n;
+            f[u] = flops[g];
+            rownnz[g] = 0;
         }
     }
-    uint64_t longm = ballot(a1 - a0 > 32);
-    while (longm) {
-        const int src = __ffsll((unsigned long long)longm) - 1;
-        longm &= longm - 1;
-        const int32_t s0 = __shfl(a0, src, kWave), s1 = __shfl(a1, src, kWave);
-        const int32_t *sai = (const int32_t *)__shfl((long long)ai, src, kWave);
-        const int32_t *sbp = (const int32_t *)__shfl((long long)bp, src, kWave);
-        int64_t acc = 0;
-        for (int32_t p = s0 + l; p < s1; p += kWave) {
-            const int32_t k = sai[p];
-            acc += sbp[k + 1] - sbp[k];
-        }
-        acc = wave_sum(acc);
-        if (l == src) f = acc;
-    }
-    int c = -1, lpos = 0;
-    if (g < rows_total && f > 0) {
-        if (f <= light_max) {
-            const int64_t bound = f < ncols ? f : ncols;
-            int64_t T = 64;
-            c = 0;
-            while (T < 2 * bound) {
-                T <<= 1;
-                ++c;
+    int c[kPer], lpos[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        c[u] = -1;
+        lpos[u] = 0;
+        if (f[u] > 0) {
+            if (f[u] <= light_max) {
+                const int64_t bound = f[u] < ncols[u] ? f[u] : ncols[u];
+                int64_t T = 64;
+                c[u] = 0;
+                while (T < 2 * bound) {
+                    T <<= 1;
+                    ++c[u];
+                }
+            } else {
+                c[u] = f[u] <= kMidMaxF ? kMidClass : kHeavyClass;
+                shf += f[u];
             }
-        } else {
-            c = f <= kMidMaxF ? kMidClass : kHeavyClass;
+            lpos[u] = atomicAdd(&s_cnt[c[u]], 1);
+            sf += f[u];
         }
-        lpos = atomicAdd(&s_cnt[c], 1);
     }
-    const unsigned long long wf = (unsigned long long)wave_sum(f);
-    const unsigned long long whf = (unsigned long long)wave_sum(c >= kHeavyClass ? f : (int64_t)0);
+    const unsigned long long wf = (unsigned long long)wave_sum(sf);
+    const unsigned long long whf = (unsigned long long)wave_sum(shf);
     if (l == 0) {
         atomicAdd(&s_f, wf);
         atomicAdd(&s_hf, whf);
@@ -362,8 +357,9 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_row_flops(const TaskDev *__re
         if (s_hf) atomicAdd(&cnt->heavy_flops, s_hf);
     }
     __syncthreads();
-    if (c >= 0) lists[(int64_t)c * rows_total + s_base[c] + lpos] = g;
-    if (g < rows_total) flops[g] = f;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+        if (c[u] >= 0) lists[(int64_t)c[u] * rows_total + s_base[c[u]] + lpos[u]] = g0 + u * kClassThreads;
 }
 
 // ---------------------------------------------------------------- symbolic, light rows
@@ -1652,9 +1648,11 @@ void launch_num_light(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
 
 }  // namespace
 
-void mul_setup(tr_ctx *ctx, Workspace &ws, MulPlan &pl, const std::vector<TaskDev> &tasks) {
-    pl.nt = (int)tasks.size();
-    pl.h_tasks = tasks;
+namespace {
+
+// buffers of a plan over pl.h_tasks
+void mul_buffers(tr_ctx *ctx, Workspace &ws, MulPlan &pl) {
+    pl.nt = (int)pl.h_tasks.size();
     pl.tune = ctx->tune;
     int64_t rows = 0;
     for (auto &t : pl.h_tasks) {
@@ -1663,25 +1661,103 @@ void mul_setup(tr_ctx *ctx, Workspace &ws, MulPlan &pl, const std::vector<TaskDe
     }
     TR_REQUIRE(rows < INT32_MAX, "spgemm: total rows of the batch exceed INT32_MAX");
     pl.rows_total = (int32_t)rows;
-    const size_t R = (size_t)rows + 1;
-    pl.d_tasks = (TaskDev *)ws.get(S_PANELS + 0, sizeof(TaskDev) * (size_t)std::max(pl.nt, 1));
+    const size_t R = (size_t)rows + 1, nt = (size_t)std::max(pl.nt, 1);
+    pl.d_tasks = (TaskDev *)ws.get(S_PANELS + 0, (sizeof(TaskDev) + sizeof(CheckJob)) * nt);
     pl.flops = (int64_t *)ws.get(S_FLOPS, sizeof(int64_t) * R);
     pl.lists = (int32_t *)ws.get(S_BINS, sizeof(int32_t) * (size_t)kNumClasses * R);
     pl.cnt = (Counters *)ws.get(S_BINCNT, sizeof(Counters));
     pl.rownnz = (int64_t *)ws.get(S_ROWNNZ, sizeof(int64_t) * R);
     pl.rowptr = (int64_t *)ws.get(S_ROWPTR64, sizeof(int64_t) * R);
     pl.scan_tmp = ws.owned ? (int64_t *)ws.get(S_SCAN_TMP, scan_tmp_bytes(rows)) : nullptr;
+}
+
+CheckJob flops_job(const MulPlan &pl, const TaskDev &t) {
+    CheckJob j{};
+    j.ptr = t.ap;
+    j.idx = t.ai;
+    j.bp = t.bp;
+    j.flops = pl.flops + t.row_base;
+    j.cap = t.a_cap;
+    j.n = t.m;
+    j.other = t.k;
+    return j;
+}
+
+TaskDev task_of_pair(const tr_csx_t *A, const tr_csx_t *B) {
+    TaskDev t{};
+    t.ap = A->ptr_vec;
+    t.ai = A->idx_vec;
+    t.av = A->val;
+    t.bp = B->ptr_vec;
+    t.bi = B->idx_vec;
+    t.bv = B->val;
+    t.m = A->nrows;
+    t.n = B->ncols;
+    t.k = A->ncols;
+    t.a_cap = A->nnz;
+    return t;
+}
+
+}  // namespace
+
+void mul_setup(tr_ctx *ctx, Workspace &ws, MulPlan &pl, const std::vector<TaskDev> &tasks) {
+    pl.h_tasks = tasks;
+    mul_buffers(ctx, ws, pl);
+    std::vector<CheckJob> jobs;
+    for (auto &t : pl.h_tasks) {
+        jobs.push_back(flops_job(pl, t));
+        check_place(jobs.back(), pl.check_grid);
+    }
+    pl.njobs = pl.nt;
+    pl.jobs = (CheckJob *)(pl.d_tasks + pl.nt);
     TR_HIP(hipMemcpyAsync(pl.d_tasks, pl.h_tasks.data(), sizeof(TaskDev) * (size_t)pl.nt, hipMemcpyHostToDevice,
                           ctx->stream));
+    TR_HIP(hipMemcpyAsync(pl.jobs, jobs.data(), sizeof(CheckJob) * jobs.size(), hipMemcpyHostToDevice, ctx->stream));
+    TR_HIP(hipStreamSynchronize(ctx->stream));  // `jobs` ends here
+}
+
+void mul_setup_plain(tr_ctx *ctx, Workspace &ws, MulPlan &pl, const tr_csx_t *A, const tr_csx_t *B) {
+    check_operand_shapes(A, B);
+    pl.h_tasks = {task_of_pair(A, B)};
+    mul_buffers(ctx, ws, pl);
+    pl.pair.j[0] = flops_job(pl, pl.h_tasks[0]);
+    check_place(pl.pair.j[0], pl.check_grid);
+    pl.njobs = 1;
+    if (!same_tile(A, B)) {
+        pl.pair.j[1] = check_job(B);
+        check_place(pl.pair.j[1], pl.check_grid);
+        pl.njobs = 2;
+    }
 }
 
 void mul_analyze(tr_ctx *ctx, MulPlan &pl) {
-    TR_LAUNCH(ctx, "zero_counters", k_zero_counters, 1, 64, 0, pl.cnt);
-    TR_LAUNCH(ctx, "zero_rownnz", k_zero_i64, cap_grid(div_up((uint64_t)pl.rows_total + 1, 256), 4096), 256, 0,
-              pl.rownnz, (int64_t)pl.rows_total + 1);
-    TR_LAUNCH(ctx, "row_flops", k_row_flops, div_up((uint64_t)pl.rows_total, kRowsPerBlock), kRowsPerBlock, 0,
-              pl.d_tasks, pl.nt, pl.rows_total, pl.flops, pl.lists, pl.cnt,
-              pl.tune.light_max_flops);
+    if (pl.jobs) {
+        TR_LAUNCH(ctx, "zero_counters", k_zero_counters, 1, 64, 0, pl.cnt);
+    } else {
+        TR_LAUNCH(ctx, "put_task", k_put_task, 1, 64, 0, pl.d_tasks, pl.h_tasks[0], pl.cnt);
+        check_open(ctx);
+        ctx->check_twin = pl.njobs == 1;
+    }
+    launch_check(ctx, pl.jobs, pl.njobs, pl.pair, pl.check_grid);
+    TR_LAUNCH(ctx, "classify", k_classify, div_up((uint64_t)pl.rows_total, kRowsPerBlock), kClassThreads, 0,
+              pl.d_tasks, pl.nt, pl.rows_total, pl.flops, pl.rownnz, pl.lists, pl.cnt, pl.tune.light_max_flops);
+}
+
+namespace {
+
+void require_sorted_operands(const int32_t (&hs)[2]) {
+    if (hs[0] & 3) fail(TR_ERR_INVALID, "spgemm: A is not a valid CSR (ptr or column index out of range)");
+    if (hs[1] & 3) fail(TR_ERR_INVALID, "spgemm: B is not a valid CSR (ptr or column index out of range)");
+    if (hs[1] & 4) fail(TR_ERR_INVALID, "spgemm: B has unsorted or duplicate columns; call tr_csx_sort_rows");
+    if (hs[0] & 4) fail(TR_ERR_INVALID, "spgemm: A has unsorted or duplicate columns; call tr_csx_sort_rows");
+}
+
+}  // namespace
+
+void mul_checked(tr_ctx *ctx) {
+    int32_t hs[2];
+    check_result(ctx, hs, 2);
+    require_sorted_operands(hs);
 }
 
 void mul_read_counts(tr_ctx *ctx, MulPlan &pl) { read_array(ctx, &pl.h, pl.cnt, sizeof(Counters)); }
@@ -1800,23 +1876,6 @@ void mul_check(tr_ctx *ctx, MulPlan &pl) {
     if (ov & 14) fail(TR_ERR_HIP, "spgemm: numeric row counts disagree with the symbolic phase (internal error)");
 }
 
-namespace {
-
-TaskDev task_of_pair(const tr_csx_t *A, const tr_csx_t *B) {
-    TaskDev t{};
-    t.ap = A->ptr_vec;
-    t.ai = A->idx_vec;
-    t.av = A->val;
-    t.bp = B->ptr_vec;
-    t.bi = B->idx_vec;
-    t.bv = B->val;
-    t.m = A->nrows;
-    t.n = B->ncols;
-    return t;
-}
-
-}  // namespace
-
 void check_operand_shapes(const tr_csx_t *A, const tr_csx_t *B) {
     check_csx(A, "A");
     check_csx(B, "B");
@@ -1826,35 +1885,29 @@ void check_operand_shapes(const tr_csx_t *A, const tr_csx_t *B) {
 
 void validate_operands(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B) {
     check_operand_shapes(A, B);
-    int32_t *st = (int32_t *)scratch(ctx, S_TMP_CSX, 64);
-    TR_HIP(hipMemsetAsync(st, 0, 2 * sizeof(int32_t), ctx->stream));
-    launch_validate(ctx, A, st);
-    launch_validate(ctx, B, st + 1);
+    const tr_csx_t *m[2] = {A, B};
     int32_t hs[2];
-    read_array(ctx, hs, st, sizeof(hs));
-    if (hs[0] & 3) fail(TR_ERR_INVALID, "spgemm: A is not a valid CSR (ptr or column index out of range)");
-    if (hs[1] & 3) fail(TR_ERR_INVALID, "spgemm: B is not a valid CSR (ptr or column index out of range)");
-    if (hs[1] & 4) fail(TR_ERR_INVALID, "spgemm: B has unsorted or duplicate columns; call tr_csx_sort_rows");
-    if (hs[0] & 4) fail(TR_ERR_INVALID, "spgemm: A has unsorted or duplicate columns; call tr_csx_sort_rows");
+    check_tiles(ctx, m, 2, hs);
+    require_sorted_operands(hs);
 }
 
 int64_t spgemm_flops(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B) {
-    validate_operands(ctx, A, B);
     Workspace ws(ctx, false);
     MulPlan pl;
-    mul_setup(ctx, ws, pl, {task_of_pair(A, B)});
+    mul_setup_plain(ctx, ws, pl, A, B);
     mul_analyze(ctx, pl);
     mul_read_counts(ctx, pl);
+    mul_checked(ctx);
     return (int64_t)pl.h.flops;
 }
 
 void spgemm_symbolic_only(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int64_t *nnz, size_t *bytes) {
-    validate_operands(ctx, A, B);
     Workspace ws(ctx, false);
     MulPlan pl;
-    mul_setup(ctx, ws, pl, {task_of_pair(A, B)});
+    mul_setup_plain(ctx, ws, pl, A, B);
     mul_analyze(ctx, pl);
     mul_read_counts(ctx, pl);
+    mul_checked(ctx);
     // the same steps as the product up to its numeric phase, so every work
     // list and the cursor array are sized exactly as the product sizes them
     mul_symbolic(ctx, ws, pl, true, false);
@@ -1864,12 +1917,11 @@ void spgemm_symbolic_only(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int
     if (bytes) {
         // Upper bound of the device memory tr_spgemm takes from a context
         // pool with nothing cached: every scratch slot at the size the product
-        // requests (grown to 1.25x, in pool granules), the cursor array, the
-        // operand checks and the output tile.  A batch places the product in
+        // requests (grown to 1.25x, in pool granules), the cursor array and the
+        // output tile.  A batch places the product in
         // two blocks (indices, values) and its row pointers in a third.
         std::vector<size_t> req = ws.req;
         if (pl.h.items > 0) req[S_CURSORS] = std::max(req[S_CURSORS], sizeof(int4) * (size_t)std::max<int64_t>(ncur, 1));
-        req[S_MISC2] = std::max(req[S_MISC2], validate_tmp_bytes(std::max(A->nnz, B->nnz)));
         req[S_TMP_CSX] = std::max(req[S_TMP_CSX], std::max<size_t>(64, sizeof(Panel)));
         size_t b = 0;
         for (size_t r : req)
@@ -1886,12 +1938,12 @@ int spgemm_panels(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int64_t max
                   int32_t *row_begin, int32_t max_panels, int32_t *npanels) {
     TR_REQUIRE(panels && row_begin && npanels && max_panels >= 1, "spgemm: null panel outputs");
     TR_REQUIRE(max_panel_nnz >= 1 && max_panel_nnz <= INT32_MAX, "spgemm: max_panel_nnz must be in [1, INT32_MAX]");
-    validate_operands(ctx, A, B);
     Workspace ws(ctx, false);
     MulPlan pl;
-    mul_setup(ctx, ws, pl, {task_of_pair(A, B)});
+    mul_setup_plain(ctx, ws, pl, A, B);
     mul_analyze(ctx, pl);
     mul_read_counts(ctx, pl);
+    mul_checked(ctx);
     mul_symbolic(ctx, ws, pl, true, false);
     const int64_t ncur = mul_cursor_prep(ctx, ws, pl, false);
     const int32_t m = pl.rows_total;

@@ -1,5 +1,5 @@
-// Utility kernels of libtrident_hip: scans, CSR validation and
-// per-row sorting.  These are not the hot path; they are written for
+// Utility kernels of libtrident_hip: scans and per-row
+// sorting.  These are not the hot path; they are written for
 // correctness with coalesced access and no host round trips.
 #include "dev_common.h"
 #include "scan.h"
@@ -46,41 +46,6 @@ __global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (; i < n; i += stride) p[i] = v;
-}
-
-// ---- validation ----
-// status bits: 1 ptr malformed, 2 idx out of range, 4 unsorted/duplicate.
-__global__ void k_validate_ptr(const int32_t *__restrict__ ptr, int32_t P, int64_t nnz,
-                               uint32_t *__restrict__ starts, int32_t *__restrict__ status) {
-    int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > P) return;
-    int32_t v = ptr[i];
-    bool bad = (v < 0) || ((int64_t)v > nnz);
-    if (i == 0 && v != 0) bad = true;
-    if (i == P && (int64_t)v != nnz) bad = true;
-    if (i < P) {
-        int32_t w = ptr[i + 1];
-        if (w < v) bad = true;
-        if (!bad && v < w && (int64_t)v < nnz) atomicOr(&starts[v >> 5], 1u << (v & 31));
-    }
-    if (bad) atomicOr(status, 1);
-}
-
-__global__ void k_validate_idx(const int32_t *__restrict__ idx, int64_t nnz, int32_t O,
-                               const uint32_t *__restrict__ starts, int32_t *__restrict__ status) {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    int flags = 0;
-    for (; p < nnz; p += stride) {
-        int32_t c = idx[p];
-        if (c < 0 || c >= O) flags |= 2;
-        if (p + 1 < nnz) {
-            int64_t q = p + 1;
-            bool row_start = (starts[q >> 5] >> (q & 31)) & 1u;
-            if (!row_start && idx[q] <= c) flags |= 4;
-        }
-    }
-    if (flags) atomicOr(status, flags);
 }
 
 __global__ void k_rowptr_rebase(const int64_t *__restrict__ rp, int32_t r0, int32_t n, int32_t *__restrict__ o) {
@@ -212,25 +177,6 @@ void launch_fill_i32(tr_ctx *ctx, int32_t *p, int32_t v, int64_t n) {
     if (n <= 0) return;
     uint32_t g = (uint32_t)std::min<int64_t>((n + 255) / 256, 65536);
     TR_LAUNCH(ctx, "fill_i32", k_fill_i32, g, 256, 0, p, v, n);
-}
-
-size_t validate_tmp_bytes(int64_t nnz) { return sizeof(uint32_t) * (size_t)(nnz / 32 + 2); }
-
-void launch_validate(tr_ctx *ctx, const tr_csx_t *m, int32_t *d_status, uint32_t *starts) {
-    const int32_t P = ptrdim(m), O = otherdim(m);
-    const size_t words = validate_tmp_bytes(m->nnz) / sizeof(uint32_t);
-    if (starts) {
-        launch_fill_i32(ctx, (int32_t *)starts, 0, (int64_t)words);
-    } else {
-        starts = (uint32_t *)scratch(ctx, S_MISC2, words * sizeof(uint32_t));
-        TR_HIP(hipMemsetAsync(starts, 0, words * sizeof(uint32_t), ctx->stream));
-    }
-    TR_LAUNCH(ctx, "validate_ptr", k_validate_ptr, div_up((uint64_t)P + 1, 256), 256, 0, m->ptr_vec, P, m->nnz,
-              starts, d_status);
-    if (m->nnz > 0) {
-        uint32_t g = (uint32_t)std::min<int64_t>((m->nnz + 255) / 256, 16384);
-        TR_LAUNCH(ctx, "validate_idx", k_validate_idx, g, 256, 0, m->idx_vec, m->nnz, O, starts, d_status);
-    }
 }
 
 void launch_rowptr_i64_to_i32(tr_ctx *ctx, const int64_t *rp64, int32_t r0, int32_t r1, int32_t *out) {

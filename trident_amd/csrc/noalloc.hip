@@ -62,25 +62,22 @@ static char *noalloc_base(int device) {
 
 int64_t noalloc_spadd_into(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, tr_csx_t *out, int64_t capacity) {
     char *base = noalloc_base(ctx->device);
-    // [status words | validation bitmap | add temporaries], 256-byte pieces
-    const size_t st_bytes = 256;
-    const size_t val_bytes = (validate_tmp_bytes(std::max(A->nnz, C->nnz)) + 255) & ~(size_t)255;
+    // [reserved | add temporaries], 256-byte pieces; the reserved part is the
+    // documented limit's share of the operand checks
+    const size_t val_bytes = (256 + sizeof(uint32_t) * (size_t)(std::max(A->nnz, C->nnz) / 32 + 2) + 255) & ~(size_t)255;
     const size_t add_bytes = spadd_fixed_bytes(A->nrows, A->nnz, C->nnz);
-    const size_t need = st_bytes + val_bytes + add_bytes;
+    const size_t need = val_bytes + add_bytes;
     if (need > kNoallocBytes)
         fail(TR_ERR_INVALID, "tr_spadd_into_noalloc: operands need " + std::to_string(need) +
                                  " bytes of scratch, more than the fixed " + std::to_string(kNoallocBytes) +
                                  " (use tr_spadd_into)");
-    int32_t *st = (int32_t *)base;
-    uint32_t *starts = (uint32_t *)(base + st_bytes);
-    launch_fill_i32(ctx, st, 0, 2);
-    launch_validate(ctx, A, st, starts);
-    launch_validate(ctx, C, st + 1, starts);  // same stream: A's checks finish first
-    const int64_t hs = read_scalar<int64_t>(ctx, (const int64_t *)st);
-    const int32_t s0 = (int32_t)(hs & 0xffffffff), s1 = (int32_t)(hs >> 32);
+    const tr_csx_t *m[2] = {A, C};
+    int32_t hs[2];
+    check_tiles(ctx, m, 2, hs);
+    const int32_t s0 = hs[0], s1 = hs[1];
     if ((s0 | s1) & 3) fail(TR_ERR_INVALID, "tr_spadd_into_noalloc: malformed CSR operand");
     if ((s0 | s1) & 4) fail(TR_ERR_INVALID, "tr_spadd_into_noalloc: operands need sorted unique columns");
-    return spadd_into_fixed(ctx, A, C, out->ptr_vec, out->idx_vec, out->val, capacity, base + st_bytes + val_bytes,
+    return spadd_into_fixed(ctx, A, C, out->ptr_vec, out->idx_vec, out->val, capacity, base + val_bytes,
                             add_bytes);
 }
 

@@ -65,7 +65,8 @@ struct TaskDev {
     int32_t m;         // rows of A_t
     int32_t n;         // columns of B_t
     int32_t row_base;  // first global row
-    int32_t pad;
+    int32_t k;         // columns of A_t, rows of B_t
+    int64_t a_cap;     // entries of A_t's arrays (a compressed A_t holds ap[m] of them)
 };
 
 // device counters written by the symbolic phase
@@ -103,6 +104,12 @@ struct MulPlan {
     int32_t rows_total = 0;
     std::vector<TaskDev> h_tasks;
     TaskDev *d_tasks = nullptr;
+    // the pass over A's entries that sums the flops: a job per task, as a device
+    // table, or by value with B's checks for a plain product
+    CheckJob *jobs = nullptr;
+    CheckPair pair{};
+    int njobs = 0;
+    CheckGrid check_grid;
     int64_t *flops = nullptr, *rownnz = nullptr, *rowptr = nullptr;
     int32_t *lists = nullptr;
     Counters *cnt = nullptr;
@@ -161,6 +168,10 @@ void add_write(tr_ctx *ctx, AddPlan &ap, int32_t *oi, double *ov);
 // grids and lists; in capture mode every size comes from a previous eager run
 // on the same operands.
 void mul_setup(tr_ctx *ctx, Workspace &ws, MulPlan &pl, const std::vector<TaskDev> &tasks);
+// One product of operands that the analysis also checks: mul_checked, after
+// the counts are read, fails if they are not sorted CSRs.
+void mul_setup_plain(tr_ctx *ctx, Workspace &ws, MulPlan &pl, const tr_csx_t *A, const tr_csx_t *B);
+void mul_checked(tr_ctx *ctx);
 void mul_analyze(tr_ctx *ctx, MulPlan &pl);
 void mul_read_counts(tr_ctx *ctx, MulPlan &pl);
 void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool capture);

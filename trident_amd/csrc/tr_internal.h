@@ -94,6 +94,8 @@ tr_tuning_t tuning_process_default();
 void tuning_check(const tr_tuning_t &t);  // throws TR_ERR_INVALID
 }  // namespace tr
 
+constexpr size_t kPinnedValues = 2048, kPinnedBytes = 4096;
+
 struct tr_ctx {
     int device = 0;
     tr_tuning_t tune = tr::tuning_process_default();
@@ -107,9 +109,13 @@ struct tr_ctx {
     std::vector<void *> scratch_ptr;
     std::vector<size_t> scratch_size;
 
-    // Pinned host staging for small device->host reads.
+    // Pinned host memory: kPinnedValues bytes for small values read back, then
+    // the findings of tile checks, a byte each that the kernels write; the
+    // latter are zero between calls.
     void *pinned = nullptr;
-    size_t pinned_size = 0;
+    uint8_t *status = nullptr;
+    bool check_running = false;  // a check was begun and its result not taken
+    bool check_twin = false;     // its second tile is the first
 
     // Launch instrumentation.
     bool timing = false;
@@ -147,7 +153,6 @@ void *scratch(tr_ctx *ctx, int slot, size_t bytes);
 // 1 MiB, 2 MiB granules above); scratch slots grow to 1.25x a request.
 size_t pool_block_bytes(size_t b);
 inline size_t scratch_block_bytes(size_t b) { return pool_block_bytes(b + b / 4); }
-void *pinned(tr_ctx *ctx, size_t bytes);
 
 // Launch bracketing for per-kernel timing.
 struct TimerScope {
@@ -191,14 +196,42 @@ size_t scan_tmp_bytes(int64_t n);
 void launch_exclusive_scan_i64(tr_ctx *ctx, const int64_t *in, int64_t *out, int64_t n, int64_t *tmp = nullptr);
 void launch_exclusive_scan_i32_to_i64(tr_ctx *ctx, const int32_t *in, int64_t *out, int64_t n,
                                       int64_t *tmp = nullptr);
-// starts: caller-owned temp of validate_tmp_bytes(nnz) bytes, or nullptr to
-// use the context scratch.
-size_t validate_tmp_bytes(int64_t nnz);
-void launch_validate(tr_ctx *ctx, const tr_csx_t *m, int32_t *d_status, uint32_t *starts = nullptr);
 void launch_fill_i32(tr_ctx *ctx, int32_t *p, int32_t v, int64_t n);
 void launch_copy16(tr_ctx *ctx, void *dst, const void *src, size_t bytes);
 void launch_sort_rows(tr_ctx *ctx, tr_csx_t *m);
 void launch_rowptr_i64_to_i32(tr_ctx *ctx, const int64_t *rp64, int32_t r0, int32_t r1, int32_t *out);
+
+// k_check.hip: well-formedness of tiles, and the multiplications per row of a
+// product, in one pass over the entries.  Per tile: bits 1 ptr malformed, 2
+// index out of range, 4 unsorted or duplicate indices in a segment.
+struct CheckJob {
+    const int32_t *ptr, *idx;
+    const int32_t *bp;   // row pointer of B: also sums its row lengths over A's entries
+    int64_t *flops;      // per segment, zeroed and summed here if bp
+    int64_t cap;         // entries (a table's job may hold fewer: ptr[n])
+    int32_t n, other;    // segments, and the bound of the indices
+    int32_t block0;      // the job's first workgroup in the pass over ptr
+    int32_t unit0;       // and in the pass over the entries
+};
+constexpr int kCheckTiles = 2;  // tiles of one plain call
+struct CheckPair {
+    CheckJob j[kCheckTiles];
+};
+struct CheckGrid {
+    int64_t blocks = 0, units = 0;
+};
+CheckJob check_job(const tr_csx_t *m);
+void check_place(CheckJob &j, CheckGrid &g);  // gives j its place in a launch
+// jobs: a device table, or nullptr for `pair` (findings go to the context's
+// status bytes; a table's jobs have none and come from checked operands)
+void launch_check(tr_ctx *ctx, const CheckJob *jobs, int nj, const CheckPair &pair, const CheckGrid &g);
+// Checks m[0..n) (n <= kCheckTiles); a tile that repeats the one before (same
+// arrays and shape) is read once.  check_result after any wait for the stream.
+bool same_tile(const tr_csx_t *a, const tr_csx_t *b);
+void check_open(tr_ctx *ctx);  // before a launch_check without a table
+void check_begin(tr_ctx *ctx, const tr_csx_t *const *m, int n);
+void check_result(tr_ctx *ctx, int32_t *status, int n);
+void check_tiles(tr_ctx *ctx, const tr_csx_t *const *m, int n, int32_t *status);  // both, with the wait
 
 // k_transpose.hip
 void launch_transpose(tr_ctx *ctx, const tr_csx_t *m, tr_csx_t *out);
@@ -220,8 +253,6 @@ struct FilterJob {
     int64_t nnz, cap;
     int32_t n, nmask, by_index, bytes, tile0, pad;
 };
-constexpr int kFilterTile = 2048;  // segments plus entries per work unit
-int32_t filter_tiles(int32_t n, int64_t nnz);
 void launch_filter_count(tr_ctx *ctx, const FilterJob *jobs, int njobs, const FilterJob &one, int32_t ntiles,
                          int32_t *counts, int64_t *first, int64_t *scan_tmp);
 void launch_filter_write(tr_ctx *ctx, const FilterJob *jobs, int njobs, const FilterJob &one, int32_t ntiles,
@@ -261,14 +292,14 @@ int64_t spadd_into_fixed(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, int3
 void noalloc_init(int device);
 int64_t noalloc_spadd_into(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, tr_csx_t *out, int64_t capacity);
 
-// Read a device value through pinned staging (synchronises the stream).
+// Read device values (synchronises the stream).
+void read_array(tr_ctx *ctx, void *host, const void *dptr, size_t bytes);
 template <typename T>
 T read_scalar(tr_ctx *ctx, const T *dptr) {
-    T *h = (T *)pinned(ctx, sizeof(T));
+    T *h = (T *)ctx->pinned;
     TR_HIP(hipMemcpyAsync(h, dptr, sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
     TR_HIP(hipStreamSynchronize(ctx->stream));
     return *h;
 }
-void read_array(tr_ctx *ctx, void *host, const void *dptr, size_t bytes);
 
 }  // namespace tr
