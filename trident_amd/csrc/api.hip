@@ -140,8 +140,43 @@ void *scratch(tr_ctx *ctx, int slot, size_t bytes) {
     return ctx->scratch_ptr[slot];
 }
 
+namespace {
+
+struct Publish {
+    const uint32_t *src[kReadParts];
+    int32_t end[kReadParts];  // words up to and with part i
+};
+
+__global__ void k_publish(const Publish p, int n, uint32_t *__restrict__ out) {
+    for (int i = threadIdx.x; i < p.end[n - 1]; i += blockDim.x) {
+        int t = 0;
+        while (i >= p.end[t]) ++t;
+        out[i] = p.src[t][i - (t ? p.end[t - 1] : 0)];
+    }
+}
+
+}  // namespace
+
+void read_parts(tr_ctx *ctx, const ReadPart *parts, int n) {
+    Publish p{};
+    int32_t words = 0;
+    for (int i = 0; i < n; ++i) {
+        p.src[i] = (const uint32_t *)parts[i].dev;
+        p.end[i] = words += (int32_t)(parts[i].bytes / 4);
+    }
+    TR_LAUNCH(ctx, "publish", k_publish, 1, 256, 0, p, n, (uint32_t *)ctx->pinned);
+    TR_HIP(hipStreamSynchronize(ctx->stream));
+    for (int i = 0; i < n; ++i)
+        std::memcpy(parts[i].host, (const uint32_t *)ctx->pinned + (i ? p.end[i - 1] : 0), parts[i].bytes);
+}
+
 void read_array(tr_ctx *ctx, void *host, const void *dptr, size_t bytes) {
     if (bytes == 0) return;
+    if (bytes <= kPinnedValues && bytes % 4 == 0) {
+        const ReadPart part{host, dptr, bytes};
+        read_parts(ctx, &part, 1);
+        return;
+    }
     TR_HIP(hipMemcpyAsync(host, dptr, bytes, hipMemcpyDeviceToHost, ctx->stream));
     TR_HIP(hipStreamSynchronize(ctx->stream));
 }
@@ -730,7 +765,11 @@ int tr_memcpy_h2d(tr_ctx_t ctx, void *dst, const void *src, size_t bytes) {
 
 int tr_memcpy_d2h(tr_ctx_t ctx, void *dst, const void *src, size_t bytes) {
     TR_CTX_REQUIRED(ctx);
-    return guarded(ctx, [&] { read_array(ctx, dst, src, bytes); });
+    return guarded(ctx, [&] {
+        if (bytes == 0) return;
+        TR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+        TR_HIP(hipStreamSynchronize(ctx->stream));
+    });
 }
 
 int tr_memcpy_d2d(tr_ctx_t ctx, void *dst, const void *src, size_t bytes) {

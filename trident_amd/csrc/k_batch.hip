@@ -193,6 +193,7 @@ struct tr_batch {
     double *o_val = nullptr;
     int32_t *o_ptr = nullptr;
     int64_t o_total = 0;
+    std::vector<int64_t> p_base;     // per task: first entry in the product arena, and the end
     std::vector<int64_t> o_base;     // per task: first entry in the output arena
     std::vector<int64_t> optr_off;   // per task: first row pointer in o_ptr
     std::vector<int64_t> o_nnz;
@@ -326,14 +327,14 @@ void batch_body(tr_batch *b, bool capture) {
     if (guarded) TR_LAUNCH(ctx, "batch_guard", k_guard_counts, 1, 64, 0, b->mp.cnt, b->guard);
     if (!capture) mul_read_counts(ctx, b->mp);
     mul_symbolic(ctx, *b->ws_mul, b->mp, true, capture);
-    const int64_t ncur = mul_cursor_prep(ctx, *b->ws_mul, b->mp, capture);
+    mul_cursor_prep(ctx, *b->ws_mul, b->mp, capture);
     if (guarded)
         TR_LAUNCH(ctx, "batch_guard", k_guard_products, 1, 64, 0, b->mp.d_tasks, b->nt, b->mp.rowptr,
                   b->mp.rows_total, b->expect_p, b->mp.cnt, b->mp.h.items > 0 ? b->mp.cbase : nullptr,
                   b->mp.item_cap, b->mp.cursor_cap, b->guard);
     if (!capture) {
-        b->p_total = read_scalar<int64_t>(ctx, b->mp.rowptr + b->mp.rows_total);
-        mul_read_counts(ctx, b->mp);
+        int64_t ncur = 0;
+        mul_read_totals(ctx, b->mp, &b->p_total, &ncur);
         if (b->mp.h.overflow & 1) fail(TR_ERR_HIP, "batch: heavy work list capacity exceeded");
         b->mp.cursor_cap = ncur;
         if (b->mp.h.items > 0)
@@ -350,11 +351,9 @@ void batch_body(tr_batch *b, bool capture) {
         // a product added into a partial-C tile must fit an int32 tile; a
         // product that is itself the result may be larger (it is then read
         // as row panels, tr_batch_result_panels)
-        std::vector<int64_t> rp(b->nt + 1);
-        for (int t = 0; t <= b->nt; ++t) {
-            const int32_t g = t < b->nt ? b->mp.h_tasks[t].row_base : b->mp.rows_total;
-            rp[t] = read_scalar<int64_t>(ctx, b->mp.rowptr + g);
-        }
+        std::vector<int64_t> &rp = b->p_base;
+        rp.resize(b->nt + 1);
+        mul_read_task_offsets(ctx, b->mp, rp.data());
         for (int t = 0; t < b->nt; ++t)
             if ((!b->no_accum || b->single_run) && rp[t + 1] - rp[t] > INT32_MAX)
                 fail(TR_ERR_OVERFLOW, "batch: a tile product exceeds INT32_MAX entries");
@@ -543,7 +542,7 @@ int tr::batch_create(tr_ctx_t ctx, int32_t ntasks, const tr_csx_t *A, const tr_c
         b->o_nnz.assign(ntasks, 0);
         for (int t = 0; t < ntasks; ++t) {
             if (b->no_accum) {
-                b->o_base[t] = read_scalar<int64_t>(ctx, b->mp.rowptr + b->mp.h_tasks[t].row_base);
+                b->o_base[t] = b->p_base[t];
                 continue;
             }
             const int32_t g = b->ap.h[t].row_base;
@@ -567,10 +566,9 @@ int tr::batch_create(tr_ctx_t ctx, int32_t ntasks, const tr_csx_t *A, const tr_c
                 add_op(b->B[t]);
                 add_op(b->Cin[t]);
             }
-            std::vector<int64_t> ep(ntasks + 1), eo(ntasks + 1);
+            const std::vector<int64_t> &ep = b->p_base;
+            std::vector<int64_t> eo(ntasks + 1);
             for (int t = 0; t <= ntasks; ++t) {
-                const int32_t g = t < ntasks ? b->mp.h_tasks[t].row_base : b->mp.rows_total;
-                ep[t] = read_scalar<int64_t>(ctx, b->mp.rowptr + g);
                 eo[t] = t < ntasks ? b->o_base[t] : b->o_total;
             }
             b->guard_nops = (int)go.size();

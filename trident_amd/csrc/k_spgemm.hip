@@ -35,6 +35,7 @@
 #include "spgemm_types.h"
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 
@@ -786,6 +787,15 @@ __global__ __launch_bounds__(256) void k_item_scatter(const Item *__restrict__ i
 __global__ void k_panel_bases(Panel *__restrict__ panels, int np, const int64_t *__restrict__ rowptr) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p < np) panels[p].nnz_begin = rowptr[panels[p].row_begin];
+}
+
+// int32 row pointers of the tile that holds global rows [r0, r0 + n], rebased,
+// and its entry of the panel table
+__global__ void k_tile_ptr(const int64_t *__restrict__ rowptr, int32_t r0, int32_t n, int32_t *__restrict__ ptr,
+                           const Panel panel, Panel *__restrict__ dst) {
+    const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) *dst = panel;
+    if (t <= n) ptr[t] = (int32_t)(rowptr[r0 + t] - rowptr[r0]);
 }
 
 // ---------------------------------------------------------------- numeric, light rows
@@ -1816,8 +1826,8 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
     launch_exclusive_scan_i64(ctx, pl.rownnz, pl.rowptr, pl.rows_total, pl.scan_tmp);
 }
 
-int64_t mul_cursor_prep(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool capture) {
-    if (!pl.h.cls[kHeavyClass] && !pl.h.cls[kMidClass]) return 0;
+void mul_cursor_prep(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool capture) {
+    if (!pl.h.cls[kHeavyClass] && !pl.h.cls[kMidClass]) return;
     if (!capture) {
         pl.clen = (int32_t *)ws.get(S_MISC, sizeof(int32_t) * ((size_t)pl.item_cap + 1));
         pl.cbase = (int64_t *)ws.get(S_MISC2, sizeof(int64_t) * ((size_t)pl.item_cap + 1));
@@ -1842,8 +1852,36 @@ int64_t mul_cursor_prep(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool capture) {
     TR_LAUNCH(ctx, "item_order", k_item_scatter, og, 256, 0, pl.items, pl.wins, pl.cnt, shift, pl.order_hist,
               pl.order);
     launch_exclusive_scan_i32_to_i64(ctx, pl.clen, pl.cbase, pl.item_cap, pl.scan_tmp);
-    if (capture) return pl.cursor_cap;
-    return read_scalar<int64_t>(ctx, pl.cbase + pl.item_cap);
+}
+
+void mul_read_totals(tr_ctx *ctx, MulPlan &pl, int64_t *nnz, int64_t *ncur) {
+    const bool heavy = pl.h.cls[kHeavyClass] || pl.h.cls[kMidClass];
+    *ncur = 0;
+    const ReadPart parts[3] = {{&pl.h, pl.cnt, sizeof(Counters)},
+                               {nnz, pl.rowptr + pl.rows_total, sizeof(int64_t)},
+                               {ncur, pl.cbase + pl.item_cap, sizeof(int64_t)}};
+    read_parts(ctx, parts, heavy ? 3 : 2);
+}
+
+namespace {
+
+__global__ void k_task_offsets(const TaskDev *__restrict__ tasks, int nt, const int64_t *__restrict__ rowptr,
+                               int32_t rows, int64_t *__restrict__ out) {
+    for (int t = threadIdx.x; t <= nt; t += blockDim.x) out[t] = rowptr[t < nt ? tasks[t].row_base : rows];
+}
+
+}  // namespace
+
+void mul_read_task_offsets(tr_ctx *ctx, MulPlan &pl, int64_t *host) {
+    if (sizeof(int64_t) * ((size_t)pl.nt + 1) > kPinnedValues) {
+        for (int t = 0; t <= pl.nt; ++t)
+            host[t] = read_scalar<int64_t>(ctx, pl.rowptr + (t < pl.nt ? pl.h_tasks[t].row_base : pl.rows_total));
+        return;
+    }
+    TR_LAUNCH(ctx, "publish", k_task_offsets, 1, 64, 0, pl.d_tasks, pl.nt, pl.rowptr, pl.rows_total,
+              (int64_t *)ctx->pinned);
+    TR_HIP(hipStreamSynchronize(ctx->stream));
+    std::memcpy(host, ctx->pinned, sizeof(int64_t) * ((size_t)pl.nt + 1));
 }
 
 void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np) {
@@ -1911,8 +1949,9 @@ void spgemm_symbolic_only(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int
     // the same steps as the product up to its numeric phase, so every work
     // list and the cursor array are sized exactly as the product sizes them
     mul_symbolic(ctx, ws, pl, true, false);
-    const int64_t ncur = mul_cursor_prep(ctx, ws, pl, false);
-    const int64_t total = read_scalar<int64_t>(ctx, pl.rowptr + pl.rows_total);
+    mul_cursor_prep(ctx, ws, pl, false);
+    int64_t total = 0, ncur = 0;
+    mul_read_totals(ctx, pl, &total, &ncur);
     if (nnz) *nnz = total;
     if (bytes) {
         // Upper bound of the device memory tr_spgemm takes from a context
@@ -1945,10 +1984,10 @@ int spgemm_panels(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int64_t max
     mul_read_counts(ctx, pl);
     mul_checked(ctx);
     mul_symbolic(ctx, ws, pl, true, false);
-    const int64_t ncur = mul_cursor_prep(ctx, ws, pl, false);
+    mul_cursor_prep(ctx, ws, pl, false);
     const int32_t m = pl.rows_total;
-    const int64_t total = read_scalar<int64_t>(ctx, pl.rowptr + m);
-    mul_read_counts(ctx, pl);
+    int64_t total = 0, ncur = 0;
+    mul_read_totals(ctx, pl, &total, &ncur);
     if (pl.h.overflow & 1) fail(TR_ERR_HIP, "spgemm: heavy work list capacity exceeded (internal bound violated)");
 
     // panel split
@@ -1974,24 +2013,19 @@ int spgemm_panels(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int64_t max
         fail(TR_ERR_OVERFLOW, "spgemm: nnz(C) = " + std::to_string(total) + " needs " + std::to_string(np) +
                                   " panels of at most " + std::to_string(max_panel_nnz) + " entries");
     }
-    std::vector<Panel> hp(np);
+    Panel *dp = (Panel *)ws.get(S_TMP_CSX, sizeof(Panel) * (size_t)np);
     for (int32_t p = 0; p < np; ++p) {
         const int64_t nb0 = np == 1 ? 0 : hrp[rb[p]];
         const int64_t nb1 = np == 1 ? total : hrp[rb[p + 1]];
         tr_csx_t *C = &panels[p];
         alloc_tile(ctx, TR_ROWS, rb[p + 1] - rb[p], pl.h_tasks[0].n, nb1 - nb0, C);
-        launch_rowptr_i64_to_i32(ctx, pl.rowptr, rb[p], rb[p + 1], C->ptr_vec);
-        hp[p].nnz_begin = nb0;
-        hp[p].row_begin = rb[p];
-        hp[p].pad = 0;
-        hp[p].idx = C->idx_vec;
-        hp[p].val = C->val;
+        const Panel hp{nb0, rb[p], 0, C->idx_vec, C->val};
+        TR_LAUNCH(ctx, "tile_ptr", k_tile_ptr, div_up((uint64_t)(rb[p + 1] - rb[p]) + 1, 256), 256, 0, pl.rowptr,
+                  rb[p], rb[p + 1] - rb[p], C->ptr_vec, hp, dp + p);
         row_begin[p] = rb[p];
     }
     row_begin[np] = m;
     *npanels = np;
-    Panel *dp = (Panel *)ws.get(S_TMP_CSX, sizeof(Panel) * (size_t)np);
-    TR_HIP(hipMemcpyAsync(dp, hp.data(), sizeof(Panel) * (size_t)np, hipMemcpyHostToDevice, ctx->stream));
     if (pl.h.items > 0)
         pl.cursors = (int4 *)ws.get(S_CURSORS, sizeof(int4) * (size_t)std::max<int64_t>(ncur, 1));
     mul_numeric(ctx, pl, dp, np);

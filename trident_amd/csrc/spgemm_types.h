@@ -175,7 +175,12 @@ void mul_checked(tr_ctx *ctx);
 void mul_analyze(tr_ctx *ctx, MulPlan &pl);
 void mul_read_counts(tr_ctx *ctx, MulPlan &pl);
 void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool capture);
-int64_t mul_cursor_prep(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool capture);  // returns cursor total (eager)
+void mul_cursor_prep(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool capture);
+// After the symbolic phase, one read (eager): refreshes the counters, returns
+// nnz(C) and the cursors that the heavy items need.
+void mul_read_totals(tr_ctx *ctx, MulPlan &pl, int64_t *nnz, int64_t *ncur);
+// The first product entry of every task, and the end (nt + 1 values).
+void mul_read_task_offsets(tr_ctx *ctx, MulPlan &pl, int64_t *host);
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np);
 void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np);
 void mul_check(tr_ctx *ctx, MulPlan &pl);  // reads the consistency flags (eager)
