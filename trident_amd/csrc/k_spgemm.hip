@@ -459,7 +459,8 @@ template <int PB, int NTH>
 // (2^19 columns) 17.8 -> 15.0 ms.
 __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 1) void k_sym_heavy(
     const TaskDev *__restrict__ tasks, int nt, const int32_t *__restrict__ rows, Counters *__restrict__ cnt, int cls,
-    int64_t *__restrict__ rownnz, int emit, int32_t win_h, int32_t item_windows, Window *__restrict__ wins,
+    int64_t *__restrict__ rownnz, int emit, int32_t win_h, int32_t item_windows, int64_t item_flops,
+    const int64_t *__restrict__ flops, Window *__restrict__ wins,
     int32_t win_cap, Item *__restrict__ items, int32_t item_cap, int32_t *__restrict__ lists, int32_t rows_total) {
     constexpr int kWords = 1 << (PB - 5);          // bitmap words of one pass
     constexpr int kFine = 1 << (PB - kFineShift);  // fine blocks of one pass
@@ -636,7 +637,10 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
             // rows of more than kLongRow entries get a quarter of the
             // windows per item: their items are the longest, and the last
             // of them would otherwise run alone at the end of the numeric
-            const int32_t iw = (a1 - a0 > kLongRow) ? max(1, item_windows / 4) : item_windows;
+            // and no item holds much more than item_flops multiplications
+            // (taking the row's as spread evenly over its windows)
+            const int32_t iw = max(1, (int32_t)min<int64_t>((a1 - a0 > kLongRow) ? item_windows / 4 : item_windows,
+                                                            item_flops * nwin / flops[g]));
             if (tid == 0) {
                 const int32_t nitems = (nwin + iw - 1) / iw;
                 const int32_t wb = atomicAdd(&cnt->windows, nwin);
@@ -1772,12 +1776,22 @@ void mul_checked(tr_ctx *ctx) {
 
 void mul_read_counts(tr_ctx *ctx, MulPlan &pl) { read_array(ctx, &pl.h, pl.cnt, sizeof(Counters)); }
 
+// Multiplications that one heavy item should hold at most.  A product with few
+// heavy rows would leave the chip to the few items that tune.item_windows
+// windows make of them: about kItemsPerSlot items for each of the five
+// workgroups a CU holds, but no item below kMinItemFlops.
+constexpr int kItemsPerSlot = 8;
+constexpr int64_t kMinItemFlops = 2048;
+int64_t item_flops(const tr_ctx *ctx, const MulPlan &pl) {
+    return std::max<int64_t>(kMinItemFlops, (int64_t)pl.h.heavy_flops / ((int64_t)ctx->cu_count * 5 * kItemsPerSlot));
+}
+
 template <int PB, int NTH>
 void launch_sym_heavy(tr_ctx *ctx, MulPlan &pl, int cls, int per_cu, bool emit) {
     TR_LAUNCH(ctx, "sym_heavy", (k_sym_heavy<PB, NTH>), cap_grid(pl.h.cls[cls], (int64_t)ctx->cu_count * per_cu), NTH,
               0, pl.d_tasks, pl.nt, pl.lists + (int64_t)cls * pl.rows_total, pl.cnt, cls, pl.rownnz, emit ? 1 : 0,
-              pl.tune.window_entries, pl.tune.item_windows, pl.wins, pl.win_cap, pl.items, pl.item_cap, pl.lists,
-              pl.rows_total);
+              pl.tune.window_entries, pl.tune.item_windows, item_flops(ctx, pl), pl.flops, pl.wins, pl.win_cap,
+              pl.items, pl.item_cap, pl.lists, pl.rows_total);
 }
 
 void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool capture) {
@@ -1797,7 +1811,9 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
             const int64_t wsplits = (int64_t)max_n / kWinMaxWidth + 1;
             const int64_t q = std::min<int64_t>(pl.tune.window_entries, kSparseH);
             const int64_t wcap = (int64_t)(pl.h.heavy_flops / q) + (int64_t)nh * (2 * passes + wsplits) + 16;
-            const int64_t icap = wcap / std::max(1, pl.tune.item_windows / 4) + (int64_t)nh * passes + 16;
+            // items: by the window count, or 2 for each item_flops multiplications
+            const int64_t icap = wcap / std::max(1, pl.tune.item_windows / 4) +
+                                 2 * ((int64_t)pl.h.heavy_flops / item_flops(ctx, pl)) + (int64_t)nh * passes + 16;
             TR_REQUIRE(wcap < INT32_MAX && icap < INT32_MAX, "spgemm: heavy work list exceeds int32 capacity");
             pl.win_cap = (int32_t)wcap;
             pl.item_cap = (int32_t)icap;
