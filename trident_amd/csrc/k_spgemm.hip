@@ -1779,8 +1779,11 @@ void mul_read_counts(tr_ctx *ctx, MulPlan &pl) { read_array(ctx, &pl.h, pl.cnt, 
 // Multiplications that one heavy item should hold at most.  A product with few
 // heavy rows would leave the chip to the few items that tune.item_windows
 // windows make of them: about kItemsPerSlot items for each of the five
-// workgroups a CU holds, but no item below kMinItemFlops.
-constexpr int kItemsPerSlot = 8;
+// workgroups a CU holds, but no item below kMinItemFlops.  (8, 32, 64 and 128
+// per slot: R-MAT s17 14.43, 13.74, 14.06, 14.44 ms; 16 served requests 21.9,
+// 20.8, 21.2, 21.7 ms; R-MAT s19, whose items the window count cuts, within
+// 1%.  A minimum of 8192 costs the R-MAT of 15013 vertices 3%.)
+constexpr int kItemsPerSlot = 32;
 constexpr int64_t kMinItemFlops = 2048;
 int64_t item_flops(const tr_ctx *ctx, const MulPlan &pl) {
     return std::max<int64_t>(kMinItemFlops, (int64_t)pl.h.heavy_flops / ((int64_t)ctx->cu_count * 5 * kItemsPerSlot));
