@@ -97,6 +97,16 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
     return v;
 }
 
+// Inclusive running maximum over the wave of unsigned values.
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+    v = max(v, dpp<0x111>(v));
+    v = max(v, dpp<0x112>(v));
+    v = max(v, dpp<0x114>(v));
+    v = max(v, dpp<0x118>(v));
+    v = max(v, dpp<0x142, 0xa>(v));
+    return max(v, dpp<0x143, 0xc>(v));
+}
+
 // Sum over the wave, wave-uniform.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {

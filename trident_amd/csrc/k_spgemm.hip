@@ -58,25 +58,40 @@ __device__ __forceinline__ int32_t lower_bound_dev(const TR_GLOBAL int32_t *__re
 
 // first q in (lo, e] with a[q] >= key (q == e if none), galloping from lo,
 // where a[lo] < key is known; vq receives a[q] (INT32_MAX when q == e), the
-// column the next window of a heavy row starts from
+// column the next window of a heavy row starts from.  A round probes 2, 8 and
+// 32 entries ahead with independent loads (then 128, 512, 2048, ...): the
+// search is a fifth of the heavy numeric, bound by its slowest lane's round
+// trips.  num_heavy of R-MAT s19: one probe a round, doubling 88.2 ms;
+// quadrupling 86.0; two probes (1, 4 / 2, 8) 84.9 / 84.6; three 84.1; with a
+// binary search of two probes a round 86.3.
 __device__ __forceinline__ int32_t gallop_from(const TR_GLOBAL int32_t *__restrict__ a, int32_t lo, int32_t e,
                                                int32_t key, int32_t &vq) {
-    int32_t step = 1, hi;
+    int32_t step = 2, hi;
     vq = INT32_MAX;
     while (true) {
-        hi = lo + step;
-        if (hi >= e) {
-            hi = e;
-            vq = INT32_MAX;
+        const int32_t rem = e - lo;  // (distances, so that no position overflows)
+        const int32_t v1 = step < rem ? a[lo + step] : INT32_MAX;
+        const int32_t v2 = 4 * step < rem ? a[lo + 4 * step] : INT32_MAX;
+        const int32_t v3 = 16 * step < rem ? a[lo + 16 * step] : INT32_MAX;
+        if (v1 >= key) {
+            vq = v1;
+            hi = lo + min(step, rem);
             break;
         }
-        const int32_t v = a[hi];
-        if (v >= key) {
-            vq = v;
+        if (v2 >= key) {
+            vq = v2;
+            hi = lo + min(4 * step, rem);
+            lo += step;
             break;
         }
-        lo = hi;
-        step <<= 1;
+        if (v3 >= key) {
+            vq = v3;
+            hi = lo + min(16 * step, rem);
+            lo += 4 * step;
+            break;
+        }
+        lo += 16 * step;
+        step <<= 6;
     }
     while (hi - lo > 1) {
         const int32_t mid = lo + ((hi - lo) >> 1);
@@ -1082,14 +1097,12 @@ struct HeavyWgLds {
     union {
         struct {                    // product steps of a window
             double pa[NT], pb[NT];  // the step's products (A value, B value) by thread
-            // segment starts of three rotating product steps: bit p of
-            // smask[b] is set where a segment starts at step position p
-            // (position 0 always holds the segment that covers the step's
-            // first product), smark[b][p] is that segment's index
-            unsigned long long smask[3][NT / kWave];
             int32_t seg_d[NT];  // B position minus flattened product position of segment (A entry) o
             uint16_t link[NT];  // next older product of the same slot in this step
-            typename std::conditional<(NT <= 256), uint8_t, uint16_t>::type smark[3][NT];
+            // segments of three rotating product steps: smark[b][p] is the
+            // index of the segment that starts at step position p, or that
+            // covers p where a wave's positions begin; 0 elsewhere
+            __align__(16) typename std::conditional<(NT <= 256), uint8_t, uint16_t>::type smark[3][NT];
         };
         struct {  // extraction of a window: presence bitmap and its prefix counts
             unsigned long long bm[kBmWords];
@@ -1100,45 +1113,76 @@ struct HeavyWgLds {
 
 // marks the segment [excl, excl + len) of the calling thread in the step that
 // starts at product `base`: at its first position in the step, and at every
-// later position of the step that starts a 64-position word, so that each
-// word's first position names the segment covering it
+// later position of the step where a wave begins, so that the segment of a
+// position is the last mark at or below it in its own wave
 template <int NT, typename M>
-__device__ __forceinline__ void mark_segment(unsigned long long *smask, M *smark, int32_t base, int32_t excl,
-                                             int32_t len) {
+__device__ __forceinline__ void mark_segment(M *smark, int32_t base, int32_t excl, int32_t len) {
     if (len <= 0) return;
     const int32_t rel = excl - base;
     const int32_t lo = rel > 0 ? rel : 0, hi = rel + len < NT ? rel + len : NT;
     if (lo >= hi) return;  // the segment has no product in this step
     smark[lo] = (M)threadIdx.x;
-    atomicOr(&smask[lo >> 6], 1ull << (lo & 63));
-    for (int32_t ws = (lo & ~63) + 64; ws < hi; ws += 64) {
-        smark[ws] = (M)threadIdx.x;
-        atomicOr(&smask[ws >> 6], 1ull);
-    }
+    for (int32_t ws = (lo & ~63) + 64; ws < hi; ws += 64) smark[ws] = (M)threadIdx.x;
 }
 
-// segment of step position rel: the mark at the highest set bit <= rel,
-// always inside rel's own word (its first position is marked)
+// segment of the calling thread's step position: segments rise with their
+// positions, so the last mark is a running maximum over the wave (one LDS read
+// and six register steps; a start mask and the mark at its highest bit took
+// two dependent reads, and marking an LDS atomic more)
 template <typename M>
-__device__ __forceinline__ int owner_marked(const unsigned long long *smask, const M *smark, int rel) {
-    const int w = rel >> 6;
-    const unsigned long long m = smask[w] & (~0ull >> (63 - (rel & 63)));
-    return (int)smark[w * 64 + 63 - __clzll((long long)m)];
+__device__ __forceinline__ int owner_marked(const M *smark) {
+    return (int)wave_incl_max((uint32_t)smark[threadIdx.x]);
 }
 
-// orders two products (thread id, A value, B value) by thread id
-__device__ __forceinline__ void order_products(uint32_t &u, double &a, double &b, uint32_t &w, double &c,
-                                               double &d) {
-    if (w < u) {
-        const uint32_t tu = u;
-        const double ta = a, tb = b;
-        u = w;
-        a = c;
-        b = d;
-        w = tu;
-        c = ta;
-        d = tb;
+template <int NT, typename M>
+__device__ __forceinline__ void clear_marks(M *smark, int n) {  // n: whole buffers
+    uint32_t *w = reinterpret_cast<uint32_t *>(smark);
+    for (int t = threadIdx.x; t < n * NT * (int)sizeof(M) / 4; t += NT) w[t] = 0u;
+}
+
+template <int K>
+__device__ __forceinline__ void exchange(uint32_t (&t)[K], int i, int j) {
+    const uint32_t a = t[i], b = t[j];
+    t[i] = min(a, b);
+    t[j] = max(a, b);
+}
+
+// ascending sort of 4 or 8 thread ids in registers
+__device__ __forceinline__ void sort_ids(uint32_t (&t)[4]) {
+    exchange(t, 0, 1), exchange(t, 2, 3);
+    exchange(t, 0, 2), exchange(t, 1, 3);
+    exchange(t, 1, 2);
+}
+__device__ __forceinline__ void sort_ids(uint32_t (&t)[8]) {
+    exchange(t, 0, 1), exchange(t, 2, 3), exchange(t, 4, 5), exchange(t, 6, 7);
+    exchange(t, 0, 2), exchange(t, 1, 3), exchange(t, 4, 6), exchange(t, 5, 7);
+    exchange(t, 1, 2), exchange(t, 5, 6), exchange(t, 0, 4), exchange(t, 3, 7);
+    exchange(t, 1, 5), exchange(t, 2, 6);
+    exchange(t, 1, 4), exchange(t, 3, 6);
+    exchange(t, 2, 4), exchange(t, 3, 5);
+    exchange(t, 3, 4);
+}
+
+// v after the products of ids t[0..K), ascending, kNoTag ids (at the end)
+// left out; t[0] and t[1] exist
+template <int K>
+__device__ __forceinline__ double apply_ids(const double *pa, const double *pb, const uint32_t (&t)[K], double v) {
+#pragma unroll
+    for (int g = 0; g < K; g += 4) {
+        double a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t q = g + i < 2 || t[g + i] != kNoTag ? t[g + i] : t[0];
+            a[i] = pa[q];
+            b[i] = pb[q];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double w = __fma_rn(a[i], b[i], v);
+            v = g + i < 2 || t[g + i] != kNoTag ? w : v;
+        }
     }
+    return v;
 }
 
 // Every word is written with a select, so the mask stays in registers
@@ -1239,7 +1283,7 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
             const uint32_t hmul = (W.c1 - W.c0) <= dense_width ? (1u << (32 - kLog)) : 0x9E3779B1u;
             int nfresh = 0;
             for (int32_t pb = a0, slot = 0; pb < a1; pb += NT, ++slot) {
-                if (tid < 2 * (NT / kWave)) (&L.smask[0][0])[tid] = 0ull;
+                clear_marks<NT>(L.smark[0], 2);
                 // this thread's k-slot: A entry p, B segment [s, e) inside the window
                 const int32_t p = pb + tid;
                 int32_t s = 0, e = 0;
@@ -1297,17 +1341,18 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                 const int32_t slen = e - s;
                 const int32_t excl = wg_excl_scan<NT>(slen, L.wsum, &total);
                 L.seg_d[tid] = s - excl;
-                // segment starts of the first two steps (their masks were
-                // cleared before the scan's barrier)
-                mark_segment<NT>(L.smask[0], L.smark[0], 0, excl, slen);
-                mark_segment<NT>(L.smask[1], L.smark[1], NT, excl, slen);
+                // segments of the first two steps (their marks were cleared
+                // before the scan's barrier)
+                mark_segment<NT>(L.smark[0], 0, excl, slen);
+                mark_segment<NT>(L.smark[1], NT, excl, slen);
                 __syncthreads();
                 // products x = x0 + tid, flattened in A-order; the B entry of the
                 // next step is loaded while the current step is applied
                 int32_t jn = 0;
                 double bn = 0.0, an = 0.0;
+                const int o0 = owner_marked(L.smark[0]);
                 if (tid < total) {
-                    const int o = owner_marked(L.smask[0], L.smark[0], tid);
+                    const int o = o0;
                     const int32_t q = L.seg_d[o] + tid;
                     an = av[pb + o];
                     jn = bi[q];
@@ -1333,14 +1378,14 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                         h = (off * hmul) >> (32 - kLog);
                         old = atomicCAS(&L.keytag[h], kSlotFree, me);
                     }
+                    const int o = owner_marked(L.smark[bA]);
                     if (xn < total) {
-                        const int o = owner_marked(L.smask[bA], L.smark[bA], tid);
                         const int32_t q = L.seg_d[o] + xn;
                         an = av[pb + o];
                         jn = bi[q];
                         bn = bv[q];
                     }
-                    if (tid < NT / kWave) L.smask[bC][tid] = 0ull;
+                    clear_marks<NT>(L.smark[bC], 1);
                     // insert: the first product of a slot in this step creates or
                     // claims it; every later one pushes itself onto the slot's
                     // list (the tag field holds the last pusher, link[] the rest)
@@ -1348,15 +1393,19 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                         const uint32_t off = key >> kTagBits;
                         // probe to a free slot (claimed) or this key's slot; the
                         // bound only guards a table the symbolic counts overfilled
-                        for (int probe = 1; old != kSlotFree && (old >> kTagBits) != off && probe < T; ++probe) {
-                            h = (h + 1) & (T - 1);
-                            old = atomicCAS(&L.keytag[h], kSlotFree, me);
+                        bool more = old != kSlotFree && (old >> kTagBits) != off;
+                        for (int probe = 1; probe < T && ballot(more); ++probe) {
+                            if (more) {
+                                h = (h + 1) & (T - 1);
+                                old = atomicCAS(&L.keytag[h], kSlotFree, me);
+                                more = old != kSlotFree && (old >> kTagBits) != off;
+                            }
                         }
                         uint32_t prev = kNoTag;
                         if (old == kSlotFree) {
                             L.vals[h] = 0.0;
                             ++nfresh;
-                        } else if ((old >> kTagBits) == off) {
+                        } else if (!more) {
                             prev = atomicExch(&L.keytag[h], me) & kNoTag;
                         } else {
                             atomicOr(&cnt->overflow, 8);  // table full: symbolic counts were wrong
@@ -1370,66 +1419,57 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                     }
                     __syncthreads();
                     // the last pusher of each slot applies the slot's products of
-                    // this step in thread (= A) order.  Each list member's
-                    // operands are read with its link; lists of up to three
-                    // are ordered in registers, longer ones walked through a
-                    // bitmask of thread ids (reading two or four operands per
-                    // round trip there measured 2% and 7% slower)
-                    if (act) {
-                        const uint32_t kt = L.keytag[h];
+                    // this step in thread (= A) order: it follows the slot's list,
+                    // sorts the thread ids in registers and reads the operands
+                    // in their order, all reads of four at once.  (R-MAT s19:
+                    // 78% of the products are alone in their slot, 14% in
+                    // pairs; a wave's longest list is over four in one step of
+                    // six, over eight in one of fifty.)  Longer lists walk a
+                    // bitmask of ids
+                    if (act && (L.keytag[h] & kNoTag) == (uint32_t)tid) {
                         const uint32_t t1 = L.link[tid];
                         double v = L.vals[h];
-                        if ((kt & kNoTag) == (uint32_t)tid) {
-                            if (t1 == kNoTag) {
-                                v = __fma_rn(ao, b, v);
+                        if (t1 == kNoTag) {
+                            v = __fma_rn(ao, b, v);
+                        } else {
+                            auto next = [&](uint32_t t) { return t == kNoTag ? kNoTag : (uint32_t)L.link[t]; };
+                            uint32_t t4[4] = {(uint32_t)tid, t1, L.link[t1], kNoTag};
+                            t4[3] = next(t4[2]);
+                            const uint32_t t5 = next(t4[3]);
+                            if (t5 == kNoTag) {
+                                sort_ids(t4);
+                                v = apply_ids(L.pa, L.pb, t4, v);
                             } else {
-                                const uint32_t t2 = L.link[t1];
-                                const double a1 = L.pa[t1], b1 = L.pb[t1];
-                                if (t2 == kNoTag) {
-                                    if ((uint32_t)tid < t1) {
-                                        v = __fma_rn(ao, b, v);
-                                        v = __fma_rn(a1, b1, v);
-                                    } else {
-                                        v = __fma_rn(a1, b1, v);
-                                        v = __fma_rn(ao, b, v);
-                                    }
+                                uint32_t t8[8] = {t4[0], t4[1], t4[2], t4[3], t5, kNoTag, kNoTag, kNoTag};
+#pragma unroll
+                                for (int i = 5; i < 8; ++i) t8[i] = next(t8[i - 1]);
+                                uint32_t t = next(t8[7]);
+                                if (t == kNoTag) {
+                                    sort_ids(t8);
+                                    v = apply_ids(L.pa, L.pb, t8, v);
                                 } else {
-                                    const uint32_t t3 = L.link[t2];
-                                    const double a2 = L.pa[t2], b2 = L.pb[t2];
-                                    if (t3 == kNoTag) {
-                                        uint32_t u0 = (uint32_t)tid, u1 = t1, u2 = t2;
-                                        double ea0 = ao, eb0 = b, ea1 = a1, eb1 = b1, ea2 = a2, eb2 = b2;
-                                        order_products(u0, ea0, eb0, u1, ea1, eb1);
-                                        order_products(u1, ea1, eb1, u2, ea2, eb2);
-                                        order_products(u0, ea0, eb0, u1, ea1, eb1);
-                                        v = __fma_rn(ea0, eb0, v);
-                                        v = __fma_rn(ea1, eb1, v);
-                                        v = __fma_rn(ea2, eb2, v);
-                                    } else {
-                                        uint64_t mk[NT / kWave];
+                                    uint64_t mk[NT / kWave];
 #pragma unroll
-                                        for (int w = 0; w < NT / kWave; ++w) mk[w] = 0ull;
-                                        mask_set<NT>(mk, (uint32_t)tid);
-                                        mask_set<NT>(mk, t1);
-                                        mask_set<NT>(mk, t2);
-                                        for (uint32_t t = t3; t != kNoTag; t = L.link[t]) mask_set<NT>(mk, t);
+                                    for (int w = 0; w < NT / kWave; ++w) mk[w] = 0ull;
 #pragma unroll
-                                        for (int w = 0; w < NT / kWave; ++w) {
-                                            uint64_t mw = mk[w];
-                                            while (mw) {
-                                                const int t = w * kWave + __ffsll((unsigned long long)mw) - 1;
-                                                mw &= mw - 1ull;
-                                                v = __fma_rn(L.pa[t], L.pb[t], v);
-                                            }
+                                    for (int i = 0; i < 8; ++i) mask_set<NT>(mk, t8[i]);
+                                    for (; t != kNoTag; t = L.link[t]) mask_set<NT>(mk, t);
+#pragma unroll
+                                    for (int w = 0; w < NT / kWave; ++w) {
+                                        uint64_t mw = mk[w];
+                                        while (mw) {
+                                            const int q = w * kWave + __ffsll((unsigned long long)mw) - 1;
+                                            mw &= mw - 1ull;
+                                            v = __fma_rn(L.pa[q], L.pb[q], v);
                                         }
                                     }
                                 }
                             }
-                            L.vals[h] = v;
-                            L.keytag[h] = key | kNoTag;
                         }
+                        L.vals[h] = v;
+                        L.keytag[h] = key | kNoTag;
                     }
-                    if (x0 + 2 * NT < total) mark_segment<NT>(L.smask[bC], L.smark[bC], x0 + 2 * NT, excl, slen);
+                    if (x0 + 2 * NT < total) mark_segment<NT>(L.smark[bC], x0 + 2 * NT, excl, slen);
                     __syncthreads();
                     bA = bC;
                     bC = bC == 2 ? 0 : bC + 1;

@@ -104,15 +104,6 @@ __device__ __forceinline__ int32_t segment_of(const int32_t *__restrict__ ptr, i
     return lo;
 }
 
-__device__ __forceinline__ int32_t wave_incl_max(int32_t v) {  // v >= 0
-    v = max(v, dpp<0x111>(v));
-    v = max(v, dpp<0x112>(v));
-    v = max(v, dpp<0x114>(v));
-    v = max(v, dpp<0x118>(v));
-    v = max(v, dpp<0x142, 0xa>(v));
-    return max(v, dpp<0x143, 0xc>(v));
-}
-
 template <bool kFirst, bool kLast>
 __global__ __launch_bounds__(kThreads) void k_radix_scatter(const Pass a) {
     // entries of a digit in the tile's waves before, then in the rounds before
@@ -171,7 +162,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const Pass a) {
                 m[u] = owner[tid * kPer + u];
                 if (u) m[u] = max(m[u], m[u - 1]);
             }
-            const int32_t inc = wave_incl_max(m[kPer - 1]);
+            const int32_t inc = (int32_t)wave_incl_max((uint32_t)m[kPer - 1]);
             int32_t run = __shfl_up(inc, 1, kWave);
             if (l == 0) run = 0;
             if (l == kWave - 1) top[w] = inc;
