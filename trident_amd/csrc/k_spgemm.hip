@@ -124,9 +124,11 @@ __device__ __forceinline__ void stream_cols(const TR_GLOBAL int32_t *__restrict_
 // Same visit with 16-byte loads for the aligned body of the segment (four
 // columns per lane per load, four loads in flight), scalar head and tail.
 // Alignment is taken from the address: caller tiles may place indices at any
-// 4-byte offset.  kEager issues the head, the tail and the first two groups
-// per lane at once (more registers: for kernels whose occupancy LDS bounds).
-template <bool kEager, typename F>
+// 4-byte offset.  Rows of up to 1024 columns, and the rest of longer ones, cost
+// one round trip: head, tail and the last four groups per lane are loaded
+// together (two to five trips before: the heavy symbolic of R-MAT s17 2245 ->
+// 1896 us, Galerkin 96^3 445 -> 380 us).
+template <typename F>
 __device__ __forceinline__ void stream_cols_v4(const TR_GLOBAL int32_t *__restrict__ bi, int32_t s, int32_t e,
                                                F &&f) {
     const int l = lane_id();
@@ -136,23 +138,7 @@ __device__ __forceinline__ void stream_cols_v4(const TR_GLOBAL int32_t *__restri
     typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
     const TR_GLOBAL i32x4 *__restrict__ b4 = (const TR_GLOBAL i32x4 *)(bi + sa);
     const int32_t ta = sa + (nv << 2);
-    if constexpr (kEager) {
-    // head, tail and the first two groups per lane are loaded together: a
-    // segment of up to 2 * 64 groups costs one round trip
-    const bool hh = s + l < sa, ht = ta + l < e, h0 = l < nv, h1 = l + kWave < nv;
-    int32_t jh = 0, jt = 0;
-    i32x4 g0 = {0, 0, 0, 0}, g1 = {0, 0, 0, 0};
-    if (hh) jh = bi[s + l];
-    if (ht) jt = bi[ta + l];
-    if (h0) g0 = b4[l];
-    if (h1) g1 = b4[l + kWave];
-    if (hh) f(jh);
-    if (ht) f(jt);
-    if (h0) f(g0.x), f(g0.y), f(g0.z), f(g0.w);
-    if (h1) f(g1.x), f(g1.y), f(g1.z), f(g1.w);
-    }
-    int32_t v = kEager ? l + 2 * kWave : l;
-    if (!kEager && s + l < sa) f(bi[s + l]);
+    int32_t v = l;
     for (; v + 3 * kWave < nv; v += 4 * kWave) {
         const i32x4 x0 = b4[v], x1 = b4[v + kWave], x2 = b4[v + 2 * kWave], x3 = b4[v + 3 * kWave];
         f(x0.x), f(x0.y), f(x0.z), f(x0.w);
@@ -160,17 +146,28 @@ __device__ __forceinline__ void stream_cols_v4(const TR_GLOBAL int32_t *__restri
         f(x2.x), f(x2.y), f(x2.z), f(x2.w);
         f(x3.x), f(x3.y), f(x3.z), f(x3.w);
     }
-    for (; v < nv; v += kWave) {
-        const i32x4 x = b4[v];
-        f(x.x), f(x.y), f(x.z), f(x.w);
-    }
-    if (!kEager && ta + l < e) f(bi[ta + l]);
+    const bool p0 = v < nv, p1 = v + kWave < nv, p2 = v + 2 * kWave < nv, p3 = v + 3 * kWave < nv;
+    const bool ph = s + l < sa, pt = ta + l < e;
+    i32x4 x0 = {0, 0, 0, 0}, x1 = x0, x2 = x0, x3 = x0;
+    int32_t xt = 0, xh = 0;
+    if (ph) xh = bi[s + l];
+    if (pt) xt = bi[ta + l];
+    if (p0) x0 = b4[v];
+    if (p1) x1 = b4[v + kWave];
+    if (p2) x2 = b4[v + 2 * kWave];
+    if (p3) x3 = b4[v + 3 * kWave];
+    if (ph) f(xh);
+    if (pt) f(xt);
+    if (p0) f(x0.x), f(x0.y), f(x0.z), f(x0.w);
+    if (p1) f(x1.x), f(x1.y), f(x1.z), f(x1.w);
+    if (p2) f(x2.x), f(x2.y), f(x2.z), f(x2.w);
+    if (p3) f(x3.x), f(x3.y), f(x3.z), f(x3.w);
 }
 
 // Streaming of B rows with their loads one round trip ahead, for kernels
 // whose LDS leaves registers to spare (the 2^20-bit heavy symbolic runs one
 // 16-wave workgroup per CU): each row's first round trip (its unaligned head
-// and tail and its first two 16-byte groups per lane, as stream_cols_v4<true>)
+// and tail and its first two 16-byte groups per lane)
 // is issued while the previous row is applied, and a long row's next 1024
 // columns while the current ones are.
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
@@ -473,7 +470,7 @@ template <int PB, int NTH>
 // few spilled bytes per lane): Galerkin 128^3 12.5 -> 12.0 ms, R-MAT s19
 // (2^19 columns) 17.8 -> 15.0 ms.
 __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 1) void k_sym_heavy(
-    const TaskDev *__restrict__ tasks, int nt, const int32_t *__restrict__ rows, Counters *__restrict__ cnt, int cls,
+    const TaskDev *__restrict__ tasks, int nt, Counters *__restrict__ cnt, int cls, int cls2,
     int64_t *__restrict__ rownnz, int emit, int32_t win_h, int32_t item_windows, int64_t item_flops,
     const int64_t *__restrict__ flops, Window *__restrict__ wins,
     int32_t win_cap, Item *__restrict__ items, int32_t item_cap, int32_t *__restrict__ lists, int32_t rows_total) {
@@ -499,9 +496,12 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
     const int tid = threadIdx.x, w = tid / kWave, l = lane_id();
     int32_t *fex_lds = (int32_t *)bm;            // [0, kFine) after marking
     int32_t *first_lds = (int32_t *)bm + kFine;  // [kFine, 2 kFine)
-    const int32_t nheavy = cnt->cls[cls];
+    // rows of class cls, then those of class cls2 (the same class: none)
+    const int32_t nfirst = cnt->cls[cls];
+    const int32_t nheavy = nfirst + (cls2 != cls ? cnt->cls[cls2] : 0);
     for (int32_t hi = blockIdx.x; hi < nheavy; hi += gridDim.x) {
-        const int32_t g = rows[hi];
+        const int32_t g = hi < nfirst ? lists[(int64_t)cls * rows_total + hi]
+                                      : lists[(int64_t)cls2 * rows_total + (hi - nfirst)];
         const TaskDev &TK = tasks[task_of(tasks, nt, g)];
         const int32_t r = g - TK.row_base;
         const TR_GLOBAL int32_t *__restrict__ ai = as_global(TK.ai);
@@ -530,15 +530,15 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
                 const int32_t rem = a1 - (pb + w);
                 const int nk = rem <= 0 ? 0 : min(kWave, (rem + kWavesB - 1) / kWavesB);
                 auto mark = [&](int32_t j) {
-                    const int64_t jj = (int64_t)j - base;
-                    if (jj >= 0 && jj < width) atomicOr(&bm[bm_word<kSwizzle>((int32_t)(jj >> 5))], 1u << (jj & 31));
+                    const uint32_t jj = (uint32_t)j - (uint32_t)base;  // (wraps for columns of earlier passes)
+                    if (jj < (uint32_t)width) atomicOr(&bm[bm_word<kSwizzle>((int32_t)(jj >> 5))], 1u << (jj & 31));
                 };
                 if constexpr (kEagerB) {
                     stream_rows_ahead(bi, bs, be, nk, mark);
                 } else {
                     for (int t = 0; t < nk; ++t) {
                         const int32_t s = __shfl(bs, t, kWave), e = __shfl(be, t, kWave);
-                        stream_cols_v4<false>(bi, s, e, mark);
+                        stream_cols_v4(bi, s, e, mark);
                     }
                 }
             }
@@ -1830,9 +1830,10 @@ int64_t item_flops(const tr_ctx *ctx, const MulPlan &pl) {
 }
 
 template <int PB, int NTH>
-void launch_sym_heavy(tr_ctx *ctx, MulPlan &pl, int cls, int per_cu, bool emit) {
-    TR_LAUNCH(ctx, "sym_heavy", (k_sym_heavy<PB, NTH>), cap_grid(pl.h.cls[cls], (int64_t)ctx->cu_count * per_cu), NTH,
-              0, pl.d_tasks, pl.nt, pl.lists + (int64_t)cls * pl.rows_total, pl.cnt, cls, pl.rownnz, emit ? 1 : 0,
+void launch_sym_heavy(tr_ctx *ctx, MulPlan &pl, int cls, int cls2, int per_cu, bool emit) {
+    const int64_t n = (int64_t)pl.h.cls[cls] + (cls2 != cls ? pl.h.cls[cls2] : 0);
+    TR_LAUNCH(ctx, "sym_heavy", (k_sym_heavy<PB, NTH>), cap_grid(n, (int64_t)ctx->cu_count * per_cu), NTH,
+              0, pl.d_tasks, pl.nt, pl.cnt, cls, cls2, pl.rownnz, emit ? 1 : 0,
               pl.tune.window_entries, pl.tune.item_windows, item_flops(ctx, pl), pl.flops, pl.wins, pl.win_cap,
               pl.items, pl.item_cap, pl.lists, pl.rows_total);
 }
@@ -1872,14 +1873,14 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
         // first (Galerkin 128^3: 12.9 -> 12.3 ms against one resident wave
         // of workgroups).
         const int pb = max_n <= (1 << 18) ? 18 : max_n <= (1 << 19) ? 19 : kPassBits;
-        if (pl.h.cls[kHeavyClass]) {
-            if (pb == 18) launch_sym_heavy<18, kMidThreads>(ctx, pl, kHeavyClass, 64, emit);
-            else if (pb == 19) launch_sym_heavy<19, kHeavyThreads>(ctx, pl, kHeavyClass, 32, emit);
-            else launch_sym_heavy<kPassBits, kHeavyThreads>(ctx, pl, kHeavyClass, 32, emit);
-        }
-        if (pl.h.cls[kMidClass]) {
-            if (pb == 18) launch_sym_heavy<18, kMidThreads>(ctx, pl, kMidClass, 64, emit);
-            else launch_sym_heavy<kMidPassBits, kHeavyThreads>(ctx, pl, kMidClass, 32, emit);
+        // Up to 2^19 columns both classes share a kernel, the heaviest rows
+        // first, in one launch: the lighter rows fill the end of the heavier
+        // ones (R-MAT s17 1896 -> 1410 us, 15013 vertices 218 -> 179 us).
+        if (pb == 18) launch_sym_heavy<18, kMidThreads>(ctx, pl, kHeavyClass, kMidClass, 64, emit);
+        else if (pb == 19) launch_sym_heavy<19, kHeavyThreads>(ctx, pl, kHeavyClass, kMidClass, 32, emit);
+        else {
+            launch_sym_heavy<kPassBits, kHeavyThreads>(ctx, pl, kHeavyClass, kHeavyClass, 32, emit);
+            launch_sym_heavy<kMidPassBits, kHeavyThreads>(ctx, pl, kMidClass, kMidClass, 32, emit);
         }
     }
     launch_exclusive_scan_i64(ctx, pl.rownnz, pl.rowptr, pl.rows_total, pl.scan_tmp);
