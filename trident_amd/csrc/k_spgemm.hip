@@ -309,6 +309,13 @@ __global__ void k_put_task(TaskDev *__restrict__ dst, const TaskDev t, Counters 
     if (threadIdx.x == 0) *dst = t;
 }
 
+// light class of n: the smallest c with 2 n <= 64 << c
+__device__ __forceinline__ int light_class(int64_t n) {
+    int c = 0;
+    while ((int64_t)(64 << c) < 2 * n) ++c;
+    return c;
+}
+
 __global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__restrict__ tasks, int nt,
                                                             int32_t rows_total, const int64_t *__restrict__ flops,
                                                             int64_t *__restrict__ rownnz,
@@ -342,13 +349,10 @@ __global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__res
         lpos[u] = 0;
         if (f[u] > 0) {
             if (f[u] <= light_max) {
-                const int64_t bound = f[u] < ncols[u] ? f[u] : ncols[u];
-                int64_t T = 64;
-                c[u] = 0;
-                while (T < 2 * bound) {
-                    T <<= 1;
-                    ++c[u];
-                }
+                // by the entries it may have, or, beyond the hashed classes, by
+                // its products (all held at once by the numeric)
+                c[u] = light_class(min(f[u], (int64_t)ncols[u]));
+                if (c[u] > kHashClassMax) c[u] = light_class(f[u]);
             } else {
                 c[u] = f[u] <= kMidMaxF ? kMidClass : kHeavyClass;
                 shf += f[u];
@@ -1061,6 +1065,258 @@ __global__ __launch_bounds__(WPB * kWave, T <= 256 ? 8 : 1) void k_num_light(con
             ov[t] = vals[t];
         }
         wave_sync();
+    }
+}
+
+// ---------------------------------------------------------------- numeric, light rows by sorting
+// Rows of 129 to 1024 multiplications that did not come from the heavy
+// symbolic: all products of a row at once, four per thread (NT = 64, 128 or 256
+// threads a row).  The products are flattened in A-order, sorted in registers by
+// (column, position), and every column's run is summed in position (= A) order
+// by the thread that holds its first product; the runs in order are the sorted
+// output.
+//
+// What bounds it: the sort, about 3.5 vector instructions per product and step
+// (strides inside a thread are minimum and maximum, inside a wave DPP moves and
+// permlane swaps; only strides of a wave and more go through LDS).  The hash
+// tables that these rows had held one wave to 12 or 24 KiB of LDS (6 to 13 waves
+// per CU), walked A's entries one after the other and sorted the table in LDS:
+// stage of R-MAT s18 2671 us for the three classes, now 481 us (22 KiB for a row
+// of 256 threads: 28 waves per CU); tile accumulate of R-MAT s16 154 -> 33 us.
+constexpr int kSortPer = 4;        // products per thread
+constexpr int kSortIdBits = 10;    // product positions < 1024
+
+template <typename K>
+__device__ __forceinline__ void order_pair(K &a, K &b, bool up) {
+    const K lo = a < b ? a : b, hi = a < b ? b : a;
+    a = up ? lo : hi;
+    b = up ? hi : lo;
+}
+
+// One step of the bitonic sort of NT * kSortPer keys, key u of thread t at
+// position t * kSortPer + u, then the smaller strides of the same size.
+template <int NT, int kSize, int kStride, typename K>
+__device__ __forceinline__ void sort_step(K (&key)[kSortPer], K *lds, int t) {
+    constexpr int P = kSortPer;
+    if constexpr (kStride < P) {
+#pragma unroll
+        for (int u = 0; u < P; ++u)
+            if (!(u & kStride)) {
+                const bool up = kSize < P ? (u & kSize) == 0 : (t & (kSize / P)) == 0;
+                order_pair(key[u], key[u | kStride], up);
+            }
+    } else {
+        constexpr int X = kStride / P;  // thread distance
+        const bool keep_min = ((t & X) == 0) == ((t & (kSize / P)) == 0);
+        if constexpr (X < kWave) {
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                const K o = lane_xor<X>(key[u]);
+                key[u] = (o < key[u]) == keep_min ? o : key[u];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < P; ++u) lds[u * NT + t] = key[u];
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                const K o = lds[u * NT + (t ^ X)];
+                key[u] = (o < key[u]) == keep_min ? o : key[u];
+            }
+            __syncthreads();
+        }
+    }
+    if constexpr (kStride > 1) sort_step<NT, kSize, kStride / 2>(key, lds, t);
+}
+
+template <int NT, int kSize = 2, typename K>
+__device__ __forceinline__ void sort_products(K (&key)[kSortPer], K *lds, int t) {
+    sort_step<NT, kSize, kSize / 2>(key, lds, t);
+    if constexpr (kSize < NT * kSortPer) sort_products<NT, kSize * 2>(key, lds, t);
+}
+
+// barrier of a row's threads
+template <int NT>
+__device__ __forceinline__ void row_sync() {
+    if constexpr (NT > kWave) __syncthreads();
+    else wave_sync();
+}
+
+template <int NT, typename K>
+struct SortLds {
+    static constexpr int kMax = NT * kSortPer;
+    double pa[kMax];  // by a B row's first position: its A value; then by position: the product's
+    double pb[kMax];
+    union {
+        int32_t sq[kMax];  // by a B row's first position: B position minus product position
+        K key[kMax];       // sorted keys
+    };
+    uint16_t mark[kMax];  // a B row's first position + 1, else 0
+    int32_t part[2][NT / kWave];
+};
+
+template <int NT, int WPB, typename K>
+__global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict__ tasks, int nt,
+                                                      const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
+                                                      int cls, const int64_t *__restrict__ rowptr,
+                                                      const Panel *__restrict__ panels, int npanels) {
+    static_assert(NT > kWave ? WPB == 1 : NT == kWave, "a row's threads are a workgroup or a wave of it");
+    constexpr int P = kSortPer, kMax = NT * P, kWaves = NT / kWave;
+    static_assert(kMax <= 1 << kSortIdBits, "positions fit their key bits");
+    constexpr K kIdMask = ((K)1 << kSortIdBits) - 1;
+    __shared__ SortLds<NT, K> lds_s[WPB];
+    const int sub = NT > kWave ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // row of the workgroup
+    const int t = threadIdx.x % NT, l = lane_id();
+    const int w = NT > kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;    // wave of the row
+    SortLds<NT, K> &L = lds_s[sub];
+    const int32_t nrows = cnt->cls[cls];
+    for (int32_t li = blockIdx.x * WPB + sub; li < nrows; li += gridDim.x * WPB) {
+        const int32_t g = __builtin_amdgcn_readfirstlane(rows[li]);
+        const TaskDev &TK = tasks[task_of(tasks, nt, g)];
+        const int32_t r = g - TK.row_base;
+        const TR_GLOBAL int32_t *__restrict__ ai = as_global(TK.ai);
+        const TR_GLOBAL double *__restrict__ av = as_global(TK.av);
+        const TR_GLOBAL int32_t *__restrict__ bp = as_global(TK.bp);
+        const TR_GLOBAL int32_t *__restrict__ bi = as_global(TK.bi);
+        const TR_GLOBAL double *__restrict__ bv = as_global(TK.bv);
+        const int32_t a0 = as_global(TK.ap)[r], a1 = as_global(TK.ap)[r + 1];
+        *reinterpret_cast<uint2 *>(&L.mark[t * P]) = make_uint2(0u, 0u);
+        row_sync<NT>();
+        // B rows of A's entries, flattened: each non-empty one is entered at its
+        // first product position
+        int32_t total = 0;
+        for (int32_t pb = a0, turn = 0; pb < a1; pb += NT, turn ^= 1) {
+            int32_t bs = 0, len = 0;
+            double a = 0.0;
+            if (pb + t < a1) {
+                const int32_t k = ai[pb + t];
+                a = av[pb + t];
+                bs = bp[k];
+                len = bp[k + 1] - bs;
+            }
+            const int32_t inc = wave_incl_scan(len);
+            int32_t pos = total + inc - len;
+            if constexpr (kWaves > 1) {
+                if (l == kWave - 1) L.part[turn][w] = inc;
+                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < kWaves; ++u) {
+                    const int32_t s = L.part[turn][u];
+                    pos += u < w ? s : 0;
+                    total += s;
+                }
+            } else {
+                total += read_lane(inc, kWave - 1);
+            }
+            if (len > 0 && pos < kMax) {
+                L.mark[pos] = (uint16_t)(pos + 1);
+                L.sq[pos] = bs - pos;
+                L.pa[pos] = a;
+            }
+        }
+        total = min(total, kMax);  // (the row's class bounds it)
+        row_sync<NT>();
+        // this thread's products t P .. t P + P - 1: the last mark at or below
+        uint32_t m[P];
+        {
+            const uint2 q = *reinterpret_cast<const uint2 *>(&L.mark[t * P]);
+            m[0] = q.x & 0xffffu;
+            m[1] = max(m[0], q.x >> 16);
+            m[2] = max(m[1], q.y & 0xffffu);
+            m[3] = max(m[2], q.y >> 16);
+            const uint32_t inc = wave_incl_max(m[3]);
+            uint32_t before = dpp<0x138>(inc);  // the lane below; 0 for lane 0
+            if constexpr (kWaves > 1) {
+                // (the entries' last use of `part` is behind the barrier above)
+                if (l == kWave - 1) L.part[0][w] = (int32_t)inc;
+                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < kWaves - 1; ++u) before = max(before, u < w ? (uint32_t)L.part[0][u] : 0u);
+            }
+#pragma unroll
+            for (int u = 0; u < P; ++u) m[u] = max(m[u], before);
+        }
+        K key[P];
+        double pa[P], pbv[P];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const int32_t x = t * P + u;
+            key[u] = ~(K)0;
+            pa[u] = pbv[u] = 0.0;
+            if (x < total) {
+                const uint32_t s = m[u] - 1;
+                const int32_t q = L.sq[s] + x;
+                pa[u] = L.pa[s];
+                key[u] = (K)(uint32_t)bi[q] << kSortIdBits | (K)x;
+                pbv[u] = bv[q];
+            }
+        }
+        row_sync<NT>();  // sq and the A values by first position are read
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            L.pa[t * P + u] = pa[u];
+            L.pb[t * P + u] = pbv[u];
+        }
+        sort_products<NT>(key, L.key, t);
+#pragma unroll
+        for (int u = 0; u < P; ++u) L.key[t * P + u] = key[u];
+        row_sync<NT>();
+        // columns that begin in this thread, and their places
+        K prev = t > 0 ? L.key[t * P - 1] : 0;
+        int32_t nhead = 0, first = P;
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const int32_t x = t * P + u;
+            if (x < total && (x == 0 || (prev >> kSortIdBits) != (key[u] >> kSortIdBits))) {
+                if (nhead == 0) first = u;
+                ++nhead;
+            }
+            prev = key[u];
+        }
+        const int32_t inc = wave_incl_scan(nhead);
+        int32_t rank = inc - nhead, n = 0;
+        if constexpr (kWaves > 1) {
+            if (l == kWave - 1) L.part[1][w] = inc;
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < kWaves; ++u) {
+                const int32_t s = L.part[1][u];
+                rank += u < w ? s : 0;
+                n += s;
+            }
+        } else {
+            n = read_lane(inc, kWave - 1);
+        }
+        const int64_t rs = rowptr[g];
+        const int32_t expect = (int32_t)(rowptr[g + 1] - rs);
+        const Panel &PN = find_panel(panels, npanels, g);
+        if (t == 0 && n != expect) atomicOr(&cnt->overflow, 2);
+        TR_GLOBAL int32_t *oi = as_global(PN.idx) + (rs - PN.nnz_begin);
+        TR_GLOBAL double *ov = as_global(PN.val) + (rs - PN.nnz_begin);
+        if (nhead > 0) {
+            int32_t x = t * P + first;
+            K col = L.key[x] >> kSortIdBits;
+            double v = 0.0;
+            while (true) {
+                const K k = L.key[x];
+                const uint32_t id = (uint32_t)(k & kIdMask);
+                v = __fma_rn(L.pa[id], L.pb[id], v);
+                ++x;
+                const bool more = x < total;
+                const K next = more ? L.key[x] >> kSortIdBits : 0;
+                if (!more || next != col) {
+                    if (rank < expect) {  // never write past the row
+                        oi[rank] = (int32_t)col;
+                        ov[rank] = v;
+                    }
+                    ++rank;
+                    if (!more || x >= t * P + P) break;  // the next column begins in another thread
+                    col = next;
+                    v = 0.0;
+                }
+            }
+        }
+        row_sync<NT>();  // the next row rewrites the arrays
     }
 }
 
@@ -1948,13 +2204,34 @@ void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np) {
     TR_LAUNCH(ctx, "panel_bases", k_panel_bases, div_up((uint64_t)np, 64), 64, 0, d_panels, np, pl.rowptr);
 }
 
+namespace {
+
+template <int NT, typename K>
+void launch_num_sort_as(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
+    constexpr int kWpb = NT > kWave ? 1 : 4;
+    const int32_t n = pl.h.cls[c];
+    TR_LAUNCH(ctx, "num_light", (k_num_sort<NT, kWpb, K>), cap_grid(div_up((uint64_t)n, kWpb), 1 << 20), NT * kWpb, 0,
+              pl.d_tasks, pl.nt, pl.lists + (int64_t)c * pl.rows_total, pl.cnt, c, pl.rowptr, panels, np);
+}
+
+// (column, position) keys of 32 bits where every column fits
+template <int NT>
+void launch_num_sort(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
+    int32_t max_n = 0;
+    for (const TaskDev &t : pl.h_tasks) max_n = std::max(max_n, t.n);
+    if (max_n <= 1 << (32 - kSortIdBits)) launch_num_sort_as<NT, uint32_t>(ctx, pl, c, panels, np);
+    else launch_num_sort_as<NT, uint64_t>(ctx, pl, c, panels, np);
+}
+
+}  // namespace
+
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *dp, int np) {
     if (pl.h.cls[0]) launch_num_light<64>(ctx, pl, 0, dp, np);
     if (pl.h.cls[1]) launch_num_light<128>(ctx, pl, 1, dp, np);
     if (pl.h.cls[2]) launch_num_light<256>(ctx, pl, 2, dp, np);
-    if (pl.h.cls[3]) launch_num_light<512>(ctx, pl, 3, dp, np);
-    if (pl.h.cls[4]) launch_num_light<1024>(ctx, pl, 4, dp, np);
-    if (pl.h.cls[5]) launch_num_light<2048>(ctx, pl, 5, dp, np);
+    if (pl.h.cls[3]) launch_num_sort<64>(ctx, pl, 3, dp, np);
+    if (pl.h.cls[4]) launch_num_sort<128>(ctx, pl, 4, dp, np);
+    if (pl.h.cls[5]) launch_num_sort<256>(ctx, pl, 5, dp, np);
     if (pl.h.items > 0) {
         // one workgroup per item, grid-stride beyond 2^22 workgroups (the
         // dispatch packet counts work-items in 32 bits)

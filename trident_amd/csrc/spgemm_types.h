@@ -13,6 +13,7 @@ namespace tr {
 // tuning constants
 constexpr int kLightMaxFCap = 1024; // largest light/heavy cut (light tables reach 2048 slots)
 constexpr int kNumLight = 6;       // light classes: T = 64 << c, c < kNumLight
+constexpr int kHashClassMax = 2;   // light rows up to this class are hashed by the numeric, the others sorted
 constexpr int kHeavyClass = kNumLight;      // heavy rows with more than kMidMaxF multiplications
 constexpr int kMidClass = kNumLight + 1;    // heavy rows up to kMidMaxF multiplications
 constexpr int kNumClasses = kNumLight + 2;
