@@ -16,11 +16,11 @@
 //                    appends them to a device work list.
 //  3. scan           row counts -> 64-bit row offsets; C is cut into int32
 //                    tiles (panels) when it exceeds INT32_MAX entries.
-//  4. numeric        light rows: one wave per row, LDS hash of (key, fp64),
-//                    A's entries walked in stored order with the lanes over
-//                    B_k (no two lanes share a column, so values need no
-//                    atomics and every output sees its products in order);
-//                    light rows are compacted and bitonic-sorted in LDS;
+//  4. numeric        light rows: all products of a row at once, sorted in
+//                    registers by (column, position in A-order) and summed
+//                    run by run;
+//                    compact heavy rows (at most 128 entries): one wave per
+//                    row, LDS hash of (key, fp64), compacted and sorted;
 //                    heavy rows: one workgroup per item (a run of windows of
 //                    one row) sharing one LDS table per window, products of
 //                    the window flattened over the workgroup in A-order,
@@ -316,8 +316,7 @@ __device__ __forceinline__ int light_class(int64_t n) {
     return c;
 }
 
-__global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__restrict__ tasks, int nt,
-                                                            int32_t rows_total, const int64_t *__restrict__ flops,
+__global__ __launch_bounds__(kClassThreads) void k_classify(int32_t rows_total, const int64_t *__restrict__ flops,
                                                             int64_t *__restrict__ rownnz,
                                                             int32_t *__restrict__ lists, Counters *__restrict__ cnt,
                                                             int32_t light_max) {
@@ -330,14 +329,11 @@ __global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__res
     if (tid == 0) s_f = s_hf = 0ull;
     __syncthreads();
     int64_t f[kPer], sf = 0, shf = 0;
-    int32_t ncols[kPer];
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
         const int32_t g = g0 + u * kClassThreads;
         f[u] = 0;
-        ncols[u] = 0;
         if (g < rows_total) {
-            ncols[u] = tasks[task_of(tasks, nt, g)].n;
             f[u] = flops[g];
             rownnz[g] = 0;
         }
@@ -349,10 +345,7 @@ __global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__res
         lpos[u] = 0;
         if (f[u] > 0) {
             if (f[u] <= light_max) {
-                // by the entries it may have, or, beyond the hashed classes, by
-                // its products (all held at once by the numeric)
-                c[u] = light_class(min(f[u], (int64_t)ncols[u]));
-                if (c[u] > kHashClassMax) c[u] = light_class(f[u]);
+                c[u] = light_class(f[u]);
             } else {
                 c[u] = f[u] <= kMidMaxF ? kMidClass : kHeavyClass;
                 shf += f[u];
@@ -595,12 +588,12 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
             }
             // A row done in one pass whose product has few entries (many
             // multiplications per entry: the coarse Galerkin product has about
-            // 55) goes to the light numeric, whose small table and lane-mask
-            // ordering suit it, instead of to windows: appended to the light
-            // class whose table holds twice its entries.
+            // 55) goes to the hashed light numeric, whose small table and
+            // lane-mask ordering suit it, instead of to windows: appended to
+            // the compact class whose table holds twice its entries.
             if (ncols <= (1 << PB) && pass_total <= kCompactMax) {
                 if (tid == 0) {
-                    const int c = pass_total <= 32 ? 0 : pass_total <= 64 ? 1 : 2;
+                    const int c = kCompactClass + (pass_total <= 32 ? 0 : pass_total <= 64 ? 1 : 2);
                     const int32_t pos = atomicAdd(&cnt->cls[c], 1);
                     lists[(int64_t)c * rows_total + pos] = g;
                 }
@@ -821,40 +814,34 @@ __global__ void k_tile_ptr(const int64_t *__restrict__ rowptr, int32_t r0, int32
     if (t <= n) ptr[t] = (int32_t)(rowptr[r0 + t] - rowptr[r0]);
 }
 
-// ---------------------------------------------------------------- numeric, light rows
-constexpr int kLightPre = 4;  // B rows prefetched together per batch of a light row
+// ---------------------------------------------------------------- numeric, compact rows
+// Rows of many multiplications over at most 128 columns (found by the heavy
+// symbolic): one wave per row with a hash table of at least twice its entries.
+constexpr int kLightPre = 4;  // B rows prefetched together per batch of a row
 
-// WPB waves per block, one row per wave (big tables use one-wave blocks so
-// that LDS, not the block shape, bounds the waves per CU)
 template <int T, int WPB>
-// Tables of <= 256 slots leave LDS for 8 waves per SIMD; the registers are
-// held to that too (63 VGPRs, 12 spilled bytes per lane; about 1% on stage
-// 22:3 and Galerkin 128^3 against 65 VGPRs and 7 waves).
-__global__ __launch_bounds__(WPB * kWave, T <= 256 ? 8 : 1) void k_num_light(const TaskDev *__restrict__ tasks, int nt,
+// The tables leave LDS for 8 waves per SIMD; the registers are held to that
+// too (63 VGPRs, 12 spilled bytes per lane; about 1% on Galerkin 128^3 against
+// 65 VGPRs and 7 waves).
+__global__ __launch_bounds__(WPB * kWave, 8) void k_num_light(const TaskDev *__restrict__ tasks, int nt,
                                                            const int32_t *__restrict__ rows,
                                                            Counters *__restrict__ cnt, int cls,
                                                            const int64_t *__restrict__ rowptr,
                                                            const Panel *__restrict__ panels, int npanels) {
-    // tables of <= 512 slots also flatten chunks of short B rows over the
-    // lanes; per-slot words order the chunk's products: lane masks (<= 256
-    // slots) or owner lanes (512 slots, where 64-bit masks would cost
-    // occupancy)
-    constexpr bool kFlat = T <= 512;
-    constexpr bool kMask = T <= 256;
-    constexpr int kOwn = kFlat ? T : 1;
-    using OwnT = typename std::conditional<kMask, unsigned long long, uint32_t>::type;
+    // chunks of short B rows are flattened over the lanes; a lane mask per slot
+    // orders the chunk's products
+    static_assert(T <= 256, "lane masks of larger tables would cost occupancy");
     __shared__ int32_t keys_s[WPB][T];
     __shared__ double vals_s[WPB][T];
-    __shared__ OwnT own_s[WPB][kOwn];
+    __shared__ unsigned long long own_s[WPB][T];
     constexpr uint32_t kLog = __builtin_ctz(T);
     // the wave index and everything per row are wave-uniform (scalar loads
     // and registers)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), l = lane_id();
     int32_t *keys = keys_s[w];
     double *vals = vals_s[w];
-    OwnT *own = own_s[w];
-    if (kFlat)
-        for (int t = l; t < kOwn; t += kWave) own[t] = kMask ? 0 : kWave;
+    unsigned long long *own = own_s[w];
+    for (int t = l; t < T; t += kWave) own[t] = 0ull;
     const int32_t nrows = cnt->cls[cls];
     const int32_t stride = gridDim.x * WPB;
     int32_t g_next = 0;
@@ -888,124 +875,109 @@ __global__ __launch_bounds__(WPB * kWave, T <= 256 ? 8 : 1) void k_num_light(con
                 be = bp[k + 1];
             }
             const int nk = min(kWave, a1 - pb);
-            if (kFlat) {
-                const int32_t len = be - bs;
-                const int32_t inc = wave_incl_scan(len);
-                const int32_t total = __shfl(inc, kWave - 1, kWave);
-                if (total < 24 * nk) {
-                    // Short B rows: 64 products of the chunk per round, flattened
-                    // in A-order over the lanes (product x belongs to the last
-                    // lane whose prefix is <= x).  Products that meet in a slot
-                    // are applied in lane (= A) order: each pass, the lowest
-                    // pending lane of every slot applies its product.
-                    const int32_t excl = inc - len;
-                    for (int32_t x0 = 0; x0 < total; x0 += kWave) {
-                        const int32_t x = x0 + l;
-                        int t = 0;
-                        int32_t q;
-                        if constexpr (kMask && T >= 2 * kWave) {
-                            // The lanes whose B rows meet this round write (lane,
-                            // B offset) at the position where their rows start in
-                            // it (or 0) and mark it in a start mask; position x
-                            // belongs to the highest start at or below it.  The
-                            // first 65 lane-mask words, all zero between rounds,
-                            // hold both and are cleared again before the round
-                            // uses them.  Three round trips instead of the six
-                            // dependent shuffles of a search over the lanes.
-                            const bool meets = len > 0 && excl < x0 + kWave && excl + len > x0;
-                            const int32_t pos = max(excl - x0, 0);
-                            if (meets) {
-                                own[pos] = ((unsigned long long)(uint32_t)l << 32) | (uint32_t)(bs - excl);
-                                atomicOr(&own[kWave], 1ull << pos);
-                            }
-                            wave_sync();
-                            const unsigned long long starts = own[kWave] & (~0ull >> (63 - l));
-                            const unsigned long long e = own[63 - __clzll((long long)starts)];
-                            t = (int)(e >> 32);
-                            q = (int32_t)(uint32_t)e + x;
-                            wave_sync();
-                            own[l] = 0ull;
-                            if (l == 0) own[kWave] = 0ull;
-                            wave_sync();
-                        } else {
-#pragma unroll
-                            for (int step = kWave / 2; step > 0; step >>= 1)
-                                if (__shfl(excl, t + step, kWave) <= x) t += step;
-                            q = __shfl(bs, t, kWave) + (x - __shfl(excl, t, kWave));
-                        }
-                        const double at = __shfl(a, t, kWave);
-                        bool pend = x < total;
-                        uint32_t h = 0;
-                        double b = 0.0;
-                        if (pend) {
-                            const int32_t j = bi[q];
-                            b = bv[q];
-                            h = hash_slot(j, kLog);
-                            bool placed = false;
-                            for (int probe = 0; probe < T; ++probe) {
-                                const int32_t old = atomicCAS(&keys[h], kEmpty, j);
-                                if (old == kEmpty) {
-                                    vals[h] = 0.0;
-                                    placed = true;
-                                    break;
-                                }
-                                if (old == j) {
-                                    placed = true;
-                                    break;
-                                }
-                                h = (h + 1) & (T - 1);
-                            }
-                            if (!placed) {
-                                atomicOr(&cnt->overflow, 2);  // table full: symbolic counts were wrong
-                                pend = false;
-                            }
+            const int32_t len = be - bs;
+            const int32_t inc = wave_incl_scan(len);
+            const int32_t total = __shfl(inc, kWave - 1, kWave);
+            if (total < 24 * nk) {
+                // Short B rows: 64 products of the chunk per round, flattened
+                // in A-order over the lanes (product x belongs to the last
+                // lane whose prefix is <= x).  Products that meet in a slot
+                // are applied in lane (= A) order: each pass, the lowest
+                // pending lane of every slot applies its product.
+                const int32_t excl = inc - len;
+                for (int32_t x0 = 0; x0 < total; x0 += kWave) {
+                    const int32_t x = x0 + l;
+                    int t = 0;
+                    int32_t q;
+                    if constexpr (T >= 2 * kWave) {
+                        // The lanes whose B rows meet this round write (lane,
+                        // B offset) at the position where their rows start in
+                        // it (or 0) and mark it in a start mask; position x
+                        // belongs to the highest start at or below it.  The
+                        // first 65 lane-mask words, all zero between rounds,
+                        // hold both and are cleared again before the round
+                        // uses them.  Three round trips instead of the six
+                        // dependent shuffles of a search over the lanes.
+                        const bool meets = len > 0 && excl < x0 + kWave && excl + len > x0;
+                        const int32_t pos = max(excl - x0, 0);
+                        if (meets) {
+                            own[pos] = ((unsigned long long)(uint32_t)l << 32) | (uint32_t)(bs - excl);
+                            atomicOr(&own[kWave], 1ull << pos);
                         }
                         wave_sync();
-                        if constexpr (kMask) {
-                            // each slot's lanes as a mask; its lowest lane
-                            // applies them all in lane order, fetching the
-                            // other lanes' operands across the wave
-                            if (pend) atomicOr(&own[h], 1ull << l);
-                            wave_sync();
-                            unsigned long long rem = 0ull;
-                            double v = 0.0;
-                            if (pend) {
-                                const unsigned long long m = own[h];
-                                if (__ffsll(m) - 1 == l) {
-                                    rem = m;
-                                    v = vals[h];
-                                }
+                        const unsigned long long starts = own[kWave] & (~0ull >> (63 - l));
+                        const unsigned long long e = own[63 - __clzll((long long)starts)];
+                        t = (int)(e >> 32);
+                        q = (int32_t)(uint32_t)e + x;
+                        wave_sync();
+                        own[l] = 0ull;
+                        if (l == 0) own[kWave] = 0ull;
+                        wave_sync();
+                    } else {
+#pragma unroll
+                        for (int step = kWave / 2; step > 0; step >>= 1)
+                            if (__shfl(excl, t + step, kWave) <= x) t += step;
+                        q = __shfl(bs, t, kWave) + (x - __shfl(excl, t, kWave));
+                    }
+                    const double at = __shfl(a, t, kWave);
+                    bool pend = x < total;
+                    uint32_t h = 0;
+                    double b = 0.0;
+                    if (pend) {
+                        const int32_t j = bi[q];
+                        b = bv[q];
+                        h = hash_slot(j, kLog);
+                        bool placed = false;
+                        for (int probe = 0; probe < T; ++probe) {
+                            const int32_t old = atomicCAS(&keys[h], kEmpty, j);
+                            if (old == kEmpty) {
+                                vals[h] = 0.0;
+                                placed = true;
+                                break;
                             }
-                            while (ballot(rem != 0ull)) {  // every lane takes part in the fetches
-                                const int t = rem ? __ffsll(rem) - 1 : l;
-                                const double ta = __shfl(at, t, kWave);
-                                const double tb = __shfl(b, t, kWave);
-                                if (rem) {
-                                    v = __fma_rn(ta, tb, v);
-                                    rem &= rem - 1ull;
-                                }
+                            if (old == j) {
+                                placed = true;
+                                break;
                             }
-                            wave_sync();
-                            if (pend && (__ffsll(own[h]) - 1 == l)) {
-                                vals[h] = v;
-                                own[h] = 0ull;
-                            }
-                            wave_sync();
-                        } else {
-                            while (ballot(pend)) {
-                                if (pend) atomicMin(&own[h], (uint32_t)l);
-                                wave_sync();
-                                if (pend && own[h] == (uint32_t)l) {
-                                    vals[h] = __fma_rn(at, b, vals[h]);
-                                    own[h] = kWave;
-                                    pend = false;
-                                }
-                                wave_sync();
-                            }
+                            h = (h + 1) & (T - 1);
+                        }
+                        if (!placed) {
+                            atomicOr(&cnt->overflow, 2);  // table full: symbolic counts were wrong
+                            pend = false;
                         }
                     }
-                    continue;
+                    wave_sync();
+                    // each slot's lanes as a mask; its lowest lane
+                    // applies them all in lane order, fetching the
+                    // other lanes' operands across the wave
+                    if (pend) atomicOr(&own[h], 1ull << l);
+                    wave_sync();
+                    unsigned long long rem = 0ull;
+                    double v = 0.0;
+                    if (pend) {
+                        const unsigned long long m = own[h];
+                        if (__ffsll(m) - 1 == l) {
+                            rem = m;
+                            v = vals[h];
+                        }
+                    }
+                    while (ballot(rem != 0ull)) {  // every lane takes part in the fetches
+                        const int t = rem ? __ffsll(rem) - 1 : l;
+                        const double ta = __shfl(at, t, kWave);
+                        const double tb = __shfl(b, t, kWave);
+                        if (rem) {
+                            v = __fma_rn(ta, tb, v);
+                            rem &= rem - 1ull;
+                        }
+                    }
+                    wave_sync();
+                    if (pend && (__ffsll(own[h]) - 1 == l)) {
+                        vals[h] = v;
+                        own[h] = 0ull;
+                    }
+                    wave_sync();
                 }
+                continue;
             }
             auto ins = [&](int32_t j, double b, double at) {
                 uint32_t h = hash_slot(j, kLog);
@@ -1069,9 +1041,9 @@ __global__ __launch_bounds__(WPB * kWave, T <= 256 ? 8 : 1) void k_num_light(con
 }
 
 // ---------------------------------------------------------------- numeric, light rows by sorting
-// Rows of 129 to 1024 multiplications that did not come from the heavy
-// symbolic: all products of a row at once, four per thread (NT = 64, 128 or 256
-// threads a row).  The products are flattened in A-order, sorted in registers by
+// Rows of up to 1024 multiplications that did not come from the heavy symbolic:
+// all products of a row at once, P per thread (one wave a row with P = 1, 2 or 4
+// products, or 128 or 256 threads with 4).  The products are flattened in A-order, sorted in registers by
 // (column, position), and every column's run is summed in position (= A) order
 // by the thread that holds its first product; the runs in order are the sorted
 // output.
@@ -1083,7 +1055,6 @@ __global__ __launch_bounds__(WPB * kWave, T <= 256 ? 8 : 1) void k_num_light(con
 // per CU), walked A's entries one after the other and sorted the table in LDS:
 // stage of R-MAT s18 2671 us for the three classes, now 481 us (22 KiB for a row
 // of 256 threads: 28 waves per CU); tile accumulate of R-MAT s16 154 -> 33 us.
-constexpr int kSortPer = 4;        // products per thread
 constexpr int kSortIdBits = 10;    // product positions < 1024
 
 template <typename K>
@@ -1093,11 +1064,10 @@ __device__ __forceinline__ void order_pair(K &a, K &b, bool up) {
     b = up ? hi : lo;
 }
 
-// One step of the bitonic sort of NT * kSortPer keys, key u of thread t at
-// position t * kSortPer + u, then the smaller strides of the same size.
-template <int NT, int kSize, int kStride, typename K>
-__device__ __forceinline__ void sort_step(K (&key)[kSortPer], K *lds, int t) {
-    constexpr int P = kSortPer;
+// One step of the bitonic sort of NT * P keys, key u of thread t at position
+// t * P + u, then the smaller strides of the same size.
+template <int NT, int kSize, int kStride, int P, typename K>
+__device__ __forceinline__ void sort_step(K (&key)[P], K *lds, int t) {
     if constexpr (kStride < P) {
 #pragma unroll
         for (int u = 0; u < P; ++u)
@@ -1126,13 +1096,13 @@ __device__ __forceinline__ void sort_step(K (&key)[kSortPer], K *lds, int t) {
             __syncthreads();
         }
     }
-    if constexpr (kStride > 1) sort_step<NT, kSize, kStride / 2>(key, lds, t);
+    if constexpr (kStride > 1) sort_step<NT, kSize, kStride / 2, P>(key, lds, t);
 }
 
-template <int NT, int kSize = 2, typename K>
-__device__ __forceinline__ void sort_products(K (&key)[kSortPer], K *lds, int t) {
-    sort_step<NT, kSize, kSize / 2>(key, lds, t);
-    if constexpr (kSize < NT * kSortPer) sort_products<NT, kSize * 2>(key, lds, t);
+template <int NT, int P, int kSize = 2, typename K>
+__device__ __forceinline__ void sort_products(K (&key)[P], K *lds, int t) {
+    sort_step<NT, kSize, kSize / 2, P>(key, lds, t);
+    if constexpr (kSize < NT * P) sort_products<NT, P, kSize * 2>(key, lds, t);
 }
 
 // barrier of a row's threads
@@ -1142,33 +1112,33 @@ __device__ __forceinline__ void row_sync() {
     else wave_sync();
 }
 
-template <int NT, typename K>
+template <int NT, int P, typename K>
 struct SortLds {
-    static constexpr int kMax = NT * kSortPer;
+    static constexpr int kMax = NT * P;
     double pa[kMax];  // by a B row's first position: its A value; then by position: the product's
     double pb[kMax];
     union {
         int32_t sq[kMax];  // by a B row's first position: B position minus product position
         K key[kMax];       // sorted keys
     };
-    uint16_t mark[kMax];  // a B row's first position + 1, else 0
+    __align__(8) uint16_t mark[kMax];  // a B row's first position + 1, else 0
     int32_t part[2][NT / kWave];
 };
 
-template <int NT, int WPB, typename K>
+template <int NT, int WPB, int P, typename K>
 __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict__ tasks, int nt,
                                                       const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
                                                       int cls, const int64_t *__restrict__ rowptr,
                                                       const Panel *__restrict__ panels, int npanels) {
     static_assert(NT > kWave ? WPB == 1 : NT == kWave, "a row's threads are a workgroup or a wave of it");
-    constexpr int P = kSortPer, kMax = NT * P, kWaves = NT / kWave;
+    constexpr int kMax = NT * P, kWaves = NT / kWave;
     static_assert(kMax <= 1 << kSortIdBits, "positions fit their key bits");
     constexpr K kIdMask = ((K)1 << kSortIdBits) - 1;
-    __shared__ SortLds<NT, K> lds_s[WPB];
+    __shared__ SortLds<NT, P, K> lds_s[WPB];
     const int sub = NT > kWave ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // row of the workgroup
     const int t = threadIdx.x % NT, l = lane_id();
     const int w = NT > kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;    // wave of the row
-    SortLds<NT, K> &L = lds_s[sub];
+    SortLds<NT, P, K> &L = lds_s[sub];
     const int32_t nrows = cnt->cls[cls];
     for (int32_t li = blockIdx.x * WPB + sub; li < nrows; li += gridDim.x * WPB) {
         const int32_t g = __builtin_amdgcn_readfirstlane(rows[li]);
@@ -1180,7 +1150,8 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
         const TR_GLOBAL int32_t *__restrict__ bi = as_global(TK.bi);
         const TR_GLOBAL double *__restrict__ bv = as_global(TK.bv);
         const int32_t a0 = as_global(TK.ap)[r], a1 = as_global(TK.ap)[r + 1];
-        *reinterpret_cast<uint2 *>(&L.mark[t * P]) = make_uint2(0u, 0u);
+#pragma unroll
+        for (int u = 0; u < P; ++u) L.mark[t * P + u] = 0;
         row_sync<NT>();
         // B rows of A's entries, flattened: each non-empty one is entered at its
         // first product position
@@ -1219,12 +1190,12 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
         // this thread's products t P .. t P + P - 1: the last mark at or below
         uint32_t m[P];
         {
-            const uint2 q = *reinterpret_cast<const uint2 *>(&L.mark[t * P]);
-            m[0] = q.x & 0xffffu;
-            m[1] = max(m[0], q.x >> 16);
-            m[2] = max(m[1], q.y & 0xffffu);
-            m[3] = max(m[2], q.y >> 16);
-            const uint32_t inc = wave_incl_max(m[3]);
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                m[u] = L.mark[t * P + u];
+                if (u) m[u] = max(m[u], m[u - 1]);
+            }
+            const uint32_t inc = wave_incl_max(m[P - 1]);
             uint32_t before = dpp<0x138>(inc);  // the lane below; 0 for lane 0
             if constexpr (kWaves > 1) {
                 // (the entries' last use of `part` is behind the barrier above)
@@ -1257,7 +1228,7 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
             L.pa[t * P + u] = pa[u];
             L.pb[t * P + u] = pbv[u];
         }
-        sort_products<NT>(key, L.key, t);
+        sort_products<NT, P>(key, L.key, t);
 #pragma unroll
         for (int u = 0; u < P; ++u) L.key[t * P + u] = key[u];
         row_sync<NT>();
@@ -1950,9 +1921,9 @@ void launch_sym_light(tr_ctx *ctx, MulPlan &pl, int c) {
 
 template <int T>
 void launch_num_light(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
-    constexpr int kWpb = T >= 1024 ? 1 : 4;
+    constexpr int kWpb = 4;
     const int32_t n = pl.h.cls[c];
-    TR_LAUNCH(ctx, "num_light", (k_num_light<T, kWpb>), cap_grid(div_up((uint64_t)n, kWpb), 1 << 20), kWpb * kWave,
+    if (n) TR_LAUNCH(ctx, "num_light", (k_num_light<T, kWpb>), cap_grid(div_up((uint64_t)n, kWpb), 1 << 20), kWpb * kWave,
               0, pl.d_tasks, pl.nt, pl.lists + (int64_t)c * pl.rows_total, pl.cnt, c, pl.rowptr, panels, np);
 }
 
@@ -2050,7 +2021,7 @@ void mul_analyze(tr_ctx *ctx, MulPlan &pl) {
     }
     launch_check(ctx, pl.jobs, pl.njobs, pl.pair, pl.check_grid);
     TR_LAUNCH(ctx, "classify", k_classify, div_up((uint64_t)pl.rows_total, kRowsPerBlock), kClassThreads, 0,
-              pl.d_tasks, pl.nt, pl.rows_total, pl.flops, pl.rownnz, pl.lists, pl.cnt, pl.tune.light_max_flops);
+              pl.rows_total, pl.flops, pl.rownnz, pl.lists, pl.cnt, pl.tune.light_max_flops);
 }
 
 namespace {
@@ -2206,32 +2177,37 @@ void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np) {
 
 namespace {
 
-template <int NT, typename K>
+template <int NT, int P, typename K>
 void launch_num_sort_as(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
     constexpr int kWpb = NT > kWave ? 1 : 4;
     const int32_t n = pl.h.cls[c];
-    TR_LAUNCH(ctx, "num_light", (k_num_sort<NT, kWpb, K>), cap_grid(div_up((uint64_t)n, kWpb), 1 << 20), NT * kWpb, 0,
-              pl.d_tasks, pl.nt, pl.lists + (int64_t)c * pl.rows_total, pl.cnt, c, pl.rowptr, panels, np);
+    TR_LAUNCH(ctx, "num_light", (k_num_sort<NT, kWpb, P, K>), cap_grid(div_up((uint64_t)n, kWpb), 1 << 20), NT * kWpb,
+              0, pl.d_tasks, pl.nt, pl.lists + (int64_t)c * pl.rows_total, pl.cnt, c, pl.rowptr, panels, np);
 }
 
-// (column, position) keys of 32 bits where every column fits
-template <int NT>
+// class c of rows of up to NT * P products; (column, position) keys of 32 bits
+// where every column fits
+template <int NT, int P>
 void launch_num_sort(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
+    if (!pl.h.cls[c]) return;
     int32_t max_n = 0;
     for (const TaskDev &t : pl.h_tasks) max_n = std::max(max_n, t.n);
-    if (max_n <= 1 << (32 - kSortIdBits)) launch_num_sort_as<NT, uint32_t>(ctx, pl, c, panels, np);
-    else launch_num_sort_as<NT, uint64_t>(ctx, pl, c, panels, np);
+    if (max_n <= 1 << (32 - kSortIdBits)) launch_num_sort_as<NT, P, uint32_t>(ctx, pl, c, panels, np);
+    else launch_num_sort_as<NT, P, uint64_t>(ctx, pl, c, panels, np);
 }
 
 }  // namespace
 
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *dp, int np) {
-    if (pl.h.cls[0]) launch_num_light<64>(ctx, pl, 0, dp, np);
-    if (pl.h.cls[1]) launch_num_light<128>(ctx, pl, 1, dp, np);
-    if (pl.h.cls[2]) launch_num_light<256>(ctx, pl, 2, dp, np);
-    if (pl.h.cls[3]) launch_num_sort<64>(ctx, pl, 3, dp, np);
-    if (pl.h.cls[4]) launch_num_sort<128>(ctx, pl, 4, dp, np);
-    if (pl.h.cls[5]) launch_num_sort<256>(ctx, pl, 5, dp, np);
+    launch_num_sort<64, 1>(ctx, pl, 0, dp, np);
+    launch_num_sort<64, 1>(ctx, pl, 1, dp, np);
+    launch_num_sort<64, 2>(ctx, pl, 2, dp, np);
+    launch_num_sort<64, 4>(ctx, pl, 3, dp, np);
+    launch_num_sort<128, 4>(ctx, pl, 4, dp, np);
+    launch_num_sort<256, 4>(ctx, pl, 5, dp, np);
+    launch_num_light<64>(ctx, pl, kCompactClass, dp, np);
+    launch_num_light<128>(ctx, pl, kCompactClass + 1, dp, np);
+    launch_num_light<256>(ctx, pl, kCompactClass + 2, dp, np);
     if (pl.h.items > 0) {
         // one workgroup per item, grid-stride beyond 2^22 workgroups (the
         // dispatch packet counts work-items in 32 bits)

@@ -12,11 +12,11 @@ namespace tr {
 
 // tuning constants
 constexpr int kLightMaxFCap = 1024; // largest light/heavy cut (light tables reach 2048 slots)
-constexpr int kNumLight = 6;       // light classes: T = 64 << c, c < kNumLight
-constexpr int kHashClassMax = 2;   // light rows up to this class are hashed by the numeric, the others sorted
+constexpr int kNumLight = 6;       // light classes: up to 32 << c multiplications, c < kNumLight
 constexpr int kHeavyClass = kNumLight;      // heavy rows with more than kMidMaxF multiplications
 constexpr int kMidClass = kNumLight + 1;    // heavy rows up to kMidMaxF multiplications
-constexpr int kNumClasses = kNumLight + 2;
+constexpr int kCompactClass = kNumLight + 2;  // + 0..2: heavy rows of <= 32, 64, 128 entries (found by the symbolic)
+constexpr int kNumClasses = kNumLight + 5;
 constexpr int kMidMaxF = 16384;
 constexpr int kMidPassBits = 19;            // mid rows: at most 2^19-column passes, two blocks per CU
 constexpr int kMidThreads = 512;
