@@ -65,3 +65,29 @@ def test_many_entries_few_products(ctx):
     rows_b = [np.sort(rng.choice(5000, 2, replace=False)) if k % 13 == 0 else [] for k in range(nb)]
     rows_a = [np.sort(rng.choice(nb, m, replace=False)) for m in (900, 1700, 3000, 6000 // 2, 5999)] + [[0], []]
     _check(ctx, _csr(rows_a, nb, rng), _csr(rows_b, 5000, rng))
+
+
+@pytest.mark.parametrize("nrows", [32767, 32768, 32775, 33001])
+@pytest.mark.parametrize("span", [6, 32, 33, 64, 5000])
+def test_short_rows(ctx, nrows, span):
+    """Eight rows to a wave, in products of 32768 rows and more: many A entries
+    over B rows of 2 to 10 entries on average (some empty, some over eight), at
+    most 128 products, over about `span` columns (sorted beyond 32 entries),
+    rows of other classes between them."""
+    rng = np.random.default_rng(nrows * 100 + span)
+    nb = 400
+    lens = rng.choice([0, 1, 2, 4, 5, 7, 8, 9, 16, 17], nb)
+    rows_b = [np.sort(rng.choice(span, min(m, span), replace=False)) * 7 for m in lens]
+    rows_a = []
+    for r in range(600):
+        row, f = [], 0
+        target = int(rng.choice([8, 40, 100, 127, 128, 128, 200]))
+        for k in rng.permutation(nb):
+            if f + len(rows_b[k]) <= target:
+                row.append(k)
+                f += len(rows_b[k])
+            if len(row) >= 60 or f == target:
+                break
+        rows_a.append(np.sort(row))
+    pick = rng.integers(0, 600, nrows)
+    _check(ctx, _csr([rows_a[i] for i in pick], nb, rng), _csr(rows_b, 7 * span + 1, rng))

@@ -316,10 +316,20 @@ __device__ __forceinline__ int light_class(int64_t n) {
     return c;
 }
 
-__global__ __launch_bounds__(kClassThreads) void k_classify(int32_t rows_total, const int64_t *__restrict__ flops,
+// Rows of up to 128 multiplications over many B rows of 2 to 10 entries (at
+// least twice as many as entries in one; a Laplacian times a prolongator: 27 of
+// 4.5): eight to a wave (k_num_short).  Few B rows meet in few columns, which
+// suits the sorted classes (ER n = 200000, 8 of 8: 302 against 394 us), longer
+// B rows would leave eight lanes several turns, emptier ones turns of nothing.
+__device__ __forceinline__ bool is_short(int64_t f, int32_t len) {
+    return f <= kShortMaxF && f >= 2 * (int64_t)len && f <= 10 * (int64_t)len && 2 * f <= (int64_t)len * len;
+}
+
+__global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__restrict__ tasks, int nt,
+                                                            int32_t rows_total, const int64_t *__restrict__ flops,
                                                             int64_t *__restrict__ rownnz,
                                                             int32_t *__restrict__ lists, Counters *__restrict__ cnt,
-                                                            int32_t light_max) {
+                                                            int32_t light_max, int allow_short) {
     constexpr int kPer = kRowsPerBlock / kClassThreads;
     __shared__ int32_t s_cnt[kNumClasses], s_base[kNumClasses];
     __shared__ unsigned long long s_f, s_hf;
@@ -329,11 +339,16 @@ __global__ __launch_bounds__(kClassThreads) void k_classify(int32_t rows_total, 
     if (tid == 0) s_f = s_hf = 0ull;
     __syncthreads();
     int64_t f[kPer], sf = 0, shf = 0;
+    int32_t len[kPer];  // A entries
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
         const int32_t g = g0 + u * kClassThreads;
         f[u] = 0;
+        len[u] = 0;
         if (g < rows_total) {
+            const TaskDev &T = tasks[task_of(tasks, nt, g)];
+            const int32_t *p = T.ap + (g - T.row_base);
+            len[u] = p[1] - p[0];
             f[u] = flops[g];
             rownnz[g] = 0;
         }
@@ -345,7 +360,7 @@ __global__ __launch_bounds__(kClassThreads) void k_classify(int32_t rows_total, 
         lpos[u] = 0;
         if (f[u] > 0) {
             if (f[u] <= light_max) {
-                c[u] = light_class(f[u]);
+                c[u] = allow_short && is_short(f[u], len[u]) ? kShortClass : light_class(f[u]);
             } else {
                 c[u] = f[u] <= kMidMaxF ? kMidClass : kHeavyClass;
                 shf += f[u];
@@ -444,6 +459,231 @@ __global__ __launch_bounds__(256) void k_sym_light(const TaskDev *__restrict__ t
         }
         cntv = wave_sum(cntv);
         if (l == 0) rownnz[g] = cntv;
+        wave_sync();
+    }
+}
+
+// ---------------------------------------------------------------- short rows
+// Eight rows to a wave, eight lanes to a row: a row's A entries are taken in
+// order, the lanes over one short B row at a time, into the row's own LDS table.
+//
+// What bounds it: vector instructions, about 35 per A entry for eight rows
+// together.  With a wave per row and its products flattened over 64 lanes, the
+// products that meet in a column (27 B rows over 17 columns) had to be put back
+// in order afterwards: A*P of Galerkin 96^3 (885 k rows, 105 M products)
+// 434 and 1150 us (symbolic, numeric), now 228 and 732 us.
+constexpr int kShortLanes = 8;
+constexpr int kShortRows = kWave / kShortLanes;  // rows per wave
+
+// value of lane kLane of the calling lane's group of eight
+template <int kLane>
+__device__ __forceinline__ int32_t group_lane(int32_t v) {
+    return __builtin_amdgcn_ds_swizzle(v, 0x18 | kLane << 5);
+}
+template <int kLane>
+__device__ __forceinline__ double group_lane(double v) {
+    return by_words(v, [](uint32_t u) { return (uint32_t)__builtin_amdgcn_ds_swizzle((int)u, 0x18 | kLane << 5); });
+}
+
+// A entries [pb, pb + 8) of a short row, one per lane of its group
+struct ShortChunk {
+    int32_t bs, len;
+    double a;
+};
+
+// The first kShortLanes entries of the chunk's B rows, loaded together
+template <bool kVals>
+struct ShortB {
+    int32_t s[kShortLanes], n[kShortLanes], j[kShortLanes];
+    double b[kVals ? kShortLanes : 1];
+};
+
+template <bool kVals, int kLane = 0>
+__device__ __forceinline__ void short_load(const ShortChunk &c, const TR_GLOBAL int32_t *__restrict__ bi,
+                                           const TR_GLOBAL double *__restrict__ bv, int q, ShortB<kVals> &x) {
+    x.s[kLane] = group_lane<kLane>(c.bs);
+    x.n[kLane] = group_lane<kLane>(c.len);
+    x.j[kLane] = 0;
+    if (q < x.n[kLane]) {
+        x.j[kLane] = bi[x.s[kLane] + q];
+        if constexpr (kVals) x.b[kLane] = bv[x.s[kLane] + q];
+    }
+    if constexpr (kLane + 1 < kShortLanes) short_load<kVals, kLane + 1>(c, bi, bv, q, x);
+}
+
+// f(column, A value, B value) for every product of the chunk, B row after B
+// row (the lanes of a group hold distinct columns of one B row)
+template <bool kVals, int kLane = 0, typename F>
+__device__ __forceinline__ void short_apply(const ShortChunk &c, const TR_GLOBAL int32_t *__restrict__ bi,
+                                            const TR_GLOBAL double *__restrict__ bv, int q, const ShortB<kVals> &x,
+                                            F &f) {
+    double a = 0.0;
+    if constexpr (kVals) a = group_lane<kLane>(c.a);
+    if (q < x.n[kLane]) f(x.j[kLane], a, kVals ? x.b[kVals ? kLane : 0] : 0.0);
+    for (int32_t o = q + kShortLanes; ballot(o < x.n[kLane]); o += kShortLanes)
+        if (o < x.n[kLane]) f(bi[x.s[kLane] + o], a, kVals ? bv[x.s[kLane] + o] : 0.0);
+    wave_sync();  // the next B row sees this one's entries
+    if constexpr (kLane + 1 < kShortLanes) short_apply<kVals, kLane + 1>(c, bi, bv, q, x, f);
+}
+
+// all products of the row [a0, a1) of each group
+template <bool kVals, typename F>
+__device__ __forceinline__ void short_products(const TaskDev &TK, int32_t a0, int32_t a1, int q, F &&f) {
+    const TR_GLOBAL int32_t *__restrict__ ai = as_global(TK.ai);
+    const TR_GLOBAL double *__restrict__ av = as_global(TK.av);
+    const TR_GLOBAL int32_t *__restrict__ bp = as_global(TK.bp);
+    const TR_GLOBAL int32_t *__restrict__ bi = as_global(TK.bi);
+    const TR_GLOBAL double *__restrict__ bv = as_global(TK.bv);
+    for (int32_t pb = a0; ballot(pb < a1); pb += kShortLanes) {
+        ShortChunk c{0, 0, 0.0};
+        if (pb + q < a1) {
+            const int32_t k = ai[pb + q];
+            if constexpr (kVals) c.a = av[pb + q];
+            c.bs = bp[k];
+            c.len = bp[k + 1] - c.bs;
+        }
+        ShortB<kVals> x;
+        short_load<kVals>(c, bi, bv, q, x);
+        short_apply<kVals>(c, bi, bv, q, x, f);
+    }
+}
+
+// slot of column j in the table (claimed, if it is new; then fresh), or -1
+template <int T>
+__device__ __forceinline__ int table_slot(int32_t *keys, int32_t j, bool &fresh) {
+    uint32_t h = hash_slot(j, __builtin_ctz(T));
+    for (int probe = 0; probe < T; ++probe) {
+        const int32_t old = atomicCAS(&keys[h], kEmpty, j);
+        if (old == kEmpty || old == j) {
+            fresh = old == kEmpty;
+            return (int)h;
+        }
+        h = (h + 1) & (T - 1);
+    }
+    return -1;
+}
+
+// Entries per row of the short class.  Rows of more entries than k_num_short's
+// table takes are counted too, so that the numeric launches only what it needs.
+__global__ __launch_bounds__(256) void k_sym_short(const TaskDev *__restrict__ tasks, int nt,
+                                                   const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
+                                                   int64_t *__restrict__ rownnz) {
+    constexpr int T = kShortMaxF;  // at most that many columns
+    __shared__ __align__(16) int32_t keys_s[4][kShortRows][T];
+    __shared__ int32_t sizes[2];
+    const int w = threadIdx.x / kWave, l = lane_id(), grp = l / kShortLanes, q = l % kShortLanes;
+    int32_t *keys = keys_s[w][grp];
+    if (threadIdx.x < 2) sizes[threadIdx.x] = 0;
+    __syncthreads();
+    const int32_t nrows = cnt->cls[kShortClass];
+    for (int32_t base = (blockIdx.x * 4 + w) * kShortRows; base < nrows; base += gridDim.x * 4 * kShortRows) {
+        const bool valid = base + grp < nrows;
+        const int32_t g = rows[valid ? base + grp : base];
+        const TaskDev &TK = tasks[task_of(tasks, nt, g)];
+        const int32_t r = g - TK.row_base;
+        const int32_t a0 = as_global(TK.ap)[r], a1 = valid ? as_global(TK.ap)[r + 1] : a0;
+        for (int t = q * 4; t < T; t += kShortLanes * 4)
+            *reinterpret_cast<int4 *>(&keys[t]) = make_int4(kEmpty, kEmpty, kEmpty, kEmpty);
+        wave_sync();
+        int32_t n = 0;
+        short_products<false>(TK, a0, a1, q, [&](int32_t j, double, double) {
+            bool fresh = false;
+            (void)table_slot<T>(keys, j, fresh);
+            n += fresh ? 1 : 0;
+        });
+        n += lane_xor<1>(n);
+        n += lane_xor<2>(n);
+        n += lane_xor<4>(n);
+        if (valid && q == 0) {
+            rownnz[g] = n;
+            atomicAdd(&sizes[n <= kShortMaxNnz ? 0 : 1], 1);
+        }
+        wave_sync();
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 && sizes[threadIdx.x]) atomicAdd(&cnt->short_rows[threadIdx.x], sizes[threadIdx.x]);
+}
+
+// Values of the short rows of at most kShortMaxNnz entries.
+__global__ __launch_bounds__(256, 6) void k_num_short(const TaskDev *__restrict__ tasks, int nt,
+                                                      const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
+                                                      const int64_t *__restrict__ rowptr,
+                                                      const Panel *__restrict__ panels, int npanels) {
+    constexpr int T = 2 * kShortMaxNnz;
+    constexpr int kSlots = T / kShortLanes;  // table slots per lane
+    constexpr int kOut = kSlots / 2;         // entries per lane
+    __shared__ __align__(16) int32_t keys_s[4][kShortRows][T];
+    __shared__ double vals_s[4][kShortRows][T];
+    __shared__ uint16_t slot_s[4][kShortRows][T / 2];
+    const int w = threadIdx.x / kWave, l = lane_id(), grp = l / kShortLanes, q = l % kShortLanes;
+    int32_t *keys = keys_s[w][grp];
+    double *vals = vals_s[w][grp];
+    uint16_t *slots = slot_s[w][grp];
+    const int32_t nrows = cnt->cls[kShortClass];
+    for (int32_t base = (blockIdx.x * 4 + w) * kShortRows; base < nrows; base += gridDim.x * 4 * kShortRows) {
+        const int32_t g = rows[base + grp < nrows ? base + grp : base];
+        const int64_t rs = rowptr[g];
+        const int32_t expect = (int32_t)(rowptr[g + 1] - rs);
+        const bool valid = base + grp < nrows && expect <= T / 2;
+        if (!ballot(valid)) continue;
+        const TaskDev &TK = tasks[task_of(tasks, nt, g)];
+        const int32_t r = g - TK.row_base;
+        const int32_t a0 = as_global(TK.ap)[r], a1 = valid ? as_global(TK.ap)[r + 1] : a0;
+        for (int t = q * 4; t < T; t += kShortLanes * 4)
+            *reinterpret_cast<int4 *>(&keys[t]) = make_int4(kEmpty, kEmpty, kEmpty, kEmpty);
+        wave_sync();
+        short_products<true>(TK, a0, a1, q, [&](int32_t j, double a, double b) {
+            bool fresh = false;
+            const int h = table_slot<T>(keys, j, fresh);
+            if (h >= 0) vals[h] = __fma_rn(a, b, fresh ? 0.0 : vals[h]);
+        });
+        // occupied slots to the front (keys, and the slots their values are in)
+        int32_t k[kSlots];
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u) k[u] = keys[u * kShortLanes + q];
+        wave_sync();
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u) {
+            const uint32_t m = (uint32_t)(ballot(k[u] != kEmpty) >> (grp * kShortLanes)) & 0xffu;
+            const int at = n + __popc(m & ((1u << q) - 1u));
+            if (k[u] != kEmpty && at < T / 2) {
+                keys[at] = k[u];
+                slots[at] = (uint16_t)(u * kShortLanes + q);
+            }
+            n += __popc(m);
+        }
+        if (valid && q == 0 && n != expect) atomicOr(&cnt->overflow, 2);
+        n = min(n, T / 2);
+        wave_sync();
+        // each lane's entries, ranked by the smaller columns of their row
+        int32_t c[kOut], rank[kOut];
+        double v[kOut];
+#pragma unroll
+        for (int i = 0; i < kOut; ++i) {
+            const int e = q + i * kShortLanes;
+            c[i] = INT32_MAX;
+            v[i] = 0.0;
+            rank[i] = 0;
+            if (valid && e < n) {
+                c[i] = keys[e];
+                v[i] = vals[slots[e]];
+            }
+        }
+        for (int x = 0; ballot(valid && x < n); ++x) {
+            const int32_t o = x < n ? keys[x] : INT32_MAX;
+#pragma unroll
+            for (int i = 0; i < kOut; ++i) rank[i] += o < c[i] ? 1 : 0;
+        }
+        const Panel &PN = find_panel(panels, npanels, g);
+        TR_GLOBAL int32_t *oi = as_global(PN.idx) + (rs - PN.nnz_begin);
+        TR_GLOBAL double *ov = as_global(PN.val) + (rs - PN.nnz_begin);
+#pragma unroll
+        for (int i = 0; i < kOut; ++i)
+            if (valid && q + i * kShortLanes < n && rank[i] < expect) {
+                oi[rank[i]] = c[i];
+                ov[rank[i]] = v[i];
+            }
         wave_sync();
     }
 }
@@ -1128,7 +1368,7 @@ struct SortLds {
 template <int NT, int WPB, int P, typename K>
 __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict__ tasks, int nt,
                                                       const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
-                                                      int cls, const int64_t *__restrict__ rowptr,
+                                                      int cls, int32_t lo, const int64_t *__restrict__ rowptr,
                                                       const Panel *__restrict__ panels, int npanels) {
     static_assert(NT > kWave ? WPB == 1 : NT == kWave, "a row's threads are a workgroup or a wave of it");
     constexpr int kMax = NT * P, kWaves = NT / kWave;
@@ -1142,6 +1382,9 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
     const int32_t nrows = cnt->cls[cls];
     for (int32_t li = blockIdx.x * WPB + sub; li < nrows; li += gridDim.x * WPB) {
         const int32_t g = __builtin_amdgcn_readfirstlane(rows[li]);
+        const int64_t rs = rowptr[g];
+        const int32_t expect = (int32_t)(rowptr[g + 1] - rs);
+        if (expect <= lo) continue;  // uniform over the row's threads: not this launch's (short rows)
         const TaskDev &TK = tasks[task_of(tasks, nt, g)];
         const int32_t r = g - TK.row_base;
         const TR_GLOBAL int32_t *__restrict__ ai = as_global(TK.ai);
@@ -1258,8 +1501,6 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
         } else {
             n = read_lane(inc, kWave - 1);
         }
-        const int64_t rs = rowptr[g];
-        const int32_t expect = (int32_t)(rowptr[g + 1] - rs);
         const Panel &PN = find_panel(panels, npanels, g);
         if (t == 0 && n != expect) atomicOr(&cnt->overflow, 2);
         TR_GLOBAL int32_t *oi = as_global(PN.idx) + (rs - PN.nnz_begin);
@@ -2021,7 +2262,8 @@ void mul_analyze(tr_ctx *ctx, MulPlan &pl) {
     }
     launch_check(ctx, pl.jobs, pl.njobs, pl.pair, pl.check_grid);
     TR_LAUNCH(ctx, "classify", k_classify, div_up((uint64_t)pl.rows_total, kRowsPerBlock), kClassThreads, 0,
-              pl.rows_total, pl.flops, pl.rownnz, pl.lists, pl.cnt, pl.tune.light_max_flops);
+              pl.d_tasks, pl.nt, pl.rows_total, pl.flops, pl.rownnz, pl.lists, pl.cnt, pl.tune.light_max_flops,
+              pl.rows_total >= kShortMinRows ? 1 : 0);
 }
 
 namespace {
@@ -2072,6 +2314,10 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
     if (pl.h.cls[3]) launch_sym_light<512>(ctx, pl, 3);
     if (pl.h.cls[4]) launch_sym_light<1024>(ctx, pl, 4);
     if (pl.h.cls[5]) launch_sym_light<2048>(ctx, pl, 5);
+    if (pl.h.cls[kShortClass])
+        TR_LAUNCH(ctx, "sym_light", k_sym_short,
+                  cap_grid(div_up((uint64_t)pl.h.cls[kShortClass], 4 * kShortRows), (int64_t)ctx->cu_count * 32), 256, 0,
+                  pl.d_tasks, pl.nt, pl.lists + (int64_t)kShortClass * pl.rows_total, pl.cnt, pl.rownnz);
     const int32_t nh = pl.h.cls[kHeavyClass] + pl.h.cls[kMidClass];
     if (nh) {
         int32_t max_n = 0;
@@ -2178,33 +2424,40 @@ void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np) {
 namespace {
 
 template <int NT, int P, typename K>
-void launch_num_sort_as(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
+void launch_num_sort_as(tr_ctx *ctx, MulPlan &pl, int c, int32_t lo, Panel *panels, int np) {
     constexpr int kWpb = NT > kWave ? 1 : 4;
     const int32_t n = pl.h.cls[c];
     TR_LAUNCH(ctx, "num_light", (k_num_sort<NT, kWpb, P, K>), cap_grid(div_up((uint64_t)n, kWpb), 1 << 20), NT * kWpb,
-              0, pl.d_tasks, pl.nt, pl.lists + (int64_t)c * pl.rows_total, pl.cnt, c, pl.rowptr, panels, np);
+              0, pl.d_tasks, pl.nt, pl.lists + (int64_t)c * pl.rows_total, pl.cnt, c, lo, pl.rowptr,
+              panels, np);
 }
 
-// class c of rows of up to NT * P products; (column, position) keys of 32 bits
+// class c of rows of up to NT * P products, those of more than lo entries; (column, position) keys of 32 bits
 // where every column fits
 template <int NT, int P>
-void launch_num_sort(tr_ctx *ctx, MulPlan &pl, int c, Panel *panels, int np) {
+void launch_num_sort(tr_ctx *ctx, MulPlan &pl, int c, int32_t lo, Panel *panels, int np) {
     if (!pl.h.cls[c]) return;
     int32_t max_n = 0;
     for (const TaskDev &t : pl.h_tasks) max_n = std::max(max_n, t.n);
-    if (max_n <= 1 << (32 - kSortIdBits)) launch_num_sort_as<NT, P, uint32_t>(ctx, pl, c, panels, np);
-    else launch_num_sort_as<NT, P, uint64_t>(ctx, pl, c, panels, np);
+    if (max_n <= 1 << (32 - kSortIdBits)) launch_num_sort_as<NT, P, uint32_t>(ctx, pl, c, lo, panels, np);
+    else launch_num_sort_as<NT, P, uint64_t>(ctx, pl, c, lo, panels, np);
 }
 
 }  // namespace
 
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *dp, int np) {
-    launch_num_sort<64, 1>(ctx, pl, 0, dp, np);
-    launch_num_sort<64, 1>(ctx, pl, 1, dp, np);
-    launch_num_sort<64, 2>(ctx, pl, 2, dp, np);
-    launch_num_sort<64, 4>(ctx, pl, 3, dp, np);
-    launch_num_sort<128, 4>(ctx, pl, 4, dp, np);
-    launch_num_sort<256, 4>(ctx, pl, 5, dp, np);
+    launch_num_sort<64, 1>(ctx, pl, 0, 0, dp, np);
+    launch_num_sort<64, 1>(ctx, pl, 1, 0, dp, np);
+    launch_num_sort<64, 2>(ctx, pl, 2, 0, dp, np);
+    launch_num_sort<64, 4>(ctx, pl, 3, 0, dp, np);
+    launch_num_sort<128, 4>(ctx, pl, 4, 0, dp, np);
+    launch_num_sort<256, 4>(ctx, pl, 5, 0, dp, np);
+    // short rows of more entries than their table takes are sorted
+    if (pl.h.short_rows[0])
+        TR_LAUNCH(ctx, "num_light", k_num_short,
+                  cap_grid(div_up((uint64_t)pl.h.cls[kShortClass], 4 * kShortRows), 1 << 20), 256, 0, pl.d_tasks, pl.nt,
+                  pl.lists + (int64_t)kShortClass * pl.rows_total, pl.cnt, pl.rowptr, dp, np);
+    if (pl.h.short_rows[1]) launch_num_sort<64, 2>(ctx, pl, kShortClass, kShortMaxNnz, dp, np);
     launch_num_light<64>(ctx, pl, kCompactClass, dp, np);
     launch_num_light<128>(ctx, pl, kCompactClass + 1, dp, np);
     launch_num_light<256>(ctx, pl, kCompactClass + 2, dp, np);

@@ -16,7 +16,14 @@ constexpr int kNumLight = 6;       // light classes: up to 32 << c multiplicatio
 constexpr int kHeavyClass = kNumLight;      // heavy rows with more than kMidMaxF multiplications
 constexpr int kMidClass = kNumLight + 1;    // heavy rows up to kMidMaxF multiplications
 constexpr int kCompactClass = kNumLight + 2;  // + 0..2: heavy rows of <= 32, 64, 128 entries (found by the symbolic)
-constexpr int kNumClasses = kNumLight + 5;
+constexpr int kShortClass = kNumLight + 5;    // light rows of short B rows
+constexpr int kNumClasses = kNumLight + 6;
+constexpr int kShortMaxF = 128;               // multiplications of a short row
+constexpr int kShortMaxNnz = 32;              // and its entries, for the table of the numeric
+// rows of a product that looks for short ones: eight to a wave, fewer leave the
+// chip idle (Galerkin n^3, short against sorted: 28 392 / 388 us, 32 385 / 394,
+// 48 509 / 568, 64 874 / 1031)
+constexpr int32_t kShortMinRows = 32768;
 constexpr int kMidMaxF = 16384;
 constexpr int kMidPassBits = 19;            // mid rows: at most 2^19-column passes, two blocks per CU
 constexpr int kMidThreads = 512;
@@ -73,6 +80,7 @@ struct TaskDev {
 // device counters written by the symbolic phase
 struct Counters {
     int32_t cls[kNumClasses];        // rows per class
+    int32_t short_rows[2];           // rows of the short class with <= kShortMaxNnz and with more entries
     unsigned long long flops;        // total multiplications
     unsigned long long heavy_flops;  // multiplications of heavy rows
     int32_t windows;                 // windows appended
