@@ -140,6 +140,13 @@ void *scratch(tr_ctx *ctx, int slot, size_t bytes) {
     return ctx->scratch_ptr[slot];
 }
 
+void scratch_drop(tr_ctx *ctx, int slot) {
+    if (slot >= (int)ctx->scratch_ptr.size() || !ctx->scratch_ptr[slot]) return;
+    ctx->pool.release(ctx->scratch_ptr[slot]);
+    ctx->scratch_ptr[slot] = nullptr;
+    ctx->scratch_size[slot] = 0;
+}
+
 namespace {
 
 struct Publish {
@@ -459,17 +466,12 @@ int tr_sp_mma(tr_ctx_t ctx, const tr_csx_t *A, const tr_csx_t *B, tr_csx_t *C) {
     });
 }
 
-// Both operands of a sorted add: CSR, same shape, well formed, sorted rows.
-static void require_add_operands(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, const char *what) {
+// Both operands of a sorted add: CSR, same shape (the add checks their arrays).
+static void require_add_shapes(const tr_csx_t *A, const tr_csx_t *C, const char *what) {
     const std::string w(what);
     check_csx(C, "C");
     TR_REQUIRE(A->majordim == TR_ROWS && C->majordim == TR_ROWS, w + ": operands must be CSR");
     TR_REQUIRE(A->nrows == C->nrows && A->ncols == C->ncols, w + ": shape mismatch");
-    const tr_csx_t *m[2] = {A, C};
-    int32_t hs[2];
-    check_tiles(ctx, m, 2, hs);
-    if ((hs[0] | hs[1]) & 3) fail(TR_ERR_INVALID, w + ": malformed CSR operand");
-    if ((hs[0] | hs[1]) & 4) fail(TR_ERR_INVALID, w + ": operands need sorted unique columns");
 }
 
 int tr_spadd(tr_ctx_t ctx, const tr_csx_t *A, tr_csx_t *C) {
@@ -482,9 +484,9 @@ int tr_spadd(tr_ctx_t ctx, const tr_csx_t *A, tr_csx_t *C) {
             copy_tile(ctx, A, C);  // KokkosWrap.hpp:403-407 (deep copy here)
             return;
         }
-        require_add_operands(ctx, A, C, "tr_spadd");
+        require_add_shapes(A, C, "tr_spadd");
         tr_csx_t acc;
-        spadd(ctx, A, C, &acc);
+        spadd(ctx, A, C, &acc, "tr_spadd");
         if (ctx_owned(ctx, C)) release_csx(ctx, C);
         *C = acc;
     });
@@ -496,14 +498,15 @@ int tr_spadd_into(tr_ctx_t ctx, const tr_csx_t *A, const tr_csx_t *B, tr_csx_t *
     return guarded(ctx, [&] {
         TR_REQUIRE(out != nullptr && nnz_needed != nullptr, "tr_spadd_into: null output");
         check_csx(A, "A");
-        require_add_operands(ctx, A, B, "tr_spadd_into");
+        require_add_shapes(A, B, "tr_spadd_into");
         TR_REQUIRE(capacity >= 0 && capacity <= INT32_MAX, "tr_spadd_into: capacity must be in [0, INT32_MAX]");
         TR_REQUIRE(out->ptr_vec != nullptr && (capacity == 0 || (out->idx_vec && out->val)),
                    "tr_spadd_into: output arrays missing");
         for (const tr_csx_t *in : {A, B})
             TR_REQUIRE(out->ptr_vec != in->ptr_vec && out->idx_vec != in->idx_vec && out->val != in->val,
                        "tr_spadd_into: output aliases an operand");
-        const int64_t nnz = spadd_into(ctx, A, B, out->ptr_vec, out->idx_vec, out->val, capacity);
+        const int64_t nnz =
+            spadd_into(ctx, A, B, out->ptr_vec, out->idx_vec, out->val, capacity, "tr_spadd_into");
         *nnz_needed = nnz;
         if (nnz > capacity) fail(TR_ERR_OVERFLOW, "tr_spadd_into: result needs " + std::to_string(nnz) +
                                                       " entries, capacity " + std::to_string(capacity));

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void k_masks(const MaskJob *__restrict__ jobs,
 // guard word (tr_batch_check reports it) and zero the device-side counts the
 // later kernels loop over, so nothing is written outside the batch's
 // buffers.  Bits: 8 operand nnz changed, 1 products differ from the plan,
-// 2/4 (the add) chunk or output offsets differ.
+// 4 (the add) output offsets differ.
 struct GuardOperand {
     const int32_t *ptr;
     int32_t n;      // ptr has n + 1 entries
@@ -386,7 +386,6 @@ void batch_body(tr_batch *b, bool capture) {
     if (!capture) {
         // add tasks: X = products (64-bit global rows), Y = C_in
         std::vector<AddTaskDev> at(b->nt);
-        int64_t ny = 0;
         for (int t = 0; t < b->nt; ++t) {
             AddTaskDev &a = at[t];
             a = AddTaskDev{};
@@ -398,7 +397,7 @@ void batch_body(tr_batch *b, bool capture) {
                 a.yp = C.ptr_vec;
                 a.yi = C.idx_vec;
                 a.yv = C.val;
-                ny += C.nnz;
+                a.ny = C.nnz;
             } else {
                 a.yp = b->zero_ptr;
                 a.yi = nullptr;
@@ -406,16 +405,19 @@ void batch_body(tr_batch *b, bool capture) {
             }
             a.optr = b->o_ptr + b->optr_off[t];
             a.m = b->A[t].nrows;
+            a.n = b->B[t].ncols;
+            a.nx = b->p_base[t + 1] - b->p_base[t];
         }
-        add_setup(ctx, *b->ws_add, b->ap, at, b->p_total, ny);
+        add_setup(ctx, *b->ws_add, b->ap, at);
     }
     add_count(ctx, b->ap, capture);
     if (!capture) {
         b->o_total = add_total(ctx, b->ap);
-        b->o_idx = (int32_t *)b->own(sizeof(int32_t) * (size_t)std::max<int64_t>(b->o_total, 1));
-        b->o_val = (double *)b->own(sizeof(double) * (size_t)std::max<int64_t>(b->o_total, 1));
+        const size_t o = (size_t)std::max<int64_t>(b->o_total, 1);
+        add_output(*b->ws_add, b->ap, [&] { b->o_idx = (int32_t *)b->own(sizeof(int32_t) * o); });
+        add_output(*b->ws_add, b->ap, [&] { b->o_val = (double *)b->own(sizeof(double) * o); });
     }
-    add_write(ctx, b->ap, b->o_idx, b->o_val);
+    add_write(ctx, b->ap, b->o_idx, b->o_val, capture);
 }
 
 }  // namespace
@@ -545,9 +547,7 @@ int tr::batch_create(tr_ctx_t ctx, int32_t ntasks, const tr_csx_t *A, const tr_c
                 b->o_base[t] = b->p_base[t];
                 continue;
             }
-            const int32_t g = b->ap.h[t].row_base;
-            const int64_t cs = read_scalar<int64_t>(ctx, b->ap.cstart + g);
-            b->o_base[t] = read_scalar<int64_t>(ctx, b->ap.coff + cs);
+            b->o_base[t] = read_scalar<int64_t>(ctx, b->ap.first + b->ap.h[t].unit0);
         }
         for (int t = 0; t < ntasks; ++t)
             b->o_nnz[t] = (t + 1 < ntasks ? b->o_base[t + 1] : b->o_total) - b->o_base[t];

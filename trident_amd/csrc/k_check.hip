@@ -189,6 +189,19 @@ void check_begin(tr_ctx *ctx, const tr_csx_t *const *m, int n) {
     launch_check(ctx, nullptr, k, pair, g);
 }
 
+void check_pointers(tr_ctx *ctx, const tr_csx_t *const *m, int n) {
+    CheckPair pair{};
+    CheckGrid g;
+    check_open(ctx);
+    ctx->check_twin = false;
+    for (int t = 0; t < n; ++t) {
+        pair.j[t] = check_job(m[t]);
+        check_place(pair.j[t], g);
+    }
+    TR_LAUNCH(ctx, "check_ptr", k_check_ptr, (uint32_t)g.blocks, 256, 0, (const CheckJob *)nullptr, n, pair,
+              ctx->status);
+}
+
 void check_result(tr_ctx *ctx, int32_t *status, int n) {
     for (int t = 0; t < n; ++t) {
         const uint8_t *f = ctx->status + 4 * (t > 0 && ctx->check_twin ? 0 : t);

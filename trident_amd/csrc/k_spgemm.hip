@@ -2132,6 +2132,13 @@ void *Workspace::get(int slot, size_t bytes) {
     return p[slot];
 }
 
+void Workspace::drop(int slot) {
+    if (!owned) return scratch_drop(ctx, slot);
+    if (p[slot]) ctx->pool.release(p[slot]);
+    p[slot] = nullptr;
+    sz[slot] = 0;
+}
+
 void Workspace::release() {
     if (!owned || !ctx) return;
     for (size_t s = 0; s < p.size(); ++s)

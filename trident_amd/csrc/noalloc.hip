@@ -4,8 +4,7 @@
 // loops, harnesses that forbid hipMalloc.  tr_spadd_into_noalloc is
 // tr_spadd_into (the double-buffer add of sp_mma_hybrid,
 // include/cusparse_helpers.cuh:708-739) with every temporary of the add
-// (task table, per-row chunk counts, chunk rows and offsets, scan partials,
-// validation bitmaps) carved from one file-scope device array instead of the
+// (unit splits, counts and offsets, scan partials, merge bits) carved from one file-scope device array instead of the
 // context's pool.  Inputs and outputs are still the caller's.
 //
 // The array is kNoallocBytes per GPU, held for the life of the process by
@@ -62,23 +61,22 @@ static char *noalloc_base(int device) {
 
 int64_t noalloc_spadd_into(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, tr_csx_t *out, int64_t capacity) {
     char *base = noalloc_base(ctx->device);
-    // [reserved | add temporaries], 256-byte pieces; the reserved part is the
-    // documented limit's share of the operand checks
-    const size_t val_bytes = (256 + sizeof(uint32_t) * (size_t)(std::max(A->nnz, C->nnz) / 32 + 2) + 255) & ~(size_t)255;
-    const size_t add_bytes = spadd_fixed_bytes(A->nrows, A->nnz, C->nnz);
-    const size_t need = val_bytes + add_bytes;
+    // The documented limit: operands are accepted by what a merge of row
+    // chunks and its checks would need.  The add needs 20 bytes per 512 rows
+    // and entries (39 MB for the most entries that pass) and works with what
+    // is left for its merge bits.
+    auto piece = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const int64_t rows = A->nrows, chunks = rows + (A->nnz + C->nnz) / 4096 + 1;
+    const size_t need = piece(256 + 4 * (size_t)(std::max(A->nnz, C->nnz) / 32 + 2)) + piece(96) +
+                        piece(4 * (size_t)(rows + 1)) + piece(8 * (size_t)(rows + 1)) + piece(4 * (size_t)chunks) +
+                        piece(4 * (size_t)(chunks + 1)) + piece(8 * (size_t)(chunks + 1)) +
+                        piece(scan_tmp_bytes(std::max(chunks, rows)));
     if (need > kNoallocBytes)
         fail(TR_ERR_INVALID, "tr_spadd_into_noalloc: operands need " + std::to_string(need) +
                                  " bytes of scratch, more than the fixed " + std::to_string(kNoallocBytes) +
                                  " (use tr_spadd_into)");
-    const tr_csx_t *m[2] = {A, C};
-    int32_t hs[2];
-    check_tiles(ctx, m, 2, hs);
-    const int32_t s0 = hs[0], s1 = hs[1];
-    if ((s0 | s1) & 3) fail(TR_ERR_INVALID, "tr_spadd_into_noalloc: malformed CSR operand");
-    if ((s0 | s1) & 4) fail(TR_ERR_INVALID, "tr_spadd_into_noalloc: operands need sorted unique columns");
-    return spadd_into_fixed(ctx, A, C, out->ptr_vec, out->idx_vec, out->val, capacity, base + val_bytes,
-                            add_bytes);
+    return spadd_into_fixed(ctx, A, C, out->ptr_vec, out->idx_vec, out->val, capacity, "tr_spadd_into_noalloc", base,
+                            kNoallocBytes);
 }
 
 }  // namespace tr

@@ -101,6 +101,7 @@ struct Workspace {
     Workspace(tr_ctx *c, bool own)
         : ctx(c), owned(own), p(S_NUM_SLOTS, nullptr), sz(S_NUM_SLOTS, 0), req(S_NUM_SLOTS, 0) {}
     void *get(int slot, size_t bytes);
+    void drop(int slot);
     void release();
     ~Workspace() { release(); }
     Workspace(const Workspace &) = delete;
@@ -148,18 +149,25 @@ struct AddTaskDev {
     const int32_t *yi;
     const double *yv;
     int32_t *optr;     // output row pointer (m + 1), rebased to the task
+    int64_t nx, ny;    // entries of X_t and Y_t (planned)
     int32_t m;
+    int32_t n;         // columns
     int32_t row_base;
+    int32_t unit0;     // first work unit
 };
 
+// One add job.  No device table (d): the plan's one task goes by value.
 struct AddPlan {
     int nt = 0;
-    int32_t rows_total = 0;
     std::vector<AddTaskDev> h;
     AddTaskDev *d = nullptr;
-    int32_t *nch = nullptr, *crow = nullptr, *ccount = nullptr;
-    int64_t *cstart = nullptr, *coff = nullptr;
-    int64_t chunk_cap = 0, nchunks = 0;
+    int32_t nunits = 0;
+    int2 *split = nullptr;      // per unit: first row, first X entry
+    int32_t *counts = nullptr;  // per unit: entries kept
+    int64_t *first = nullptr;   // per unit: first output entry (and the total)
+    uint64_t *bits = nullptr;   // the merge of `kept` units and the one behind them
+    int32_t kept = 0;
+    bool wide = false;          // columns beyond the 32-bit merge keys
     int64_t *scan_tmp = nullptr;
     // replay guard (batches): device word set on a mismatch with the plan,
     // and the planned first output entry of every task (nt + 1 entries)
@@ -167,11 +175,23 @@ struct AddPlan {
     const int64_t *expect = nullptr;
 };
 
-void add_setup(tr_ctx *ctx, Workspace &ws, AddPlan &ap, const std::vector<AddTaskDev> &tasks, int64_t nnz_x,
-               int64_t nnz_y);
-void add_count(tr_ctx *ctx, AddPlan &ap, bool capture);
+void add_setup(tr_ctx *ctx, Workspace &ws, AddPlan &ap, const std::vector<AddTaskDev> &tasks);
+void add_count(tr_ctx *ctx, AddPlan &ap, bool capture, uint8_t *findings = nullptr);
 int64_t add_total(tr_ctx *ctx, AddPlan &ap);
-void add_write(tr_ctx *ctx, AddPlan &ap, int32_t *oi, double *ov);
+bool add_make_room(Workspace &ws, AddPlan &ap);
+void add_write(tr_ctx *ctx, AddPlan &ap, int32_t *oi, double *ov, bool capture);
+
+// Allocates an add's output; the merge bits make room if that fails.
+template <typename F>
+void add_output(Workspace &ws, AddPlan &ap, F &&alloc) {
+    try {
+        alloc();
+        return;
+    } catch (const Error &e) {
+        if (e.code != TR_ERR_OOM || !add_make_room(ws, ap)) throw;
+    }
+    alloc();
+}
 
 // Pipeline steps.  In eager mode the host reads counts between steps to size
 // grids and lists; in capture mode every size comes from a previous eager run

@@ -149,6 +149,7 @@ enum ScratchSlot : int {
 };
 
 void *scratch(tr_ctx *ctx, int slot, size_t bytes);
+void scratch_drop(tr_ctx *ctx, int slot);  // back to the pool
 // Bytes the pool sets aside for a request of `b` bytes (256-byte steps up to
 // 1 MiB, 2 MiB granules above); scratch slots grow to 1.25x a request.
 size_t pool_block_bytes(size_t b);
@@ -230,6 +231,7 @@ void launch_check(tr_ctx *ctx, const CheckJob *jobs, int nj, const CheckPair &pa
 bool same_tile(const tr_csx_t *a, const tr_csx_t *b);
 void check_open(tr_ctx *ctx);  // before a launch_check without a table
 void check_begin(tr_ctx *ctx, const tr_csx_t *const *m, int n);
+void check_pointers(tr_ctx *ctx, const tr_csx_t *const *m, int n);  // the pointers alone, every tile
 void check_result(tr_ctx *ctx, int32_t *status, int n);
 void check_tiles(tr_ctx *ctx, const tr_csx_t *const *m, int n, int32_t *status);  // both, with the wait
 
@@ -275,15 +277,15 @@ int spgemm_panels(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *B, int64_t max
                   tr_csx_t *panels, int32_t *row_begin, int32_t max_panels, int32_t *npanels);
 
 // k_spadd.hip
-void spadd(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, tr_csx_t *out);
+// check: the entry point's name, to check both operands on the way (fails with
+// TR_ERR_INVALID), or nullptr for operands that are known to be sorted CSRs.
+void spadd(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, tr_csx_t *out, const char *check = nullptr);
 int64_t spadd_into(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, int32_t *optr, int32_t *oi, double *ov,
-                   int64_t capacity);
+                   int64_t capacity, const char *check);
 // The same add with every temporary carved from the device region
 // [base, base + bytes) instead of the context's pool: no allocation.
-// spadd_fixed_bytes gives the bytes it needs (256-byte aligned pieces).
-size_t spadd_fixed_bytes(int32_t rows, int64_t nnz_x, int64_t nnz_y);
 int64_t spadd_into_fixed(tr_ctx *ctx, const tr_csx_t *A, const tr_csx_t *C, int32_t *optr, int32_t *oi, double *ov,
-                         int64_t capacity, char *base, size_t bytes);
+                         int64_t capacity, const char *check, char *base, size_t bytes);
 
 // noalloc.hip: the per-device static scratch of the allocation-free entry
 // points; noalloc_init runs once per device (from tr_ctx_create, with the
