@@ -1537,40 +1537,49 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
 // sharing one T-slot LDS table per window.  For each window the row's A
 // entries are taken NT at a time (one per thread): each thread finds the
 // part of B_k inside the window (register cursor for rows with <= NT
-// entries, the item's cursor array otherwise), a workgroup scan flattens the
-// products in A-order, and each step applies NT of them.  Slot keys carry the
-// column offset in the high bits and the slot's last pusher of the step in
-// the low bits: products of one step that meet in a slot form a list that
-// the last pusher applies in thread order (= A-order).  A presence bitmap
-// over the window, built after the window's last step, gives every entry its
-// sorted rank (prefix popcounts) for the write-out.
+// entries, the item's cursor array otherwise) and a workgroup scan flattens
+// the products in A-order.
+//
+// The waves take the products in groups of 64 and work on their groups at the
+// same time, but for the sum itself: finding the slots, the operands' loads
+// and the search for lanes that meet in a slot need no order (a free slot
+// holds 0, whoever claims it).  Only the addition to the slots waits for its
+// turn, a count in LDS that every group passes on, so that every slot sums in
+// A-order; lanes of a group that share a slot add one after the other.  The
+// turn is a read, an fma and a write, so the wait is short: it has no cost
+// that a raised wave priority, a sleep in the wait or weaker fences change.
+// (Steps of NT products between barriers, where a slot's last pusher walked a
+// list of the step's products: product of R-MAT s17 12.1 ms, now 10.5; s19
+// 95.5 and 82.5.  With tags of each wave's own, T/2 or T/4 of them, s17 11.1
+// and 11.9: a shared tag costs a round of the search below.)
+// A presence bitmap over the window, built after the window's last group,
+// gives every entry its sorted rank (prefix popcounts) for the write-out.
 //
 // Occupancy: the kernel is bound by the latency of its dependent LDS and
 // memory chains, so resident waves matter most.  The bitmap shares LDS with
-// the step arrays (31 KB per 2048-slot, 256-thread workgroup: five per CU)
+// the group arrays (29 KB per 2048-slot, 256-thread workgroup: five per CU)
 // and the register budget is held to 96 VGPRs (five waves per SIMD); the
-// 4096-slot table (62 KB, 512 threads) fits two workgroups per CU.
+// 4096-slot table (66 KB, 512 threads) fits two workgroups per CU.
 constexpr int kRegSlots = 1;  // register-held A entries per thread in the heavy numeric kernel
 constexpr int kSmallNT = 256;  // threads of the 2048-slot heavy numeric
 constexpr uint32_t kSlotFree = 0xffffffffu;
-constexpr int kTagBits = 10;                        // thread ids < 1023
-constexpr uint32_t kNoTag = (1u << kTagBits) - 1u;  // slot key = column offset << kTagBits | tag
 
 template <int T, int NT>
 struct HeavyWgLds {
-    uint32_t keytag[T];
-    double vals[T];
+    static constexpr int kMarks = 8 * NT;   // products of a round
+    using Id = typename std::conditional<(NT <= 256), uint8_t, uint16_t>::type;  // of a thread
+    uint32_t key[T];                        // column offset of the slot, or kSlotFree
+    double vals[T];                         // 0 in free slots
     int32_t wsum[NT / kWave];
     int32_t nocc;
+    int32_t turn;                           // group of 64 products that is applied next
     union {
-        struct {                    // product steps of a window
-            double pa[NT], pb[NT];  // the step's products (A value, B value) by thread
+        struct {                // products of a window
             int32_t seg_d[NT];  // B position minus flattened product position of segment (A entry) o
-            uint16_t link[NT];  // next older product of the same slot in this step
-            // segments of three rotating product steps: smark[b][p] is the
-            // index of the segment that starts at step position p, or that
-            // covers p where a wave's positions begin; 0 elsewhere
-            __align__(16) typename std::conditional<(NT <= 256), uint8_t, uint16_t>::type smark[3][NT];
+            // smark[p] is the index of the segment that starts at the round's
+            // position p, or that covers p where a group of 64 begins; 0 elsewhere
+            __align__(16) Id smark[kMarks];
+            Id tag[T];  // the last thread that met the slot
         };
         struct {  // extraction of a window: presence bitmap and its prefix counts
             unsigned long long bm[kBmWords];
@@ -1579,88 +1588,37 @@ struct HeavyWgLds {
     };
 };
 
-// marks the segment [excl, excl + len) of the calling thread in the step that
-// starts at product `base`: at its first position in the step, and at every
-// later position of the step where a wave begins, so that the segment of a
-// position is the last mark at or below it in its own wave
-template <int NT, typename M>
+// marks the segment [excl, excl + len) of the calling thread in the round of N
+// products that starts at product `base`: at its first position in the round,
+// and at every later position where a group of 64 begins, so that the segment
+// of a position is the last mark at or below it in its own group
+template <int N, typename M>
 __device__ __forceinline__ void mark_segment(M *smark, int32_t base, int32_t excl, int32_t len) {
     if (len <= 0) return;
     const int32_t rel = excl - base;
-    const int32_t lo = rel > 0 ? rel : 0, hi = rel + len < NT ? rel + len : NT;
-    if (lo >= hi) return;  // the segment has no product in this step
+    const int32_t lo = rel > 0 ? rel : 0, hi = rel + len < N ? rel + len : N;
+    if (lo >= hi) return;  // the segment has no product in this round
     smark[lo] = (M)threadIdx.x;
     for (int32_t ws = (lo & ~63) + 64; ws < hi; ws += 64) smark[ws] = (M)threadIdx.x;
 }
 
-// segment of the calling thread's step position: segments rise with their
-// positions, so the last mark is a running maximum over the wave (one LDS read
-// and six register steps; a start mask and the mark at its highest bit took
-// two dependent reads, and marking an LDS atomic more)
+// segment of the calling lane's position of the group that begins at `group`:
+// segments rise with their positions, so the last mark is a running maximum
+// over the wave (one LDS read and six register steps)
 template <typename M>
-__device__ __forceinline__ int owner_marked(const M *smark) {
-    return (int)wave_incl_max((uint32_t)smark[threadIdx.x]);
+__device__ __forceinline__ int owner_marked(const M *group) {
+    return (int)wave_incl_max((uint32_t)group[lane_id()]);
 }
 
-template <int NT, typename M>
-__device__ __forceinline__ void clear_marks(M *smark, int n) {  // n: whole buffers
+template <int NT, int N, typename M>
+__device__ __forceinline__ void clear_marks(M *smark) {
     uint32_t *w = reinterpret_cast<uint32_t *>(smark);
-    for (int t = threadIdx.x; t < n * NT * (int)sizeof(M) / 4; t += NT) w[t] = 0u;
+    for (int t = threadIdx.x; t < N * (int)sizeof(M) / 4; t += NT) w[t] = 0u;
 }
 
-template <int K>
-__device__ __forceinline__ void exchange(uint32_t (&t)[K], int i, int j) {
-    const uint32_t a = t[i], b = t[j];
-    t[i] = min(a, b);
-    t[j] = max(a, b);
-}
-
-// ascending sort of 4 or 8 thread ids in registers
-__device__ __forceinline__ void sort_ids(uint32_t (&t)[4]) {
-    exchange(t, 0, 1), exchange(t, 2, 3);
-    exchange(t, 0, 2), exchange(t, 1, 3);
-    exchange(t, 1, 2);
-}
-__device__ __forceinline__ void sort_ids(uint32_t (&t)[8]) {
-    exchange(t, 0, 1), exchange(t, 2, 3), exchange(t, 4, 5), exchange(t, 6, 7);
-    exchange(t, 0, 2), exchange(t, 1, 3), exchange(t, 4, 6), exchange(t, 5, 7);
-    exchange(t, 1, 2), exchange(t, 5, 6), exchange(t, 0, 4), exchange(t, 3, 7);
-    exchange(t, 1, 5), exchange(t, 2, 6);
-    exchange(t, 1, 4), exchange(t, 3, 6);
-    exchange(t, 2, 4), exchange(t, 3, 5);
-    exchange(t, 3, 4);
-}
-
-// v after the products of ids t[0..K), ascending, kNoTag ids (at the end)
-// left out; t[0] and t[1] exist
-template <int K>
-__device__ __forceinline__ double apply_ids(const double *pa, const double *pb, const uint32_t (&t)[K], double v) {
-#pragma unroll
-    for (int g = 0; g < K; g += 4) {
-        double a[4], b[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t q = g + i < 2 || t[g + i] != kNoTag ? t[g + i] : t[0];
-            a[i] = pa[q];
-            b[i] = pb[q];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const double w = __fma_rn(a[i], b[i], v);
-            v = g + i < 2 || t[g + i] != kNoTag ? w : v;
-        }
-    }
-    return v;
-}
-
-// Every word is written with a select, so the mask stays in registers
-// (a conditional store to one element becomes an indexed private array).
-template <int NT>
-__device__ __forceinline__ void mask_set(uint64_t (&mk)[NT / kWave], uint32_t t) {
-    const uint64_t bit = 1ull << (t & 63);
-#pragma unroll
-    for (int w = 0; w < NT / kWave; ++w) mk[w] |= ((int)(t >> 6) == w) ? bit : 0ull;
-}
+// LDS only: loads in flight from global memory are not waited for
+__device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
+__device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
 
 // workgroup exclusive scan of v; returns the exclusive prefix, *total = sum
 template <int NT>
@@ -1691,9 +1649,14 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                                                      int32_t dense_width) {
     constexpr uint32_t kLog = __builtin_ctz(T);
     __shared__ HeavyWgLds<T, NT> L;
-    const int tid = threadIdx.x, l = lane_id();
-    for (int t = tid; t < T; t += NT) L.keytag[t] = kSlotFree;
-    if (tid == 0) L.nocc = 0;
+    constexpr int kWaves = NT / kWave, kMarks = HeavyWgLds<T, NT>::kMarks;
+    using Id = typename HeavyWgLds<T, NT>::Id;
+    const int tid = threadIdx.x, l = lane_id(), w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    for (int t = tid; t < T; t += NT) {
+        L.key[t] = kSlotFree;
+        L.vals[t] = 0.0;
+    }
+    if (tid == 0) L.nocc = L.turn = 0;
     __syncthreads();
     const int32_t nitems = cnt->items;
     const int32_t slot = (int32_t)blockIdx.x;
@@ -1751,7 +1714,7 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
             const uint32_t hmul = (W.c1 - W.c0) <= dense_width ? (1u << (32 - kLog)) : 0x9E3779B1u;
             int nfresh = 0;
             for (int32_t pb = a0, slot = 0; pb < a1; pb += NT, ++slot) {
-                clear_marks<NT>(L.smark[0], 2);
+                clear_marks<NT, kMarks>(L.smark);
                 // this thread's k-slot: A entry p, B segment [s, e) inside the window
                 const int32_t p = pb + tid;
                 int32_t s = 0, e = 0;
@@ -1809,140 +1772,88 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                 const int32_t slen = e - s;
                 const int32_t excl = wg_excl_scan<NT>(slen, L.wsum, &total);
                 L.seg_d[tid] = s - excl;
-                // segments of the first two steps (their marks were cleared
-                // before the scan's barrier)
-                mark_segment<NT>(L.smark[0], 0, excl, slen);
-                mark_segment<NT>(L.smark[1], NT, excl, slen);
+                // (the marks were cleared before the scan's barrier)
+                mark_segment<kMarks>(L.smark, 0, excl, slen);
                 __syncthreads();
-                // products x = x0 + tid, flattened in A-order; the B entry of the
-                // next step is loaded while the current step is applied
-                int32_t jn = 0;
-                double bn = 0.0, an = 0.0;
-                const int o0 = owner_marked(L.smark[0]);
-                if (tid < total) {
-                    const int o = o0;
-                    const int32_t q = L.seg_d[o] + tid;
-                    an = av[pb + o];
-                    jn = bi[q];
-                    bn = bv[q];
-                }
-                // step k reads the marks of step k + 1 (buffer bA), clears
-                // buffer bC before its first barrier and marks step k + 2 in it
-                // between its barriers
-                int bA = 1, bC = 2;
-                for (int32_t x0 = 0; x0 < total; x0 += NT) {
-                    const int32_t x = x0 + tid;
-                    bool act = x < total;
-                    const int32_t j = jn;
-                    const double b = bn, ao = an;
-                    const int32_t xn = x + NT;
-                    // claim or join this product's slot first: the CAS round
-                    // trip overlaps the next step's owner lookup below
-                    uint32_t h = 0, key = 0, me = 0, old = kSlotFree;
-                    if (act) {
-                        const uint32_t off = (uint32_t)(j - W.c0);
-                        key = off << kTagBits;
-                        me = key | (uint32_t)tid;
-                        h = (off * hmul) >> (32 - kLog);
-                        old = atomicCAS(&L.keytag[h], kSlotFree, me);
+                // products flattened in A-order, in groups of 64: the waves take
+                // the groups in turn
+                const int32_t ngroups = (total + kWave - 1) / kWave;
+                for (int32_t base = 0; base < total; base += kMarks) {
+                    if (base > 0) {
+                        __syncthreads();
+                        clear_marks<NT, kMarks>(L.smark);
+                        __syncthreads();
+                        mark_segment<kMarks>(L.smark, base, excl, slen);
+                        __syncthreads();
                     }
-                    const int o = owner_marked(L.smark[bA]);
-                    if (xn < total) {
-                        const int32_t q = L.seg_d[o] + xn;
-                        an = av[pb + o];
-                        jn = bi[q];
-                        bn = bv[q];
-                    }
-                    clear_marks<NT>(L.smark[bC], 1);
-                    // insert: the first product of a slot in this step creates or
-                    // claims it; every later one pushes itself onto the slot's
-                    // list (the tag field holds the last pusher, link[] the rest)
-                    if (act) {
-                        const uint32_t off = key >> kTagBits;
-                        // probe to a free slot (claimed) or this key's slot; the
-                        // bound only guards a table the symbolic counts overfilled
-                        bool more = old != kSlotFree && (old >> kTagBits) != off;
-                        for (int probe = 1; probe < T && ballot(more); ++probe) {
+                    const int32_t gend = min(ngroups, (base + kMarks) / kWave);
+                    int32_t grp = base / kWave + w;
+                    int32_t jn = 0;
+                    double bn = 0.0, an = 0.0;
+                    // product of group q that is this lane's
+                    auto load = [&](int32_t q) {
+                        if (q >= gend) return;
+                        const int32_t x = q * kWave + l;
+                        const int o = owner_marked(&L.smark[q * kWave - base]);
+                        if (x < total) {
+                            const int32_t t = L.seg_d[o] + x;
+                            an = av[pb + o];
+                            jn = bi[t];
+                            bn = bv[t];
+                        }
+                    };
+                    load(grp);
+                    for (; grp < gend; grp += kWaves) {
+                        bool act = grp * kWave + l < total;
+                        const double a = an, b = bn;
+                        // find or claim the slot: in any order, a free slot holds 0
+                        const uint32_t off = (uint32_t)(jn - W.c0);
+                        uint32_t h = (off * hmul) >> (32 - kLog);
+                        bool more = act;
+                        for (int probe = 0; probe < T && ballot(more); ++probe) {
                             if (more) {
-                                h = (h + 1) & (T - 1);
-                                old = atomicCAS(&L.keytag[h], kSlotFree, me);
-                                more = old != kSlotFree && (old >> kTagBits) != off;
+                                const uint32_t old = atomicCAS(&L.key[h], kSlotFree, off);
+                                nfresh += old == kSlotFree ? 1 : 0;
+                                more = old != kSlotFree && old != off;
+                                if (more) h = (h + 1) & (T - 1);
                             }
                         }
-                        uint32_t prev = kNoTag;
-                        if (old == kSlotFree) {
-                            L.vals[h] = 0.0;
-                            ++nfresh;
-                        } else if (!more) {
-                            prev = atomicExch(&L.keytag[h], me) & kNoTag;
-                        } else {
+                        if (more) {
                             atomicOr(&cnt->overflow, 8);  // table full: symbolic counts were wrong
                             act = false;
                         }
-                        if (act) {
-                            L.link[tid] = (uint16_t)prev;
-                            L.pa[tid] = ao;
-                            L.pb[tid] = b;
+                        // lanes of the group that meet in a slot: every lane
+                        // writes itself to the slot's tag, and one that reads
+                        // another may share the slot (or another wave came in
+                        // between): of lanes that share one, all but one do.
+                        // turn_of: lanes of the same slot before this one
+                        if (act) L.tag[h] = (Id)tid;
+                        wave_sync();
+                        uint64_t shared = ballot(act && L.tag[h] != (Id)tid);
+                        int turn_of = 0, turns = 1;
+                        while (shared) {
+                            const int f = __ffsll((unsigned long long)shared) - 1;
+                            const bool same = act && h == read_lane(h, f);
+                            const uint64_t m = ballot(same);
+                            if (same) turn_of = rank_below(m);
+                            turns = max(turns, __popcll(m));
+                            shared &= ~m;
                         }
-                    }
-                    __syncthreads();
-                    // the last pusher of each slot applies the slot's products of
-                    // this step in thread (= A) order: it follows the slot's list,
-                    // sorts the thread ids in registers and reads the operands
-                    // in their order, all reads of four at once.  (R-MAT s19:
-                    // 78% of the products are alone in their slot, 14% in
-                    // pairs; a wave's longest list is over four in one step of
-                    // six, over eight in one of fifty.)  Longer lists walk a
-                    // bitmask of ids
-                    if (act && (L.keytag[h] & kNoTag) == (uint32_t)tid) {
-                        const uint32_t t1 = L.link[tid];
-                        double v = L.vals[h];
-                        if (t1 == kNoTag) {
-                            v = __fma_rn(ao, b, v);
-                        } else {
-                            auto next = [&](uint32_t t) { return t == kNoTag ? kNoTag : (uint32_t)L.link[t]; };
-                            uint32_t t4[4] = {(uint32_t)tid, t1, L.link[t1], kNoTag};
-                            t4[3] = next(t4[2]);
-                            const uint32_t t5 = next(t4[3]);
-                            if (t5 == kNoTag) {
-                                sort_ids(t4);
-                                v = apply_ids(L.pa, L.pb, t4, v);
-                            } else {
-                                uint32_t t8[8] = {t4[0], t4[1], t4[2], t4[3], t5, kNoTag, kNoTag, kNoTag};
-#pragma unroll
-                                for (int i = 5; i < 8; ++i) t8[i] = next(t8[i - 1]);
-                                uint32_t t = next(t8[7]);
-                                if (t == kNoTag) {
-                                    sort_ids(t8);
-                                    v = apply_ids(L.pa, L.pb, t8, v);
-                                } else {
-                                    uint64_t mk[NT / kWave];
-#pragma unroll
-                                    for (int w = 0; w < NT / kWave; ++w) mk[w] = 0ull;
-#pragma unroll
-                                    for (int i = 0; i < 8; ++i) mask_set<NT>(mk, t8[i]);
-                                    for (; t != kNoTag; t = L.link[t]) mask_set<NT>(mk, t);
-#pragma unroll
-                                    for (int w = 0; w < NT / kWave; ++w) {
-                                        uint64_t mw = mk[w];
-                                        while (mw) {
-                                            const int q = w * kWave + __ffsll((unsigned long long)mw) - 1;
-                                            mw &= mw - 1ull;
-                                            v = __fma_rn(L.pa[q], L.pb[q], v);
-                                        }
-                                    }
-                                }
-                            }
+                        load(grp + kWaves);
+                        // wait for the groups before this one, which other waves hold
+                        while (__hip_atomic_load(&L.turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != grp) {
                         }
-                        L.vals[h] = v;
-                        L.keytag[h] = key | kNoTag;
+                        lds_acquire();
+                        for (int q = 0; q < turns; ++q) {
+                            if (act && turn_of == q) L.vals[h] = __fma_rn(a, b, L.vals[h]);
+                            wave_sync();
+                        }
+                        lds_release();
+                        if (l == 0) __hip_atomic_store(&L.turn, grp + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     }
-                    if (x0 + 2 * NT < total) mark_segment<NT>(L.smark[bC], x0 + 2 * NT, excl, slen);
-                    __syncthreads();
-                    bA = bC;
-                    bC = bC == 2 ? 0 : bC + 1;
                 }
-                __syncthreads();  // seg_* are rewritten by the next batch
+                __syncthreads();  // seg_d and the marks are rewritten by the next batch
+                if (tid == 0) L.turn = 0;
             }
             if (!full) have_cursor = true;
             // entries created in this window (each thread counted its fresh inserts)
@@ -1965,7 +1876,7 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
             uint32_t st_rk[kSt];
             double st_v[kStash];
             const int32_t lim = min(W.cnt, kStage);  // never write past the window
-            int32_t *sidx = reinterpret_cast<int32_t *>(L.keytag);
+            int32_t *sidx = reinterpret_cast<int32_t *>(L.key);
             if (dense) {
                 // the thread's slots (h = tid + u NT) by column offset, ranked
                 // one kBmWidth-column pass at a time with a presence bitmap
@@ -1978,14 +1889,14 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
 #pragma unroll
                 for (int u = 0; u < kSt; ++u) {
                     const int h = tid + u * NT;
-                    const uint32_t kt = h < T ? L.keytag[h] : kSlotFree;
-                    st_rk[u] = kt == kSlotFree ? kNone : kt >> kTagBits;
+                    const uint32_t kt = h < T ? L.key[h] : kSlotFree;
+                    st_rk[u] = kt;  // (kNone is kSlotFree)
                 }
                 if (direct) {
                     const int wsl = __builtin_amdgcn_readfirstlane(tid / kWave);  // word of slot tid in round 0
 #pragma unroll 1
                     for (int u = 0; u < kSt; ++u) {
-                        const uint64_t m = ballot(L.keytag[tid + u * NT] != kSlotFree);
+                        const uint64_t m = ballot(L.key[tid + u * NT] != kSlotFree);
                         if (l == 0) L.bm[u * (NT / kWave) + wsl] = m;
                     }
                 }
@@ -2062,15 +1973,15 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                 uint32_t *lkey = reinterpret_cast<uint32_t *>(L.bm);
                 uint16_t *lslot = L.wpre;
                 int32_t mine = 0;
-                for (int h = tid; h < T; h += NT) mine += (L.keytag[h] != kSlotFree) ? 1 : 0;
+                for (int h = tid; h < T; h += NT) mine += (L.key[h] != kSlotFree) ? 1 : 0;
                 int32_t tot;
                 int32_t pos = wg_excl_scan<NT>(mine, L.wsum, &tot);
                 const bool fits = tot <= kSparseH + 127;  // bound of a sparse window
                 if (fits)
                     for (int h = tid; h < T; h += NT) {
-                        const uint32_t kt = L.keytag[h];
+                        const uint32_t kt = L.key[h];
                         if (kt == kSlotFree) continue;
-                        lkey[pos] = kt >> kTagBits;
+                        lkey[pos] = kt;
                         lslot[pos] = (uint16_t)h;
                         ++pos;
                     }
@@ -2107,7 +2018,10 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                 __builtin_nontemporal_store(L.vals[e], &ov[e]);
             }
             __syncthreads();
-            for (int t = tid; t < T; t += NT) L.keytag[t] = kSlotFree;
+            for (int t = tid; t < T; t += NT) {
+                L.key[t] = kSlotFree;
+                L.vals[t] = 0.0;
+            }
             if (tid == 0) L.nocc = 0;
             __syncthreads();
         }
