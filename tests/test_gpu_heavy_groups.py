@@ -46,3 +46,23 @@ def test_shared_slots(kind, entries, table):
             ctx.set_tuning(dict(tuning_default(), heavy_table=4096, window_entries=1920, dense_width=4096))
         c = spgemm(ctx.upload(a), ctx.upload(b)).download()
     assert np.array_equal(c.ptr, p) and np.array_equal(c.idx, i) and np.array_equal(c.val, v)
+
+
+@pytest.mark.parametrize("ncols", [400, 300000, 600000])
+def test_b_row_lengths(ctx, ncols):
+    """Heavy rows over B rows of every length around those that are taken four
+    at a time (up to 128 columns), in any order, empty ones between them."""
+    rng = np.random.default_rng(ncols)
+    lens = [n for n in (0, 1, 15, 16, 17, 32, 33, 63, 64, 65, 112, 113, 127, 128, 129, 191, 255, 256, 257, 300) for _ in range(40)]
+    rng.shuffle(lens)
+    b = _csr([np.sort(rng.choice(ncols, n, replace=False)) for n in lens], ncols, rng)
+    some = [np.sort(rng.choice(len(lens), k, replace=False)) for k in (20, 63, 64, 65, 500, 513, 800)]
+    only = [np.flatnonzero(np.array(lens) == n) for n in (128, 129, 300)]
+    a = _csr(some + only, len(lens), rng)
+    p, i, v = oracle.spgemm(a, b)
+    da, db = ctx.upload(a), ctx.upload(b)
+    d = spgemm(da, db)
+    c = d.download()
+    assert np.array_equal(c.ptr, p) and np.array_equal(c.idx, i) and np.array_equal(c.val, v)
+    for x in (d, da, db):
+        x.free()

@@ -164,6 +164,40 @@ __device__ __forceinline__ void stream_cols_v4(const TR_GLOBAL int32_t *__restri
     if (p3) f(x3.x), f(x3.y), f(x3.z), f(x3.w);
 }
 
+// Same visit of the B rows of up to kShortB columns that the lanes in `rows`
+// hold (first position, length), four rows at a time with 16 lanes each: a row
+// by itself is a round trip that fills few lanes.  The order of the rows is
+// free.  (One row at a time, then rows of up to 32, 64, 128, 192 columns by
+// four, up to 256 by two: product of 15013 vertices 665, 628, 608, 590, 595,
+// 608 us; R-MAT s17 10.60, 10.60, 10.54, 10.45, 10.43, 10.49 ms; Galerkin 96^3
+// 2078, 2025, 2030, 2022, 2018, 2019 us.)
+constexpr int kShortB = 128, kShortBLanes = 16;
+template <typename F>
+__device__ __forceinline__ void stream_short_rows(const TR_GLOBAL int32_t *__restrict__ bi, int32_t bs, int32_t len,
+                                                  uint64_t rows, F &&f) {
+    constexpr int kAtOnce = kWave / kShortBLanes, kLoads = kShortB / kShortBLanes;
+    const int l = lane_id(), grp = l / kShortBLanes;
+    while (rows) {
+        int t = -1;
+#pragma unroll
+        for (int g = 0; g < kAtOnce; ++g) {
+            if (rows) t = grp == g ? __ffsll((unsigned long long)rows) - 1 : t;
+            rows &= rows - 1;
+        }
+        const int32_t s = __shfl(bs, t & (kWave - 1), kWave), all = __shfl(len, t & (kWave - 1), kWave);
+        const int32_t n = t >= 0 ? all : 0;
+        int32_t j[kLoads];
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const int32_t e = q * kShortBLanes + l % kShortBLanes;
+            if (e < n) j[q] = bi[s + e];
+        }
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q)
+            if (q * kShortBLanes + l % kShortBLanes < n) f(j[q]);
+    }
+}
+
 // Streaming of B rows with their loads one round trip ahead, for kernels
 // whose LDS leaves registers to spare (the 2^20-bit heavy symbolic runs one
 // 16-wave workgroup per CU): each row's first round trip (its unaligned head
@@ -773,9 +807,11 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
                 if constexpr (kEagerB) {
                     stream_rows_ahead(bi, bs, be, nk, mark);
                 } else {
-                    for (int t = 0; t < nk; ++t) {
-                        const int32_t s = __shfl(bs, t, kWave), e = __shfl(be, t, kWave);
-                        stream_cols_v4(bi, s, e, mark);
+                    const int32_t len = be - bs;
+                    stream_short_rows(bi, bs, len, ballot(len > 0 && len <= kShortB), mark);
+                    for (uint64_t rows = ballot(len > kShortB); rows; rows &= rows - 1) {
+                        const int t = __ffsll((unsigned long long)rows) - 1;
+                        stream_cols_v4(bi, read_lane(bs, t), read_lane(be, t), mark);
                     }
                 }
             }
