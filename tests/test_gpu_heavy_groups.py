@@ -2,7 +2,7 @@
 oracle with values over 2^+-20, so that a sum in another order shows.  Products
 of one A entry fall in groups of 64 of every wave, columns are met once, by two
 entries, or by every entry, next to each other or rounds apart, and a batch
-holds more products than a round (2048) of marks."""
+holds more products than a round of marks (4096)."""
 import numpy as np
 import pytest
 

@@ -1585,72 +1585,48 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
 // turn is a read, an fma and a write, so the wait is short: it has no cost
 // that a raised wave priority, a sleep in the wait or weaker fences change.
 // (Steps of NT products between barriers, where a slot's last pusher walked a
-// list of the step's products: product of R-MAT s17 12.1 ms, now 10.5; s19
-// 95.5 and 82.5.  With tags of each wave's own, T/2 or T/4 of them, s17 11.1
-// and 11.9: a shared tag costs a round of the search below.)
+// list of the step's products: product of R-MAT s17 12.1 ms, with turns 10.5;
+// s19 95.5 and 82.5.  With tags of each wave's own, T/2 or T/4 of them, s17
+// 11.1 and 11.9: a shared tag costs a round of the search below.  Also slower,
+// s19: buckets of four keys read at once 85.9, a second hash for the step 83.6,
+// B as 16-byte records 89.)
 // A presence bitmap over the window, built after the window's last group,
 // gives every entry its sorted rank (prefix popcounts) for the write-out.
 //
 // Occupancy: the kernel is bound by the latency of its dependent LDS and
-// memory chains, so resident waves matter most.  The bitmap shares LDS with
-// the group arrays (29 KB per 2048-slot, 256-thread workgroup: five per CU)
-// and the register budget is held to 96 VGPRs (five waves per SIMD); the
-// 4096-slot table (66 KB, 512 threads) fits two workgroups per CU.
+// memory chains, so resident waves matter most: product of R-MAT s19 97.6 ms
+// with four workgroups per CU, 82.4 with five, 75.0 with six (s17 12.3, 10.5,
+// 9.6).  For the six, a 2048-slot, 256-thread workgroup keeps to 26.4 KB: the
+// tags are the keys' upper bits, the bitmap takes the keys' space once they
+// are in registers, and the segments of a round of 4096 products are one bit
+// per start.  The register budget is held to 80 VGPRs; the 4096-slot table (53
+// KB, 512 threads) fits three workgroups per CU.
 constexpr int kRegSlots = 1;  // register-held A entries per thread in the heavy numeric kernel
 constexpr int kSmallNT = 256;  // threads of the 2048-slot heavy numeric
 constexpr uint32_t kSlotFree = 0xffffffffu;
+constexpr int kOffBits = 20;  // a slot's key: column offset, the last thread that met it above
+constexpr uint32_t kOffMask = (1u << kOffBits) - 1u;
+constexpr int kRound = kWave * kWave;  // products of a round of marks
 
 template <int T, int NT>
 struct HeavyWgLds {
-    static constexpr int kMarks = 8 * NT;   // products of a round
-    using Id = typename std::conditional<(NT <= 256), uint8_t, uint16_t>::type;  // of a thread
-    uint32_t key[T];                        // column offset of the slot, or kSlotFree
-    double vals[T];                         // 0 in free slots
-    int32_t wsum[NT / kWave];
-    int32_t nocc;
-    int32_t turn;                           // group of 64 products that is applied next
     union {
-        struct {                // products of a window
-            int32_t seg_d[NT];  // B position minus flattened product position of segment (A entry) o
-            // smark[p] is the index of the segment that starts at the round's
-            // position p, or that covers p where a group of 64 begins; 0 elsewhere
-            __align__(16) Id smark[kMarks];
-            Id tag[T];  // the last thread that met the slot
-        };
+        __align__(16) uint32_t key[T];  // kSlotFree in free slots
         struct {  // extraction of a window: presence bitmap and its prefix counts
             unsigned long long bm[kBmWords];
             uint16_t wpre[kBmWords];
         };
     };
+    double vals[T];                     // 0 in free slots
+    // segments (A entries with products in the window) of a batch, in A-order
+    int32_t seg_d[NT];                  // B position minus flattened product position
+    uint64_t starts[kRound / kWave];    // positions of the round where a segment starts
+    typename std::conditional<(NT <= 256), uint8_t, uint16_t>::type seg_o[NT];  // its A entry, from the batch's first
+    int32_t wsum[NT / kWave];
+    int32_t nocc;
+    int32_t turn;                       // group of 64 products that is applied next
 };
-
-// marks the segment [excl, excl + len) of the calling thread in the round of N
-// products that starts at product `base`: at its first position in the round,
-// and at every later position where a group of 64 begins, so that the segment
-// of a position is the last mark at or below it in its own group
-template <int N, typename M>
-__device__ __forceinline__ void mark_segment(M *smark, int32_t base, int32_t excl, int32_t len) {
-    if (len <= 0) return;
-    const int32_t rel = excl - base;
-    const int32_t lo = rel > 0 ? rel : 0, hi = rel + len < N ? rel + len : N;
-    if (lo >= hi) return;  // the segment has no product in this round
-    smark[lo] = (M)threadIdx.x;
-    for (int32_t ws = (lo & ~63) + 64; ws < hi; ws += 64) smark[ws] = (M)threadIdx.x;
-}
-
-// segment of the calling lane's position of the group that begins at `group`:
-// segments rise with their positions, so the last mark is a running maximum
-// over the wave (one LDS read and six register steps)
-template <typename M>
-__device__ __forceinline__ int owner_marked(const M *group) {
-    return (int)wave_incl_max((uint32_t)group[lane_id()]);
-}
-
-template <int NT, int N, typename M>
-__device__ __forceinline__ void clear_marks(M *smark) {
-    uint32_t *w = reinterpret_cast<uint32_t *>(smark);
-    for (int t = threadIdx.x; t < N * (int)sizeof(M) / 4; t += NT) w[t] = 0u;
-}
+static_assert(sizeof(HeavyWgLds<2048, 256>) <= 26880, "six workgroups per CU");
 
 // LDS only: loads in flight from global memory are not waited for
 __device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
@@ -1675,7 +1651,7 @@ __device__ __forceinline__ int32_t wg_excl_scan(int32_t v, int32_t *wsum, int32_
 }
 
 template <int T, int NT>
-__global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const TaskDev *__restrict__ tasks, int nt,
+__global__ __launch_bounds__(NT, 6) void k_num_heavy_wg(const TaskDev *__restrict__ tasks, int nt,
                                                      const Item *__restrict__ items, Counters *__restrict__ cnt,
                                                      const Window *__restrict__ wins,
                                                      const int32_t *__restrict__ order,
@@ -1685,8 +1661,7 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                                                      int32_t dense_width) {
     constexpr uint32_t kLog = __builtin_ctz(T);
     __shared__ HeavyWgLds<T, NT> L;
-    constexpr int kWaves = NT / kWave, kMarks = HeavyWgLds<T, NT>::kMarks;
-    using Id = typename HeavyWgLds<T, NT>::Id;
+    constexpr int kWaves = NT / kWave;
     const int tid = threadIdx.x, l = lane_id(), w = __builtin_amdgcn_readfirstlane(tid / kWave);
     for (int t = tid; t < T; t += NT) {
         L.key[t] = kSlotFree;
@@ -1750,7 +1725,7 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
             const uint32_t hmul = (W.c1 - W.c0) <= dense_width ? (1u << (32 - kLog)) : 0x9E3779B1u;
             int nfresh = 0;
             for (int32_t pb = a0, slot = 0; pb < a1; pb += NT, ++slot) {
-                clear_marks<NT, kMarks>(L.smark);
+                if (tid < kRound / kWave) L.starts[tid] = 0;
                 // this thread's k-slot: A entry p, B segment [s, e) inside the window
                 const int32_t p = pb + tid;
                 int32_t s = 0, e = 0;
@@ -1804,25 +1779,43 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                         }
                     }
                 }
-                int32_t total;
+                // one scan for the products and the segments before this one
+                // (a segment's columns are entries of the window, 3/4 T at most)
+                constexpr int kSegShift = 21;
+                static_assert(3 * T / 4 * NT < 1 << kSegShift, "packed counts");
+                int32_t packed;
                 const int32_t slen = e - s;
-                const int32_t excl = wg_excl_scan<NT>(slen, L.wsum, &total);
-                L.seg_d[tid] = s - excl;
-                // (the marks were cleared before the scan's barrier)
-                mark_segment<kMarks>(L.smark, 0, excl, slen);
+                const uint32_t ex = (uint32_t)wg_excl_scan<NT>(slen > 0 ? slen + (1 << kSegShift) : 0, L.wsum, &packed);
+                const int32_t total = packed & ((1 << kSegShift) - 1);
+                const int32_t excl = (int32_t)(ex & ((1u << kSegShift) - 1u));
+                if (slen > 0) {
+                    const uint32_t rank = ex >> kSegShift;
+                    L.seg_d[rank] = s - excl;
+                    L.seg_o[rank] = tid;
+                    // (cleared before the scan's barrier)
+                    if (excl < kRound) atomicOr((unsigned long long *)&L.starts[excl / kWave], 1ull << (excl % kWave));
+                }
                 __syncthreads();
                 // products flattened in A-order, in groups of 64: the waves take
                 // the groups in turn
                 const int32_t ngroups = (total + kWave - 1) / kWave;
-                for (int32_t base = 0; base < total; base += kMarks) {
+                int32_t segs = -1;  // last segment that starts before the round
+                for (int32_t base = 0; base < total; base += kRound) {
                     if (base > 0) {
                         __syncthreads();
-                        clear_marks<NT, kMarks>(L.smark);
+                        if (tid < kRound / kWave) L.starts[tid] = 0;
                         __syncthreads();
-                        mark_segment<kMarks>(L.smark, base, excl, slen);
+                        if (slen > 0 && excl >= base && excl < base + kRound)
+                            atomicOr((unsigned long long *)&L.starts[(excl - base) / kWave], 1ull << (excl % kWave));
                         __syncthreads();
                     }
-                    const int32_t gend = min(ngroups, (base + kMarks) / kWave);
+                    // lane i: the starts in the round's group i, and the last
+                    // segment that starts before it
+                    const uint64_t word = L.starts[l];
+                    const int32_t upto = wave_incl_scan((int32_t)__popcll(word));
+                    const int32_t before = segs + upto - __popcll(word);
+                    segs += read_lane(upto, kWave - 1);
+                    const int32_t gend = min(ngroups, (base + kRound) / kWave);
                     int32_t grp = base / kWave + w;
                     int32_t jn = 0;
                     double bn = 0.0, an = 0.0;
@@ -1830,10 +1823,12 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                     auto load = [&](int32_t q) {
                         if (q >= gend) return;
                         const int32_t x = q * kWave + l;
-                        const int o = owner_marked(&L.smark[q * kWave - base]);
+                        const uint64_t starts = read_lane(word, q - base / kWave);
+                        const int32_t o = read_lane(before, q - base / kWave) + rank_below(starts) +
+                                          (int32_t)__builtin_amdgcn_inverse_ballot_w64(starts);
                         if (x < total) {
                             const int32_t t = L.seg_d[o] + x;
-                            an = av[pb + o];
+                            an = av[pb + L.seg_o[o]];
                             jn = bi[t];
                             bn = bv[t];
                         }
@@ -1848,9 +1843,9 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                         bool more = act;
                         for (int probe = 0; probe < T && ballot(more); ++probe) {
                             if (more) {
-                                const uint32_t old = atomicCAS(&L.key[h], kSlotFree, off);
+                                const uint32_t old = atomicCAS(&L.key[h], kSlotFree, off | (uint32_t)tid << kOffBits);
                                 nfresh += old == kSlotFree ? 1 : 0;
-                                more = old != kSlotFree && old != off;
+                                more = old != kSlotFree && (old & kOffMask) != off;
                                 if (more) h = (h + 1) & (T - 1);
                             }
                         }
@@ -1859,13 +1854,15 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                             act = false;
                         }
                         // lanes of the group that meet in a slot: every lane
-                        // writes itself to the slot's tag, and one that reads
+                        // writes itself to the upper half of the slot's key
+                        // (the offset's bits there are the same), and one that reads
                         // another may share the slot (or another wave came in
                         // between): of lanes that share one, all but one do.
                         // turn_of: lanes of the same slot before this one
-                        if (act) L.tag[h] = (Id)tid;
+                        static_assert(NT <= 1 << (32 - kOffBits) && kOffBits >= 16, "a thread above the offset");
+                        if (act) ((volatile uint16_t *)&L.key[h])[1] = (uint16_t)(off >> 16 | (uint32_t)tid << (kOffBits - 16));
                         wave_sync();
-                        uint64_t shared = ballot(act && L.tag[h] != (Id)tid);
+                        uint64_t shared = ballot(act && ((volatile uint32_t *)L.key)[h] >> kOffBits != (uint32_t)tid);
                         int turn_of = 0, turns = 1;
                         while (shared) {
                             const int f = __ffsll((unsigned long long)shared) - 1;
@@ -1913,27 +1910,27 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
             double st_v[kStash];
             const int32_t lim = min(W.cnt, kStage);  // never write past the window
             int32_t *sidx = reinterpret_cast<int32_t *>(L.key);
+            // the thread's slots (h = tid + u NT) by column offset; the keys'
+            // space is the bitmap's from here on
+#pragma unroll
+            for (int u = 0; u < kSt; ++u) {
+                const int h = tid + u * NT;
+                const uint32_t kt = h < T ? L.key[h] : kSlotFree;
+                st_rk[u] = kt == kSlotFree ? kNone : kt & kOffMask;
+            }
+            __syncthreads();
             if (dense) {
-                // the thread's slots (h = tid + u NT) by column offset, ranked
-                // one kBmWidth-column pass at a time with a presence bitmap
-                // (it shares LDS with the step arrays, which are dead now).
-                // A direct window's slots are its column offsets, so a ballot
-                // over 64 consecutive slots is its presence word, and its one
-                // pass (width <= T < kBmWidth) needs no clearing or atomics.
+                // ranked one kBmWidth-column pass at a time with a presence
+                // bitmap.  A direct window's slots are its column offsets, so a
+                // ballot over 64 consecutive slots is its presence word, and its
+                // one pass (width <= T < kBmWidth) needs no clearing or atomics.
                 const int32_t width = W.c1 - W.c0;
                 const bool direct = width <= dense_width;
-#pragma unroll
-                for (int u = 0; u < kSt; ++u) {
-                    const int h = tid + u * NT;
-                    const uint32_t kt = h < T ? L.key[h] : kSlotFree;
-                    st_rk[u] = kt;  // (kNone is kSlotFree)
-                }
                 if (direct) {
-                    const int wsl = __builtin_amdgcn_readfirstlane(tid / kWave);  // word of slot tid in round 0
-#pragma unroll 1
+#pragma unroll
                     for (int u = 0; u < kSt; ++u) {
-                        const uint64_t m = ballot(L.key[tid + u * NT] != kSlotFree);
-                        if (l == 0) L.bm[u * (NT / kWave) + wsl] = m;
+                        const uint64_t m = ballot(st_rk[u] != kNone);
+                        if (l == 0) L.bm[u * (NT / kWave) + w] = m;
                     }
                 }
                 static_assert(T / kWave <= kBmWords, "a direct window's slots fit one pass");
@@ -2009,16 +2006,17 @@ __global__ __launch_bounds__(NT, (NT <= 256 ? 5 : 4)) void k_num_heavy_wg(const 
                 uint32_t *lkey = reinterpret_cast<uint32_t *>(L.bm);
                 uint16_t *lslot = L.wpre;
                 int32_t mine = 0;
-                for (int h = tid; h < T; h += NT) mine += (L.key[h] != kSlotFree) ? 1 : 0;
+#pragma unroll
+                for (int u = 0; u < kSt; ++u) mine += st_rk[u] != kNone ? 1 : 0;
                 int32_t tot;
                 int32_t pos = wg_excl_scan<NT>(mine, L.wsum, &tot);
                 const bool fits = tot <= kSparseH + 127;  // bound of a sparse window
                 if (fits)
-                    for (int h = tid; h < T; h += NT) {
-                        const uint32_t kt = L.key[h];
-                        if (kt == kSlotFree) continue;
-                        lkey[pos] = kt;
-                        lslot[pos] = (uint16_t)h;
+#pragma unroll
+                    for (int u = 0; u < kSt; ++u) {
+                        if (st_rk[u] == kNone) continue;
+                        lkey[pos] = st_rk[u];
+                        lslot[pos] = (uint16_t)(tid + u * NT);
                         ++pos;
                     }
                 __syncthreads();
@@ -2244,8 +2242,8 @@ void mul_read_counts(tr_ctx *ctx, MulPlan &pl) { read_array(ctx, &pl.h, pl.cnt, 
 
 // Multiplications that one heavy item should hold at most.  A product with few
 // heavy rows would leave the chip to the few items that tune.item_windows
-// windows make of them: about kItemsPerSlot items for each of the five
-// workgroups a CU holds, but no item below kMinItemFlops.  (8, 32, 64 and 128
+// windows make of them: about kItemsPerSlot items for each of five workgroups
+// a CU, but no item below kMinItemFlops.  (8, 32, 64 and 128
 // per slot: R-MAT s17 14.43, 13.74, 14.06, 14.44 ms; 16 served requests 21.9,
 // 20.8, 21.2, 21.7 ms; R-MAT s19, whose items the window count cuts, within
 // 1%.  A minimum of 8192 costs the R-MAT of 15013 vertices 3%.)
