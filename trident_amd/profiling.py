@@ -7,7 +7,7 @@ queue -- the measure of the accumulation overlap of a stage loop, where the
 add of stage s runs on the accumulation thread's stream while the main
 thread multiplies stage s + 1.
 
-    python -m trident_amd.profiling overlap TRACE.csv --a k_add_ --b k_num_,k_sym_,k_row_flops
+    python -m trident_amd.profiling overlap TRACE.csv --a k_add_ --b k_num_,k_sym_,k_check_,k_classify
 """
 from __future__ import annotations
 
@@ -94,7 +94,7 @@ def main(argv=None) -> int:
     o = sub.add_parser("overlap", help="time group-A kernels ran alongside group-B kernels on other queues")
     o.add_argument("trace", help="kernel_trace.csv or a rocprofv3 output directory")
     o.add_argument("--a", default="k_add_", help="comma list of name fragments of group A")
-    o.add_argument("--b", default="k_num_,k_sym_,k_row_flops", help="comma list of name fragments of group B")
+    o.add_argument("--b", default="k_num_,k_sym_,k_check_,k_classify", help="comma list of name fragments of group B")
     args = ap.parse_args(argv)
     res = overlap(read_trace(args.trace), args.a.split(","), args.b.split(","))
     for k, v in res.items():
