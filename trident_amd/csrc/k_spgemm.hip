@@ -1858,19 +1858,26 @@ __global__ __launch_bounds__(NT, 6) void k_num_heavy_wg(const TaskDev *__restric
                         // (the offset's bits there are the same), and one that reads
                         // another may share the slot (or another wave came in
                         // between): of lanes that share one, all but one do.
-                        // turn_of: lanes of the same slot before this one
+                        // turn_of: lanes of the same slot before this one.
+                        // A round takes the slots of the lowest and the
+                        // highest such lane (one slot a round: product of
+                        // R-MAT s17 9.54 ms, two 9.15, the lowest two, three
+                        // or four lanes 9.31, 9.46, 9.50)
                         static_assert(NT <= 1 << (32 - kOffBits) && kOffBits >= 16, "a thread above the offset");
                         if (act) ((volatile uint16_t *)&L.key[h])[1] = (uint16_t)(off >> 16 | (uint32_t)tid << (kOffBits - 16));
                         wave_sync();
                         uint64_t shared = ballot(act && ((volatile uint32_t *)L.key)[h] >> kOffBits != (uint32_t)tid);
                         int turn_of = 0, turns = 1;
+                        const uint32_t hm = act ? h : ~0u;
                         while (shared) {
-                            const int f = __ffsll((unsigned long long)shared) - 1;
-                            const bool same = act && h == read_lane(h, f);
-                            const uint64_t m = ballot(same);
+                            const uint32_t hf = read_lane(hm, __ffsll((unsigned long long)shared) - 1);
+                            const uint32_t hf2 = read_lane(hm, 63 - __clzll((long long)shared));
+                            const bool same = hm == hf, same2 = hm == hf2;
+                            const uint64_t m = ballot(same), m2 = ballot(same2);
                             if (same) turn_of = rank_below(m);
-                            turns = max(turns, __popcll(m));
-                            shared &= ~m;
+                            if (same2) turn_of = rank_below(m2);
+                            turns = max(turns, max(__popcll(m), __popcll(m2)));
+                            shared &= ~(m | m2);
                         }
                         load(grp + kWaves);
                         // wait for the groups before this one, which other waves hold
