@@ -85,3 +85,28 @@ def test_flops_of_rows_over_units(ctx, shape):
     assert np.array_equal(h.ptr, p) and np.array_equal(h.idx, i) and np.array_equal(h.val, v)
     for x in (c, da, db):
         x.free()
+
+
+def _status_by_definition(m):
+    n, nnz, p = m.nrows, m.nnz, m.ptr.astype(np.int64)
+    bad = (p < 0).any() or (p > nnz).any() or p[0] != 0 or p[-1] != nnz or (np.diff(p) < 0).any()
+    start = {v for i, v in enumerate(p[:-1]) if 0 <= v < p[i + 1] and (i > 0 or v == 0)}
+    order = any(m.idx[q] <= m.idx[q - 1] and q not in start for q in range(1, nnz))
+    return int(bad) | 2 * bool((m.idx < 0).any() or (m.idx >= m.ncols).any()) | 4 * order
+
+
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("fault", ["short", "long", "descent", "negative", "first"])
+def test_entries_under_malformed_pointers(ctx, shape, fault):
+    """A tile's entries are judged all the same where its pointers are wrong."""
+    m = _rows(SHAPES[shape], 1 << 20)
+    at, v = {"short": (-1, m.nnz // 2), "long": (-1, m.nnz + 5), "descent": (len(m.ptr) // 2, 1),
+             "negative": (len(m.ptr) // 2, -7), "first": (0, 2)}[fault]
+    q = m.ptr.copy()
+    q[at] = v
+    for place, value in ((None, 0), (m.nnz - 1, 1 << 20), (m.nnz - 1, -1), (m.nnz - 2, 1 << 19)):
+        c = m.idx.copy()
+        if place is not None:
+            c[place] = value
+        t = Csr(m.nrows, m.ncols, q, c, m.val)
+        assert _status(ctx, t) == _status_by_definition(t), (place, value)

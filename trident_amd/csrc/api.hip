@@ -691,7 +691,10 @@ int tr_csx_validate(tr_ctx_t ctx, const tr_csx_t *M, int32_t *status) {
     return guarded(ctx, [&] {
         check_csx(M, "M");
         TR_REQUIRE(status != nullptr, "tr_csx_validate: null status");
-        check_tiles(ctx, &M, 1, status);
+        int32_t st = 0;
+        check_tiles(ctx, &M, 1, &st);
+        if (st & 1) st = 1 | check_positions(ctx, M);
+        *status = st;
     });
 }
 

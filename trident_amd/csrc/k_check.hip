@@ -135,6 +135,29 @@ __global__ __launch_bounds__(kUnitThreads) void k_check_entries(const CheckJob *
     if (order) report(findings, t, 2);
 }
 
+// Units need monotone pointers.  The entries of a tile whose pointers are not
+// well formed are checked by position: a segment starts where a sound,
+// non-empty pair of pointers says so.
+__global__ __launch_bounds__(256) void k_mark_starts(const CheckJob J, uint32_t *__restrict__ starts) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= J.n) return;
+    const int32_t v = J.ptr[i];
+    if (v < 0 || (int64_t)v >= J.cap || (i == 0 && v != 0) || J.ptr[i + 1] <= v) return;
+    atomicOr(&starts[v >> 5], 1u << (v & 31));
+}
+
+__global__ __launch_bounds__(256) void k_check_positions(const CheckJob J, const uint32_t *__restrict__ starts,
+                                                         uint8_t *__restrict__ findings) {
+    bool range = false, order = false;
+    for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < J.cap; p += (int64_t)gridDim.x * 256) {
+        const int32_t c = J.idx[p];
+        range |= c < 0 || c >= J.other;
+        order |= p > 0 && !((starts[p >> 5] >> (p & 31)) & 1u) && c <= J.idx[p - 1];
+    }
+    if (range) report(findings, 0, 1);
+    if (order) report(findings, 0, 2);
+}
+
 }  // namespace
 
 CheckJob check_job(const tr_csx_t *m) {
@@ -215,6 +238,22 @@ void check_tiles(tr_ctx *ctx, const tr_csx_t *const *m, int n, int32_t *status) 
     check_begin(ctx, m, n);
     TR_HIP(hipStreamSynchronize(ctx->stream));
     check_result(ctx, status, n);
+}
+
+int32_t check_positions(tr_ctx *ctx, const tr_csx_t *m) {
+    const CheckJob j = check_job(m);
+    const int64_t words = j.cap / 32 + 1;
+    uint32_t *starts = (uint32_t *)scratch(ctx, S_MISC2, sizeof(uint32_t) * (size_t)words);
+    check_open(ctx);
+    ctx->check_twin = false;
+    launch_fill_i32(ctx, (int32_t *)starts, 0, words);
+    TR_LAUNCH(ctx, "mark_starts", k_mark_starts, div_up((uint64_t)j.n, 256), 256, 0, j, starts);
+    TR_LAUNCH(ctx, "check_positions", k_check_positions, (uint32_t)std::min<int64_t>((j.cap + 255) / 256, 16384), 256,
+              0, j, (const uint32_t *)starts, ctx->status);
+    TR_HIP(hipStreamSynchronize(ctx->stream));
+    int32_t status = 0;
+    check_result(ctx, &status, 1);
+    return status;
 }
 
 }  // namespace tr

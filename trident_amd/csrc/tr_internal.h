@@ -234,6 +234,7 @@ void check_begin(tr_ctx *ctx, const tr_csx_t *const *m, int n);
 void check_pointers(tr_ctx *ctx, const tr_csx_t *const *m, int n);  // the pointers alone, every tile
 void check_result(tr_ctx *ctx, int32_t *status, int n);
 void check_tiles(tr_ctx *ctx, const tr_csx_t *const *m, int n, int32_t *status);  // both, with the wait
+int32_t check_positions(tr_ctx *ctx, const tr_csx_t *m);  // bits 2 and 4 where the pointers are malformed
 
 // k_transpose.hip
 void launch_transpose(tr_ctx *ctx, const tr_csx_t *m, tr_csx_t *out);
