@@ -91,3 +91,25 @@ def test_short_rows(ctx, nrows, span):
         rows_a.append(np.sort(row))
     pick = rng.integers(0, 600, nrows)
     _check(ctx, _csr([rows_a[i] for i in pick], nb, rng), _csr(rows_b, 7 * span + 1, rng))
+
+
+@pytest.mark.parametrize("repeats", [1, 3000])
+@pytest.mark.parametrize("ncols", [300, (1 << 22) + 1])
+def test_classes_together(ctx, repeats, ncols):
+    """Every light class in one product: few rows share a launch, many do not."""
+    rng = np.random.default_rng(repeats + ncols)
+    cols = np.sort(rng.choice(ncols, 200, replace=False)) if ncols > 1000 else np.arange(50, 250)
+    rows_b = [np.sort(rng.choice(cols, n, replace=False)) for n in (1, 2, 7, 31, 64, 150)]
+    sizes = [1, 31, 32, 33, 64, 65, 128, 129, 256, 257, 512, 513, 1024]
+    spread = [r for _ in range(120) for r in rows_b]  # B's rows again and again
+    rows_a = []
+    for n in sizes:
+        row, i = [], 0
+        while n > 0:
+            if len(spread[i]) <= n:
+                row.append(i)
+                n -= len(spread[i])
+            i += 1
+        rows_a.append(row)
+    a, b = _csr(rows_a * repeats, len(spread), rng), _csr(spread, ncols, rng)
+    _check(ctx, a, b)

@@ -425,17 +425,17 @@ __global__ __launch_bounds__(kClassThreads) void k_classify(const TaskDev *__res
 // One wave per row, rows taken from the class list (grid-stride, count read
 // on the device so the launch can be replayed from a graph).
 template <int T>
-__global__ __launch_bounds__(256) void k_sym_light(const TaskDev *__restrict__ tasks, int nt,
-                                                   const int32_t *__restrict__ rows, const Counters *__restrict__ cnt,
-                                                   int cls, int64_t *__restrict__ rownnz) {
-    __shared__ int32_t tabs[4][T];
+__device__ __forceinline__ void sym_light_rows(int32_t *lds, int32_t block, int32_t blocks,
+                                               const TaskDev *__restrict__ tasks, int nt,
+                                               const int32_t *__restrict__ rows, const Counters *__restrict__ cnt,
+                                               int cls, int64_t *__restrict__ rownnz) {
     constexpr uint32_t kLog = __builtin_ctz(T);
     // (marking the row wave-uniform here moves its values to scalar
     // registers, 101 SGPRs: 7 waves per SIMD instead of 8, and slower)
     const int w = threadIdx.x / kWave, l = lane_id();
-    int32_t *tab = tabs[w];
+    int32_t *tab = lds + w * T;
     const int32_t nrows = cnt->cls[cls];
-    for (int32_t li = blockIdx.x * 4 + w; li < nrows; li += gridDim.x * 4) {
+    for (int32_t li = block * 4 + w; li < nrows; li += blocks * 4) {
         const int32_t g = rows[li];
         const TaskDev &TK = tasks[task_of(tasks, nt, g)];
         const int32_t r = g - TK.row_base;
@@ -495,6 +495,45 @@ __global__ __launch_bounds__(256) void k_sym_light(const TaskDev *__restrict__ t
         if (l == 0) rownnz[g] = cntv;
         wave_sync();
     }
+}
+
+template <int T>
+__global__ __launch_bounds__(256) void k_sym_light(const TaskDev *__restrict__ tasks, int nt,
+                                                   const int32_t *__restrict__ rows, const Counters *__restrict__ cnt,
+                                                   int cls, int64_t *__restrict__ rownnz) {
+    __shared__ int32_t tabs[4 * T];
+    sym_light_rows<T>(tabs, blockIdx.x, gridDim.x, tasks, nt, rows, cnt, cls, rownnz);
+}
+
+// Workgroups of the light classes in one launch: class c has [end[c + 1],
+// end[c]), the longest rows first.
+struct LightBlocks {
+    int32_t end[kNumLight + 1];
+};
+
+// class of this workgroup (block-uniform)
+__device__ __forceinline__ int light_block_class(const LightBlocks &lb) {
+    int c = kNumLight - 1;
+    while (c > 0 && (int32_t)blockIdx.x >= lb.end[c]) --c;
+    return c;
+}
+
+// All light classes at once, where they are few rows (light_blocks); 32 KiB of
+// LDS, five workgroups a CU
+__global__ __launch_bounds__(256) void k_sym_light_all(const TaskDev *__restrict__ tasks, int nt,
+                                                       const int32_t *__restrict__ lists, int32_t rows_total,
+                                                       const Counters *__restrict__ cnt, const LightBlocks lb,
+                                                       int64_t *__restrict__ rownnz) {
+    __shared__ int32_t tabs[4 * 2048];
+    const int c = light_block_class(lb);
+    const int32_t block = (int32_t)blockIdx.x - lb.end[c + 1], blocks = lb.end[c] - lb.end[c + 1];
+    const int32_t *rows = lists + (int64_t)c * rows_total;
+    if (c == 5) sym_light_rows<2048>(tabs, block, blocks, tasks, nt, rows, cnt, c, rownnz);
+    else if (c == 4) sym_light_rows<1024>(tabs, block, blocks, tasks, nt, rows, cnt, c, rownnz);
+    else if (c == 3) sym_light_rows<512>(tabs, block, blocks, tasks, nt, rows, cnt, c, rownnz);
+    else if (c == 2) sym_light_rows<256>(tabs, block, blocks, tasks, nt, rows, cnt, c, rownnz);
+    else if (c == 1) sym_light_rows<128>(tabs, block, blocks, tasks, nt, rows, cnt, c, rownnz);
+    else sym_light_rows<64>(tabs, block, blocks, tasks, nt, rows, cnt, c, rownnz);
 }
 
 // ---------------------------------------------------------------- short rows
@@ -1402,21 +1441,21 @@ struct SortLds {
 };
 
 template <int NT, int WPB, int P, typename K>
-__global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict__ tasks, int nt,
-                                                      const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
-                                                      int cls, int32_t lo, const int64_t *__restrict__ rowptr,
-                                                      const Panel *__restrict__ panels, int npanels) {
+__device__ __forceinline__ void num_sort_rows(SortLds<NT, P, K> *lds_s, int32_t block, int32_t blocks,
+                                              const TaskDev *__restrict__ tasks, int nt,
+                                              const int32_t *__restrict__ rows, Counters *__restrict__ cnt, int cls,
+                                              int32_t lo, const int64_t *__restrict__ rowptr,
+                                              const Panel *__restrict__ panels, int npanels) {
     static_assert(NT > kWave ? WPB == 1 : NT == kWave, "a row's threads are a workgroup or a wave of it");
     constexpr int kMax = NT * P, kWaves = NT / kWave;
     static_assert(kMax <= 1 << kSortIdBits, "positions fit their key bits");
     constexpr K kIdMask = ((K)1 << kSortIdBits) - 1;
-    __shared__ SortLds<NT, P, K> lds_s[WPB];
     const int sub = NT > kWave ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // row of the workgroup
     const int t = threadIdx.x % NT, l = lane_id();
     const int w = NT > kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;    // wave of the row
     SortLds<NT, P, K> &L = lds_s[sub];
     const int32_t nrows = cnt->cls[cls];
-    for (int32_t li = blockIdx.x * WPB + sub; li < nrows; li += gridDim.x * WPB) {
+    for (int32_t li = block * WPB + sub; li < nrows; li += blocks * WPB) {
         const int32_t g = __builtin_amdgcn_readfirstlane(rows[li]);
         const int64_t rs = rowptr[g];
         const int32_t expect = (int32_t)(rowptr[g + 1] - rs);
@@ -1566,6 +1605,41 @@ __global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict_
         }
         row_sync<NT>();  // the next row rewrites the arrays
     }
+}
+
+template <int NT, int WPB, int P, typename K>
+__global__ __launch_bounds__(NT *WPB) void k_num_sort(const TaskDev *__restrict__ tasks, int nt,
+                                                      const int32_t *__restrict__ rows, Counters *__restrict__ cnt,
+                                                      int cls, int32_t lo, const int64_t *__restrict__ rowptr,
+                                                      const Panel *__restrict__ panels, int npanels) {
+    __shared__ SortLds<NT, P, K> lds_s[WPB];
+    num_sort_rows<NT, WPB, P, K>(lds_s, blockIdx.x, gridDim.x, tasks, nt, rows, cnt, cls, lo, rowptr, panels, npanels);
+}
+
+// All light classes at once, where they are few rows (light_blocks); a
+// workgroup is 256 threads in every class (a row of 257 to 512 products takes
+// two a thread instead of four of half as many threads).
+template <typename K>
+__global__ __launch_bounds__(256) void k_num_sort_all(const TaskDev *__restrict__ tasks, int nt,
+                                                      const int32_t *__restrict__ lists, int32_t rows_total,
+                                                      Counters *__restrict__ cnt, const LightBlocks lb,
+                                                      const int64_t *__restrict__ rowptr,
+                                                      const Panel *__restrict__ panels, int npanels) {
+    __shared__ union {
+        SortLds<64, 1, K> a[4];
+        SortLds<64, 2, K> b[4];
+        SortLds<64, 4, K> c[4];
+        SortLds<256, 2, K> d[1];
+        SortLds<256, 4, K> e[1];
+    } L;
+    const int c = light_block_class(lb);
+    const int32_t block = (int32_t)blockIdx.x - lb.end[c + 1], blocks = lb.end[c] - lb.end[c + 1];
+    const int32_t *rows = lists + (int64_t)c * rows_total;
+    if (c == 5) num_sort_rows<256, 1, 4, K>(L.e, block, blocks, tasks, nt, rows, cnt, c, 0, rowptr, panels, npanels);
+    else if (c == 4) num_sort_rows<256, 1, 2, K>(L.d, block, blocks, tasks, nt, rows, cnt, c, 0, rowptr, panels, npanels);
+    else if (c == 3) num_sort_rows<64, 4, 4, K>(L.c, block, blocks, tasks, nt, rows, cnt, c, 0, rowptr, panels, npanels);
+    else if (c == 2) num_sort_rows<64, 4, 2, K>(L.b, block, blocks, tasks, nt, rows, cnt, c, 0, rowptr, panels, npanels);
+    else num_sort_rows<64, 4, 1, K>(L.a, block, blocks, tasks, nt, rows, cnt, c, 0, rowptr, panels, npanels);
 }
 
 // ---------------------------------------------------------------- numeric, heavy rows (workgroup)
@@ -2115,6 +2189,30 @@ uint32_t cap_grid(int64_t need, int64_t cap) {
 }
 
 
+// Workgroups of the light classes if they go into one launch: more than one
+// class has rows, and together they are at most kLightPerCu workgroups a CU.
+// `wide`: classes 4 and 5 take a workgroup a row.
+// A class of few rows leaves most CUs idle for the whole chain of its longest
+// row, so up to six such launches wait for each other (5 to 22 us each); in one
+// they overlap.  Every workgroup then holds the LDS of the largest class, which
+// costs occupancy once the rows fill the chip several times.  (Separate
+// launches, then one launch up to 4, 16 and 32 a CU: tile accumulate of R-MAT
+// s16 347, 339, 270, 271 us; Galerkin 19^3 345, 279, 261, 264 us; product of
+// 15013 vertices 568, 561, 493, 497 us.)
+constexpr int kLightPerCu = 16;
+bool light_blocks(tr_ctx *ctx, const MulPlan &pl, bool wide, LightBlocks &lb) {
+    int64_t all = 0;
+    int used = 0;
+    lb.end[kNumLight] = 0;
+    for (int c = kNumLight - 1; c >= 0; --c) {
+        const int64_t n = pl.h.cls[c];
+        all += wide && c >= 4 ? n : (n + 3) / 4;
+        used += n > 0 ? 1 : 0;
+        lb.end[c] = (int32_t)std::min<int64_t>(all, INT32_MAX);
+    }
+    return used > 1 && all <= (int64_t)ctx->cu_count * kLightPerCu;
+}
+
 template <int T>
 void launch_sym_light(tr_ctx *ctx, MulPlan &pl, int c) {
     const int32_t n = pl.h.cls[c];
@@ -2270,12 +2368,18 @@ void launch_sym_heavy(tr_ctx *ctx, MulPlan &pl, int cls, int cls2, int per_cu, b
 }
 
 void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool capture) {
-    if (pl.h.cls[0]) launch_sym_light<64>(ctx, pl, 0);
-    if (pl.h.cls[1]) launch_sym_light<128>(ctx, pl, 1);
-    if (pl.h.cls[2]) launch_sym_light<256>(ctx, pl, 2);
-    if (pl.h.cls[3]) launch_sym_light<512>(ctx, pl, 3);
-    if (pl.h.cls[4]) launch_sym_light<1024>(ctx, pl, 4);
-    if (pl.h.cls[5]) launch_sym_light<2048>(ctx, pl, 5);
+    LightBlocks lb;
+    if (light_blocks(ctx, pl, false, lb)) {
+        TR_LAUNCH(ctx, "sym_light", k_sym_light_all, (uint32_t)lb.end[0], 256, 0, pl.d_tasks, pl.nt, pl.lists,
+                  pl.rows_total, pl.cnt, lb, pl.rownnz);
+    } else {
+        if (pl.h.cls[0]) launch_sym_light<64>(ctx, pl, 0);
+        if (pl.h.cls[1]) launch_sym_light<128>(ctx, pl, 1);
+        if (pl.h.cls[2]) launch_sym_light<256>(ctx, pl, 2);
+        if (pl.h.cls[3]) launch_sym_light<512>(ctx, pl, 3);
+        if (pl.h.cls[4]) launch_sym_light<1024>(ctx, pl, 4);
+        if (pl.h.cls[5]) launch_sym_light<2048>(ctx, pl, 5);
+    }
     if (pl.h.cls[kShortClass])
         TR_LAUNCH(ctx, "sym_light", k_sym_short,
                   cap_grid(div_up((uint64_t)pl.h.cls[kShortClass], 4 * kShortRows), (int64_t)ctx->cu_count * 32), 256, 0,
@@ -2394,26 +2498,40 @@ void launch_num_sort_as(tr_ctx *ctx, MulPlan &pl, int c, int32_t lo, Panel *pane
               panels, np);
 }
 
-// class c of rows of up to NT * P products, those of more than lo entries; (column, position) keys of 32 bits
-// where every column fits
+// (column, position) keys of 32 bits hold every column
+bool narrow_keys(const MulPlan &pl) {
+    int32_t max_n = 0;
+    for (const TaskDev &t : pl.h_tasks) max_n = std::max(max_n, t.n);
+    return max_n <= 1 << (32 - kSortIdBits);
+}
+
+// class c of rows of up to NT * P products, those of more than lo entries
 template <int NT, int P>
 void launch_num_sort(tr_ctx *ctx, MulPlan &pl, int c, int32_t lo, Panel *panels, int np) {
     if (!pl.h.cls[c]) return;
-    int32_t max_n = 0;
-    for (const TaskDev &t : pl.h_tasks) max_n = std::max(max_n, t.n);
-    if (max_n <= 1 << (32 - kSortIdBits)) launch_num_sort_as<NT, P, uint32_t>(ctx, pl, c, lo, panels, np);
+    if (narrow_keys(pl)) launch_num_sort_as<NT, P, uint32_t>(ctx, pl, c, lo, panels, np);
     else launch_num_sort_as<NT, P, uint64_t>(ctx, pl, c, lo, panels, np);
 }
 
 }  // namespace
 
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *dp, int np) {
-    launch_num_sort<64, 1>(ctx, pl, 0, 0, dp, np);
-    launch_num_sort<64, 1>(ctx, pl, 1, 0, dp, np);
-    launch_num_sort<64, 2>(ctx, pl, 2, 0, dp, np);
-    launch_num_sort<64, 4>(ctx, pl, 3, 0, dp, np);
-    launch_num_sort<128, 4>(ctx, pl, 4, 0, dp, np);
-    launch_num_sort<256, 4>(ctx, pl, 5, 0, dp, np);
+    LightBlocks lb;
+    if (light_blocks(ctx, pl, true, lb)) {
+        if (narrow_keys(pl))
+            TR_LAUNCH(ctx, "num_light", k_num_sort_all<uint32_t>, (uint32_t)lb.end[0], 256, 0, pl.d_tasks, pl.nt,
+                      pl.lists, pl.rows_total, pl.cnt, lb, pl.rowptr, dp, np);
+        else
+            TR_LAUNCH(ctx, "num_light", k_num_sort_all<uint64_t>, (uint32_t)lb.end[0], 256, 0, pl.d_tasks, pl.nt,
+                      pl.lists, pl.rows_total, pl.cnt, lb, pl.rowptr, dp, np);
+    } else {
+        launch_num_sort<64, 1>(ctx, pl, 0, 0, dp, np);
+        launch_num_sort<64, 1>(ctx, pl, 1, 0, dp, np);
+        launch_num_sort<64, 2>(ctx, pl, 2, 0, dp, np);
+        launch_num_sort<64, 4>(ctx, pl, 3, 0, dp, np);
+        launch_num_sort<128, 4>(ctx, pl, 4, 0, dp, np);
+        launch_num_sort<256, 4>(ctx, pl, 5, 0, dp, np);
+    }
     // short rows of more entries than their table takes are sorted
     if (pl.h.short_rows[0])
         TR_LAUNCH(ctx, "num_light", k_num_short,
