@@ -1009,6 +1009,14 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
     }
 }
 
+// Items of the work list.  A list that would not fit (a batch's replay on
+// operands with another sparsity pattern than the planned one) holds none:
+// its count runs on past its capacity, and refused rows leave gaps that were
+// never written.
+__device__ __forceinline__ int32_t listed_items(const Counters *__restrict__ cnt) {
+    return (cnt->overflow & 1) ? 0 : cnt->items;
+}
+
 // per item: cursor slots it needs (multi-window items of rows longer than
 // reg_max entries; shorter rows keep their cursors in registers)
 __global__ void k_item_cursor_len(const Item *__restrict__ items, const Counters *__restrict__ cnt,
@@ -1017,7 +1025,7 @@ __global__ void k_item_cursor_len(const Item *__restrict__ items, const Counters
     const int32_t it = blockIdx.x * blockDim.x + threadIdx.x;
     if (it >= cap) return;
     int32_t v = 0;
-    if (it < cnt->items) {
+    if (it < listed_items(cnt)) {
         const Item I = items[it];
         if (I.wend - I.wbeg > 1) {
             const TaskDev &TK = tasks[task_of(tasks, nt, I.row)];
@@ -1055,7 +1063,7 @@ __global__ __launch_bounds__(256) void k_item_hist(const Item *__restrict__ item
     __shared__ int32_t h[kOrderBuckets];
     for (int t = threadIdx.x; t < kOrderBuckets; t += 256) h[t] = 0;
     __syncthreads();
-    const int32_t n = cnt->items;
+    const int32_t n = listed_items(cnt);
     for (int32_t it = blockIdx.x * 256 + threadIdx.x; it < n; it += gridDim.x * 256)
         atomicAdd(&h[item_bucket(items, wins, it, shift)], 1);
     __syncthreads();
@@ -1095,7 +1103,7 @@ __global__ __launch_bounds__(256) void k_item_scatter(const Item *__restrict__ i
                                                       int32_t *__restrict__ order) {
     __shared__ int32_t h[kOrderBuckets];
     __shared__ unsigned long long base[kOrderBuckets];
-    const int32_t n = cnt->items;
+    const int32_t n = listed_items(cnt);
     for (int32_t it0 = blockIdx.x * 256; it0 < n; it0 += gridDim.x * 256) {
         for (int t = threadIdx.x; t < kOrderBuckets; t += 256) h[t] = 0;
         __syncthreads();
