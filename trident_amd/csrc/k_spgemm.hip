@@ -961,13 +961,7 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
 #pragma unroll
             for (int u = 0; u < kPerThread; ++u)
                 if (flags & (1 << u)) first_lds[rk++] = tid * kPerThread + u;
-            // rows of more than kLongRow entries get a quarter of the
-            // windows per item: their items are the longest, and the last
-            // of them would otherwise run alone at the end of the numeric
-            // and no item holds much more than item_flops multiplications
-            // (taking the row's as spread evenly over its windows)
-            const int32_t iw = max(1, (int32_t)min<int64_t>((a1 - a0 > kLongRow) ? item_windows / 4 : item_windows,
-                                                            item_flops * nwin / flops[g]));
+            const int32_t iw = heavy_item_windows(item_windows, a1 - a0, item_flops, flops[g], heavy_passes(ncols, PB), nwin);
             if (tid == 0) {
                 const int32_t nitems = (nwin + iw - 1) / iw;
                 const int32_t wb = atomicAdd(&cnt->windows, nwin);
@@ -2353,17 +2347,8 @@ void mul_checked(tr_ctx *ctx) {
 
 void mul_read_counts(tr_ctx *ctx, MulPlan &pl) { read_array(ctx, &pl.h, pl.cnt, sizeof(Counters)); }
 
-// Multiplications that one heavy item should hold at most.  A product with few
-// heavy rows would leave the chip to the few items that tune.item_windows
-// windows make of them: about kItemsPerSlot items for each of five workgroups
-// a CU, but no item below kMinItemFlops.  (8, 32, 64 and 128
-// per slot: R-MAT s17 14.43, 13.74, 14.06, 14.44 ms; 16 served requests 21.9,
-// 20.8, 21.2, 21.7 ms; R-MAT s19, whose items the window count cuts, within
-// 1%.  A minimum of 8192 costs the R-MAT of 15013 vertices 3%.)
-constexpr int kItemsPerSlot = 32;
-constexpr int64_t kMinItemFlops = 2048;
 int64_t item_flops(const tr_ctx *ctx, const MulPlan &pl) {
-    return std::max<int64_t>(kMinItemFlops, (int64_t)pl.h.heavy_flops / ((int64_t)ctx->cu_count * 5 * kItemsPerSlot));
+    return heavy_item_flops((int64_t)pl.h.heavy_flops, ctx->cu_count);
 }
 
 template <int PB, int NTH>
@@ -2397,19 +2382,13 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
         int32_t max_n = 0;
         for (auto &t : pl.h_tasks) max_n = std::max(max_n, t.n);
         if (emit && !capture) {
-            // windows per pass <= ceil(pass_nnz / H) + width splits (mid rows use the shorter pass)
-            const int64_t passes = ((int64_t)max_n + (1 << kMidPassBits) - 1) >> kMidPassBits;
-            const int64_t wsplits = (int64_t)max_n / kWinMaxWidth + 1;
-            const int64_t q = std::min<int64_t>(pl.tune.window_entries, kSparseH);
-            const int64_t wcap = (int64_t)(pl.h.heavy_flops / q) + (int64_t)nh * (2 * passes + wsplits) + 16;
-            // items: by the window count, or 2 for each item_flops multiplications
-            const int64_t icap = wcap / std::max(1, pl.tune.item_windows / 4) +
-                                 2 * ((int64_t)pl.h.heavy_flops / item_flops(ctx, pl)) + (int64_t)nh * passes + 16;
-            TR_REQUIRE(wcap < INT32_MAX && icap < INT32_MAX, "spgemm: heavy work list exceeds int32 capacity");
-            pl.win_cap = (int32_t)wcap;
-            pl.item_cap = (int32_t)icap;
-            pl.wins = (Window *)ws.get(S_WINDOWS, sizeof(Window) * (size_t)wcap);
-            pl.items = (Item *)ws.get(S_ITEMS, sizeof(Item) * (size_t)icap);
+            const HeavyLists cap = heavy_lists((int64_t)pl.h.heavy_flops, nh, max_n, pl.tune.window_entries,
+                                               pl.tune.item_windows, item_flops(ctx, pl));
+            TR_REQUIRE(cap.windows < INT32_MAX && cap.items < INT32_MAX, "spgemm: heavy work list exceeds int32 capacity");
+            pl.win_cap = (int32_t)cap.windows;
+            pl.item_cap = (int32_t)cap.items;
+            pl.wins = (Window *)ws.get(S_WINDOWS, sizeof(Window) * (size_t)cap.windows);
+            pl.items = (Item *)ws.get(S_ITEMS, sizeof(Item) * (size_t)cap.items);
         }
         // The bitmap covers 2^PB columns per pass and its LDS bounds the
         // resident workgroups: 2^20 bits (128 KiB) hold one per CU, 2^19 two,

@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "heavy_items.h"
 
 namespace tr {
 
@@ -24,21 +25,10 @@ constexpr int kShortMaxNnz = 32;              // and its entries, for the table 
 // chip idle (Galerkin n^3, short against sorted: 28 392 / 388 us, 32 385 / 394,
 // 48 509 / 568, 64 874 / 1031)
 constexpr int32_t kShortMinRows = 32768;
-constexpr int kMidMaxF = 16384;
-constexpr int kMidPassBits = 19;            // mid rows: at most 2^19-column passes, two blocks per CU
 constexpr int kMidThreads = 512;
-constexpr int kPassBits = 20;      // heavy bitmap covers 2^20 columns per pass
-constexpr int kFineShift = 7;      // fine block = 128 columns
-constexpr int kWinLog = 19;                                // window width cap: 2^19 columns
-constexpr int kWinMaxWidth = 1 << kWinLog;                 // (column offsets stay below 2^20)
-constexpr int kWidthShift = kWinLog - kFineShift;          // fine blocks per width quantum
 constexpr int kBmWidth = 32768;                            // columns ranked per presence-bitmap pass
 constexpr int kBmWords = kBmWidth / 64;                    // presence words per pass
-static_assert(kWinMaxWidth <= (1 << 20) && kPassBits <= 20, "window column offsets fit 20 bits");
-constexpr int kSparseAvg = 192;    // a pass with <= this many entries per width quantum is sparse
-constexpr int kSparseH = 256;      // sparse windows: count quantum (<= kSparseH + 127 entries, any width)
 constexpr int kHeavyThreads = 1024;  // symbolic heavy block
-constexpr int kLongRow = 2048;       // heavy rows with more A entries take shorter items
 constexpr int kCompactMax = 128;     // one-pass heavy rows with <= this many entries take the light numeric
 static_assert(kCompactMax * 2 <= (64 << 2), "compact rows fit the light tables of classes 0..2");
 
