@@ -270,17 +270,63 @@ struct Temp {
     Temp &operator=(const Temp &) = delete;
 };
 
-template <bool kFirst, bool kLast>
-void radix_pass(tr_ctx *ctx, const Pass &a, int64_t *off) {
-    TR_LAUNCH(ctx, "transpose_count", k_radix_count<kFirst>, tile_blocks(a.ntiles), kThreads, 0, a);
-    scan::launch(ctx, scan::ArrayIn<int32_t>{a.hist}, off, (int64_t)a.ntiles << a.nbits, nullptr);
-    TR_LAUNCH(ctx, "transpose_scatter", (k_radix_scatter<kFirst, kLast>), tile_blocks(a.ntiles), kThreads, 0, a);
-}
-
 int bits_for(int32_t n) {
     int b = 1;
     while (b < 31 && ((int64_t)1 << b) < n) ++b;
     return b;
+}
+
+template <bool kFirst>
+void count_digits(tr_ctx *ctx, const Pass &a, int64_t *off) {
+    TR_LAUNCH(ctx, "transpose_count", k_radix_count<kFirst>, tile_blocks(a.ntiles), kThreads, 0, a);
+    scan::launch(ctx, scan::ArrayIn<int32_t>{a.hist}, off, (int64_t)a.ntiles << a.nbits, nullptr);
+}
+
+template <bool kFirst, bool kLast>
+void scatter(tr_ctx *ctx, const Pass &a) {
+    TR_LAUNCH(ctx, "transpose_scatter", (k_radix_scatter<kFirst, kLast>), tile_blocks(a.ntiles), kThreads, 0, a);
+}
+
+int32_t tiles_of(int64_t n) { return (int32_t)((n + kTileEntries - 1) / kTileEntries); }
+
+// Sorts the entries of the destinations [a.klo, a.klo + a.kspan) into the
+// result from entry `done` on, and returns how many they are.  all: they are
+// all entries, so that nothing is read back to learn it.  cnt: their number, as
+// soon as it is known.
+int64_t transpose_range(tr_ctx *ctx, Pass a, const tr_csx_t *out, int64_t done, bool all, int64_t &cnt) {
+    const int bits = bits_for(a.kspan), passes = (bits + kMaxDigitBits - 1) / kMaxDigitBits;
+    a.nbits = (bits + passes - 1) / passes;
+    const size_t cells = (size_t)a.ntiles << a.nbits;
+    Temp hist(ctx, sizeof(int32_t) * cells), offsets(ctx, sizeof(int64_t) * (cells + 1));
+    int64_t *off = (int64_t *)offsets.p;
+    a.hist = (int32_t *)hist.p;
+    a.off = off;
+    cnt = a.n;
+    if (!all) {
+        count_digits<true>(ctx, a, off);
+        cnt = read_scalar<int64_t>(ctx, off + cells);
+    }
+    const size_t n = (size_t)std::max<int64_t>(cnt, 1);
+    Temp keys(ctx, sizeof(int32_t) * n), r0(ctx, passes > 1 ? sizeof(Rec) * n : 1),
+        r1(ctx, passes > 2 ? sizeof(Rec) * n : 1);
+    a.okey = (int32_t *)keys.p;
+    a.oidx = out->idx_vec + done;
+    a.oval = out->val + done;
+    if (all) count_digits<true>(ctx, a, off);
+    a.out = (Rec *)r0.p;
+    if (cnt > 0) passes > 1 ? scatter<true, false>(ctx, a) : scatter<true, true>(ctx, a);
+    a.n = cnt;
+    a.ntiles = tiles_of(cnt);
+    for (int p = 1; p < passes && cnt > 0; ++p) {
+        a.shift = p * a.nbits;
+        a.in = (const Rec *)(p % 2 ? r0.p : r1.p);
+        a.out = (Rec *)(p % 2 ? r1.p : r0.p);
+        count_digits<false>(ctx, a, off);
+        p + 1 < passes ? scatter<false, false>(ctx, a) : scatter<false, true>(ctx, a);
+    }
+    TR_LAUNCH(ctx, "transpose_starts", k_segment_starts, div_up((uint64_t)a.kspan + 1, 256), 256, 0, a.okey,
+              (int32_t)cnt, done, a.klo, a.kspan, out->ptr_vec);
+    return cnt;
 }
 
 }  // namespace
@@ -289,75 +335,43 @@ int bits_for(int32_t n) {
 // m^T); its descriptor and storage are prepared by the caller and m is valid.
 //
 // Scratch: 20 bytes an entry (36 beyond 2^20 destinations) plus 12 << digit
-// bits a tile.  Where that cannot be had, the destinations are taken 1024 at a
-// time: one pass each, straight from the matrix to the result, for 4 bytes an
-// entry of the fullest 1024 and one read of the indices per 1024 destinations.
+// bits a tile.  Where that cannot be had, the destinations are taken in ranges
+// that are halved until one's entries fit, down to 1024 destinations (4 bytes
+// an entry, straight from the matrix to the result).  A range costs one read
+// of the matrix and a wait, so their number follows from the room that is
+// missing and not from the number of destinations; ranges grow again where
+// they held few entries.  (With room for 10 bytes an entry: 2 M entries over
+// 2^20 destinations 53.4 ms by 1024 destinations a range, now 0.44; 8 M over
+// 2^22 372 ms, now 0.83.)
 void launch_transpose(tr_ctx *ctx, const tr_csx_t *m, tr_csx_t *out) {
-    const int32_t P = ptrdim(m), O = otherdim(m);
+    const int64_t O = otherdim(m);
     if (m->nnz == 0) {
-        launch_fill_i32(ctx, out->ptr_vec, 0, (int64_t)O + 1);
+        launch_fill_i32(ctx, out->ptr_vec, 0, O + 1);
         return;
     }
     Pass a{};
     a.ptr = m->ptr_vec;
     a.idx = m->idx_vec;
     a.val = m->val;
-    a.oidx = out->idx_vec;
-    a.oval = out->val;
     a.n = m->nnz;
-    a.nseg = P;
-    a.ntiles = (int32_t)((m->nnz + kTileEntries - 1) / kTileEntries);
-    auto starts = [&](int32_t cnt, int64_t base, int32_t klo, int32_t n) {
-        TR_LAUNCH(ctx, "transpose_starts", k_segment_starts, div_up((uint64_t)n + 1, 256), 256, 0, a.okey, cnt, base,
-                  klo, n, out->ptr_vec);
-    };
-    const int bits = bits_for(O), passes = (bits + kMaxDigitBits - 1) / kMaxDigitBits;
-    const int digit = (bits + passes - 1) / passes;
-    const size_t nnz = (size_t)m->nnz, cells = (size_t)a.ntiles << digit;
-    try {
-        Temp hist(ctx, sizeof(int32_t) * cells), off(ctx, sizeof(int64_t) * (cells + 1));
-        Temp keys(ctx, sizeof(int32_t) * nnz), r0(ctx, passes > 1 ? sizeof(Rec) * nnz : 1),
-            r1(ctx, passes > 2 ? sizeof(Rec) * nnz : 1);
-        a.hist = (int32_t *)hist.p;
-        a.off = (int64_t *)off.p;
-        a.okey = (int32_t *)keys.p;
-        a.kspan = O;
-        a.nbits = digit;
-        for (int p = 0; p < passes; ++p) {
-            a.shift = p * digit;
-            a.in = (const Rec *)(p % 2 ? r0.p : r1.p);
-            a.out = (Rec *)(p % 2 ? r1.p : r0.p);
-            if (passes == 1) radix_pass<true, true>(ctx, a, (int64_t *)off.p);
-            else if (p == 0) radix_pass<true, false>(ctx, a, (int64_t *)off.p);
-            else if (p + 1 < passes) radix_pass<false, false>(ctx, a, (int64_t *)off.p);
-            else radix_pass<false, true>(ctx, a, (int64_t *)off.p);
-        }
-        starts((int32_t)m->nnz, 0, 0, O);
-        return;
-    } catch (const Error &e) {
-        if (e.code != TR_ERR_OOM || passes == 1) throw;
-    }
-    const size_t cells1 = (size_t)a.ntiles << kMaxDigitBits;
-    Temp hist(ctx, sizeof(int32_t) * cells1), off(ctx, sizeof(int64_t) * (cells1 + 1));
-    a.hist = (int32_t *)hist.p;
-    a.off = (int64_t *)off.p;
-    a.shift = 0;
-    a.nbits = kMaxDigitBits;
-    int64_t done = 0;
-    for (int64_t k = 0; k < O; k += kMaxDigits) {
+    a.nseg = ptrdim(m);
+    a.ntiles = tiles_of(m->nnz);
+    int64_t done = 0, span = O, refused = INT64_MAX;  // refused: entries of the least range that did not fit
+    for (int64_t k = 0; k < O;) {
         a.klo = (int32_t)k;
-        a.kspan = (int32_t)std::min<int64_t>(kMaxDigits, O - k);
-        TR_LAUNCH(ctx, "transpose_count", k_radix_count<true>, tile_blocks(a.ntiles), kThreads, 0, a);
-        scan::launch(ctx, scan::ArrayIn<int32_t>{a.hist}, (int64_t *)off.p, (int64_t)cells1, nullptr);
-        const int64_t cnt = read_scalar<int64_t>(ctx, a.off + cells1);
-        Temp keys(ctx, sizeof(int32_t) * (size_t)std::max<int64_t>(cnt, 1));
-        a.okey = (int32_t *)keys.p;
-        a.oidx = out->idx_vec + done;
-        a.oval = out->val + done;
-        if (cnt)
-            TR_LAUNCH(ctx, "transpose_scatter", (k_radix_scatter<true, true>), tile_blocks(a.ntiles), kThreads, 0, a);
-        starts((int32_t)cnt, done, a.klo, a.kspan);
-        done += cnt;
+        a.kspan = (int32_t)std::min(span, O - k);
+        int64_t cnt = 0;
+        try {
+            done += transpose_range(ctx, a, out, done, a.kspan == O, cnt);
+        } catch (const Error &e) {
+            if (e.code != TR_ERR_OOM || a.kspan <= kMaxDigits) throw;
+            if (cnt > 0) refused = std::min(refused, cnt);
+            span = kMaxDigits;
+            while (2 * span < a.kspan) span *= 2;
+            continue;
+        }
+        k += a.kspan;
+        if (cnt <= refused / 4) span *= 2;
     }
 }
 
