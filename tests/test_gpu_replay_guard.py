@@ -29,16 +29,19 @@ def _put_columns(ctx, d, idx):
 
 
 def _refused_then_valid(ctx, batch, da, a, b, changed_idx):
-    assert _exact(batch, a, b)
-    _put_columns(ctx, da, changed_idx)
-    batch.run()
-    with pytest.raises(TridentError) as e:
+    try:
+        assert _exact(batch, a, b)
+        _put_columns(ctx, da, changed_idx)
+        batch.run()
+        with pytest.raises(TridentError) as e:
+            batch.check()
+        assert e.value.code == TR_ERR_INVALID
+        _put_columns(ctx, da, a.idx)
+        batch.run()
         batch.check()
-    assert e.value.code == TR_ERR_INVALID
-    _put_columns(ctx, da, a.idx)
-    batch.run()
-    batch.check()
-    assert _exact(batch, a, b)
+        assert _exact(batch, a, b)
+    finally:
+        batch.close()
 
 
 @pytest.mark.parametrize("graph", [True, False])
@@ -54,6 +57,24 @@ def test_more_windows_than_planned(ctx, graph):
     da, db = ctx.upload(a), ctx.upload(b)
     batch = Batch(ctx, [da], [db], None, graph=graph)
     _refused_then_valid(ctx, batch, da, a, b, np.tile(np.arange(entries, 2 * entries), rows))
-    batch.close()
+    da.free()
+    db.free()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_rows_that_no_planned_launch_takes(ctx, graph):
+    """Short rows of 32 entries, the most that their kernel takes; then one row
+    of 48, which the plan has no launch for, and one of 16, so that every size
+    of the plan still fits."""
+    rng = np.random.default_rng(2)
+    rows, sets = 32768, 16  # B rows 4 s .. 4 s + 3 hold the columns of set s
+    b = _rows([4 * (k // 4) + np.arange(4) for k in range(4 * sets)], 4 * sets, rng)
+    planned = np.concatenate([[4 * s, 4 * s + 1] for s in range(8)])
+    a = _rows([planned] * rows, 4 * sets, rng)
+    more = np.concatenate([[4 * s, 4 * s + 1] for s in range(4)] + [[4 * s] for s in range(4, 12)])
+    less = np.arange(16)
+    da, db = ctx.upload(a), ctx.upload(b)
+    batch = Batch(ctx, [da], [db], None, graph=graph)
+    _refused_then_valid(ctx, batch, da, a, b, np.concatenate([more, less, a.idx[32:]]))
     da.free()
     db.free()

@@ -127,17 +127,23 @@ __global__ void k_guard_counts(Counters *__restrict__ cnt, const int32_t *__rest
 }
 
 // after the symbolic phase: every task's products start where the plan put
-// them (expect[t], expect[nt] = total), the heavy work lists fit and the
-// cursor total is the planned one; otherwise no numeric row runs
+// them (expect[t], expect[nt] = total), the heavy work lists fit, the cursor
+// total is the planned one and every row is of a kind that the plan has a
+// launch for (taken, mul_taken); otherwise no numeric row runs
 __global__ void k_guard_products(const TaskDev *__restrict__ tasks, int nt, const int64_t *__restrict__ rowptr,
                                  int32_t rows, const int64_t *__restrict__ expect, Counters *__restrict__ cnt,
                                  const int64_t *__restrict__ cbase, int32_t item_cap, int64_t cursor_cap,
-                                 int32_t *__restrict__ guard) {
+                                 uint32_t taken, int32_t *__restrict__ guard) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     int bad = cnt->overflow & 1;
     for (int t = 0; t <= nt && !bad; ++t)
         if (rowptr[t < nt ? tasks[t].row_base : rows] != expect[t]) bad = 1;
     if (cbase && cbase[item_cap] > cursor_cap) bad = 1;
+    for (int c = 0; c < kNumClasses; ++c)
+        if (cnt->cls[c] > 0 && !(taken >> c & 1u)) bad = 1;
+    for (int i = 0; i < 2; ++i)
+        if (cnt->short_rows[i] > 0 && !(taken >> (kShortRowsBit + i) & 1u)) bad = 1;
+    if (cnt->items > 0 && !(taken >> kItemsBit & 1u)) bad = 1;
     if (bad) atomicOr(guard, 1);
     if (*guard) {
         for (int c = 0; c < kNumClasses; ++c) cnt->cls[c] = 0;
@@ -331,7 +337,7 @@ void batch_body(tr_batch *b, bool capture) {
     if (guarded)
         TR_LAUNCH(ctx, "batch_guard", k_guard_products, 1, 64, 0, b->mp.d_tasks, b->nt, b->mp.rowptr,
                   b->mp.rows_total, b->expect_p, b->mp.cnt, b->mp.h.items > 0 ? b->mp.cbase : nullptr,
-                  b->mp.item_cap, b->mp.cursor_cap, b->guard);
+                  b->mp.item_cap, b->mp.cursor_cap, mul_taken(b->mp), b->guard);
     if (!capture) {
         int64_t ncur = 0;
         mul_read_totals(ctx, b->mp, &b->p_total, &ncur);

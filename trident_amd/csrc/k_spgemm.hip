@@ -2360,6 +2360,18 @@ void launch_sym_heavy(tr_ctx *ctx, MulPlan &pl, int cls, int cls2, int per_cu, b
               pl.items, pl.item_cap, pl.lists, pl.rows_total);
 }
 
+namespace {
+
+int32_t widest(const MulPlan &pl) {
+    int32_t n = 0;
+    for (const TaskDev &t : pl.h_tasks) n = std::max(n, t.n);
+    return n;
+}
+
+int heavy_pass_bits(int32_t max_n) { return max_n <= (1 << 18) ? 18 : max_n <= (1 << 19) ? 19 : kPassBits; }
+
+}  // namespace
+
 void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool capture) {
     LightBlocks lb;
     if (light_blocks(ctx, pl, false, lb)) {
@@ -2379,8 +2391,7 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
                   pl.d_tasks, pl.nt, pl.lists + (int64_t)kShortClass * pl.rows_total, pl.cnt, pl.rownnz);
     const int32_t nh = pl.h.cls[kHeavyClass] + pl.h.cls[kMidClass];
     if (nh) {
-        int32_t max_n = 0;
-        for (auto &t : pl.h_tasks) max_n = std::max(max_n, t.n);
+        const int32_t max_n = widest(pl);
         if (emit && !capture) {
             const HeavyLists cap = heavy_lists((int64_t)pl.h.heavy_flops, nh, max_n, pl.tune.window_entries,
                                                pl.tune.item_windows, item_flops(ctx, pl));
@@ -2398,7 +2409,7 @@ void mul_symbolic(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool emit, bool captu
         // widely in cost, and queued workgroups go to whichever CU frees
         // first (Galerkin 128^3: 12.9 -> 12.3 ms against one resident wave
         // of workgroups).
-        const int pb = max_n <= (1 << 18) ? 18 : max_n <= (1 << 19) ? 19 : kPassBits;
+        const int pb = heavy_pass_bits(max_n);
         // Up to 2^19 columns both classes share a kernel, the heaviest rows
         // first, in one launch: the lighter rows fill the end of the heavier
         // ones (R-MAT s17 1896 -> 1410 us, 15013 vertices 218 -> 179 us).
@@ -2427,8 +2438,7 @@ void mul_cursor_prep(tr_ctx *ctx, Workspace &ws, MulPlan &pl, bool capture) {
         pl.order_hist = (unsigned long long *)ws.get(S_ORDER_HIST, sizeof(unsigned long long) * kOrderBuckets);
     }
     const uint32_t og = cap_grid(div_up((uint64_t)pl.item_cap, 256), (int64_t)ctx->cu_count * 8);
-    int32_t maxn = 1;
-    for (const TaskDev &t : pl.h_tasks) maxn = std::max(maxn, t.n);
+    const int32_t maxn = widest(pl);
     int shift = 0;
     while (((int64_t)kOrderBuckets << shift) < (int64_t)maxn) ++shift;
     TR_LAUNCH(ctx, "item_order", k_fill_u64, div_up((uint64_t)kOrderBuckets, 256), 256, 0, pl.order_hist,
@@ -2487,9 +2497,7 @@ void launch_num_sort_as(tr_ctx *ctx, MulPlan &pl, int c, int32_t lo, Panel *pane
 
 // (column, position) keys of 32 bits hold every column
 bool narrow_keys(const MulPlan &pl) {
-    int32_t max_n = 0;
-    for (const TaskDev &t : pl.h_tasks) max_n = std::max(max_n, t.n);
-    return max_n <= 1 << (32 - kSortIdBits);
+    return widest(pl) <= 1 << (32 - kSortIdBits);
 }
 
 // class c of rows of up to NT * P products, those of more than lo entries
@@ -2539,6 +2547,17 @@ void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *dp, int np) {
             TR_LAUNCH(ctx, "num_heavy", (k_num_heavy_wg<2048, kSmallNT>), grid, kSmallNT, 0, pl.d_tasks, pl.nt, pl.items,
                       pl.cnt, pl.wins, pl.order, pl.cbase, pl.cursors, pl.rowptr, dp, np, pl.tune.dense_width);
     }
+}
+
+// A class that had no row gets no launch; the two heavy classes share theirs
+// where they share a kernel.
+uint32_t mul_taken(const MulPlan &pl) {
+    uint32_t m = 0;
+    for (int c = 0; c < kNumClasses; ++c) m |= pl.h.cls[c] > 0 ? 1u << c : 0u;
+    if (heavy_pass_bits(widest(pl)) != kPassBits && (m & (1u << kHeavyClass | 1u << kMidClass)))
+        m |= 1u << kHeavyClass | 1u << kMidClass;
+    for (int i = 0; i < 2; ++i) m |= pl.h.short_rows[i] > 0 ? 1u << (kShortRowsBit + i) : 0u;
+    return m | (pl.h.items > 0 ? 1u << kItemsBit : 0u);
 }
 
 void mul_check(tr_ctx *ctx, MulPlan &pl) {

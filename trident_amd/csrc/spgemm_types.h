@@ -203,5 +203,9 @@ void mul_read_task_offsets(tr_ctx *ctx, MulPlan &pl, int64_t *host);
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np);
 void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np);
 void mul_check(tr_ctx *ctx, MulPlan &pl);  // reads the consistency flags (eager)
+// The rows that the plan's launches take (after its counts are read): a bit per
+// class, then one per part of short_rows, then one for the heavy items.
+constexpr int kShortRowsBit = kNumClasses, kItemsBit = kNumClasses + 2;
+uint32_t mul_taken(const MulPlan &pl);
 
 }  // namespace tr
