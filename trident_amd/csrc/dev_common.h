@@ -140,19 +140,6 @@ __device__ __forceinline__ uint32_t hash_slot(int32_t key, uint32_t log2T) {
     return ((uint32_t)key * 0x9E3779B1u) >> (32u - log2T);
 }
 
-// Largest lane l with excl[l] <= x, given non-decreasing per-lane `excl`
-// (excl[0] == 0).  Binary search over lanes through shuffles.
-__device__ __forceinline__ int owner_lane(int64_t excl, int64_t x) {
-    int lo = 0;
-#pragma unroll
-    for (int step = 32; step > 0; step >>= 1) {
-        int probe = lo + step;
-        int64_t v = __shfl(excl, probe & 63, kWave);
-        if (probe < kWave && v <= x) lo = probe;
-    }
-    return lo;
-}
-
 template <int kSize, int kStride, typename V>
 __device__ __forceinline__ void bitonic_step(int32_t &k, V &v, int l) {
     const int32_t pk = lane_xor<kStride>(k);

@@ -1116,12 +1116,6 @@ __global__ __launch_bounds__(256) void k_item_scatter(const Item *__restrict__ i
     }
 }
 
-// panel p starts at global row row_begin: its first entry's global offset
-__global__ void k_panel_bases(Panel *__restrict__ panels, int np, const int64_t *__restrict__ rowptr) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < np) panels[p].nnz_begin = rowptr[panels[p].row_begin];
-}
-
 // int32 row pointers of the tile that holds global rows [r0, r0 + n], rebased,
 // and its entry of the panel table
 __global__ void k_tile_ptr(const int64_t *__restrict__ rowptr, int32_t r0, int32_t n, int32_t *__restrict__ ptr,
@@ -2478,10 +2472,6 @@ void mul_read_task_offsets(tr_ctx *ctx, MulPlan &pl, int64_t *host) {
               (int64_t *)ctx->pinned);
     TR_HIP(hipStreamSynchronize(ctx->stream));
     std::memcpy(host, ctx->pinned, sizeof(int64_t) * ((size_t)pl.nt + 1));
-}
-
-void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np) {
-    TR_LAUNCH(ctx, "panel_bases", k_panel_bases, div_up((uint64_t)np, 64), 64, 0, d_panels, np, pl.rowptr);
 }
 
 namespace {

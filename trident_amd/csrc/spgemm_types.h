@@ -12,7 +12,6 @@
 namespace tr {
 
 // tuning constants
-constexpr int kLightMaxFCap = 1024; // largest light/heavy cut (light tables reach 2048 slots)
 constexpr int kNumLight = 6;       // light classes: up to 32 << c multiplications, c < kNumLight
 constexpr int kHeavyClass = kNumLight;      // heavy rows with more than kMidMaxF multiplications
 constexpr int kMidClass = kNumLight + 1;    // heavy rows up to kMidMaxF multiplications
@@ -124,7 +123,6 @@ struct MulPlan {
     unsigned long long *order_hist = nullptr;
     int64_t cursor_cap = 0;
     int64_t *scan_tmp = nullptr;  // owned scan temp (graph mode)
-    size_t scan_tmp_bytes = 0;
     tr_tuning_t tune{};           // the context's tuning when the plan was set up
 };
 
@@ -201,7 +199,6 @@ void mul_read_totals(tr_ctx *ctx, MulPlan &pl, int64_t *nnz, int64_t *ncur);
 // The first product entry of every task, and the end (nt + 1 values).
 void mul_read_task_offsets(tr_ctx *ctx, MulPlan &pl, int64_t *host);
 void mul_numeric(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np);
-void mul_panel_bases(tr_ctx *ctx, MulPlan &pl, Panel *d_panels, int np);
 void mul_check(tr_ctx *ctx, MulPlan &pl);  // reads the consistency flags (eager)
 // The rows that the plan's launches take (after its counts are read): a bit per
 // class, then one per part of short_rows, then one for the heavy items.
