@@ -163,8 +163,9 @@ int tr_spgemm_flops(tr_ctx_t ctx, const tr_csx_t *A, const tr_csx_t *B, int64_t 
  *    heavy (column-windowed) path, [64, 1024];
  *  - window_entries: heavy window packing quantum H (a window holds at most
  *    H + 127 entries), [64, 3 * heavy_table / 4 - 127];
- *  - item_windows: heavy windows per work item, [1, 64] (rows of more than
- *    2048 entries use a quarter of it, at least 1);
+ *  - item_windows: heavy windows per work item at most, [1, 64] (rows of more
+ *    than 2048 entries use a quarter of it, at least 1); an item takes fewer
+ *    where they would hold more multiplications than the product's even share;
  *  - heavy_table: slots of the heavy numeric table, 2048 (256-thread
  *    workgroups) or 4096 (512-thread workgroups);
  *  - dense_width: heavy windows spanning at most this many columns use a

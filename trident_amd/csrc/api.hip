@@ -364,7 +364,8 @@ static int guarded(tr_ctx *ctx, F &&body) {
 extern "C" {
 
 const char *tr_version(void) {
-    return "trident_hip gfx950: light rows wave hash, heavy rows bitmap windows + 2048-slot workgroup tables, merge-path add";
+    return "trident_hip gfx950: light rows sorted in registers, heavy rows bitmap windows + 2048-slot workgroup tables, "
+           "unit merge add";
 }
 
 int tr_ctx_create(tr_ctx_t *out, int device, void *hip_stream) {

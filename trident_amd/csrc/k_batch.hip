@@ -11,7 +11,7 @@
 //   2. the product P_t = A_t * B_t through the multiply pipeline, all tasks
 //      in one task table, so every kernel launch covers all tile products
 //      (uneven products fill the GPU together instead of one after another);
-//   3. the accumulation C_t = C_in_t + P_t through the merge-path add, again
+//   3. the accumulation C_t = C_in_t + P_t through the sorted add, again
 //      one launch per phase over all tasks.
 // The plan step runs the whole stage once eagerly (host reads size every
 // list and output), then captures the same launch sequence, with every size

@@ -252,8 +252,9 @@ __device__ __forceinline__ uint64_t word_span(int32_t lo, int32_t hi, int r) {
 // front and Y descending from the back are a bitonic sequence, so the merge is
 // 9 exchange steps in registers, 3 between a lane's own 8 keys and 6 between
 // lanes: no search, no LDS and no barrier, and a wave reads X and Y in whole
-// lines.  Vector instructions bound it (85% of the cycles; a block that
-// searched each thread's merge split in LDS: 627 us where this takes 221).
+// lines.  Vector instructions bound it (78% of the cycles, scalar ones 64%; a
+// block that searched each thread's merge split in LDS: 627 us where this takes
+// 221).
 // Only a unit with row ends goes through LDS, for the entries' rows.
 // K: 32-bit keys hold 513 rows and 21 bits of column, which is all that the
 // exchanges move; wider tiles take 64-bit keys.

@@ -5,27 +5,31 @@
 //
 //  1. row analysis   flops_i = sum_{k in A_i} nnz(B_k), summed in equal units
 //                    of entries by the pass that also checks the operands
-//                    (k_check.hip); rows are binned by flops (empty / light
-//                    classes by hash table size / heavy).
+//                    (k_check.hip); rows are binned by flops (empty / six
+//                    light classes / short rows / two heavy classes).
 //  2. symbolic       light rows (flops <= the tuned cut): one wave per row, LDS
-//                    open-addressing hash of column keys;
-//                    heavy rows: one 1024-thread block per row, a bitmap of
-//                    2^20 columns in LDS (128 KiB of the 160 KiB), popcounted
-//                    per 128-column fine block; the block packs fine blocks
-//                    into column windows of at most H+127 entries and
-//                    appends them to a device work list.
+//                    open-addressing hash of column keys; short rows eight to
+//                    a wave;
+//                    heavy rows: one 512- or 1024-thread block per row, a
+//                    bitmap of 2^18, 2^19 or 2^20 columns in LDS (128 KiB of
+//                    the 160 KiB at most), popcounted per 128-column fine
+//                    block; the block packs fine blocks into column windows of
+//                    at most H+127 entries and appends them to a device work
+//                    list (heavy_items.h).
 //  3. scan           row counts -> 64-bit row offsets; C is cut into int32
 //                    tiles (panels) when it exceeds INT32_MAX entries.
 //  4. numeric        light rows: all products of a row at once, sorted in
 //                    registers by (column, position in A-order) and summed
-//                    run by run;
+//                    run by run; short rows of at most 32 entries eight to a
+//                    wave, B row after B row;
 //                    compact heavy rows (at most 128 entries): one wave per
 //                    row, LDS hash of (key, fp64), compacted and sorted;
 //                    heavy rows: one workgroup per item (a run of windows of
 //                    one row) sharing one LDS table per window, products of
-//                    the window flattened over the workgroup in A-order,
-//                    column conflicts inside a step applied in thread (= A)
-//                    order, sorted ranks from a presence bitmap.
+//                    the window flattened in A-order into groups of 64, which
+//                    its waves prepare together and add in turn, lanes that
+//                    share a column one after the other; sorted ranks from a
+//                    presence bitmap.
 //
 // Every output entry therefore receives c = fma(a_ik, b_kj, c) in the order
 // of A's stored entries, starting from +0.0: the results are bit-identical to

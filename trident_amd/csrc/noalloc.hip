@@ -4,8 +4,9 @@
 // loops, harnesses that forbid hipMalloc.  tr_spadd_into_noalloc is
 // tr_spadd_into (the double-buffer add of sp_mma_hybrid,
 // include/cusparse_helpers.cuh:708-739) with every temporary of the add
-// (unit splits, counts and offsets, scan partials, merge bits) carved from one file-scope device array instead of the
-// context's pool.  Inputs and outputs are still the caller's.
+// (unit splits, counts and offsets, scan partials, merge bits) carved from one
+// file-scope device array instead of the context's pool.  Inputs and outputs
+// are still the caller's.
 //
 // The array is kNoallocBytes per GPU, held for the life of the process by
 // every GPU the library runs on.  Host code never uses the array's name as
@@ -13,9 +14,9 @@
 // address is looked up once per device with hipGetSymbolAddress while that
 // device is current (noalloc_init, called from tr_ctx_create), and kernels
 // receive that address.  Every call on one GPU shares the array and it keeps
-// the last call's contents, so everything that must start at zero is cleared
-// by a fill kernel on the call's stream, and calls that overlap on one GPU
-// (two streams or threads at once) race.
+// the last call's contents, of which a call reads nothing that it has not
+// written itself; calls that overlap on one GPU (two streams or threads at
+// once) race.
 #include <mutex>
 #include <string>
 

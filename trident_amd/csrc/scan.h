@@ -8,7 +8,8 @@
 // entries) launches and dependent latencies, not bandwidth.  A wave owns 1024
 // consecutive items and loads its 16 groups of 64 together; the groups are
 // scanned in registers and joined by one barrier, where the kernels before
-// walked 16 groups with three barriers each (11 us at any size, 4 us now).
+// walked 16 groups with three barriers each (11 us for their last launch alone
+// at any size; the one launch now 6.5 us for 1024 items, 8.2 for 15013).
 // One workgroup does up to 16384 items in one launch (three before); up to
 // kScanDirect tiles every tile sums the tile totals before it by itself (two
 // launches); beyond, a third launch scans the totals, so that the totals read
