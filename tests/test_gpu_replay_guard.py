@@ -47,8 +47,8 @@ def _refused_then_valid(ctx, batch, da, a, b, changed_idx):
 @pytest.mark.parametrize("graph", [True, False])
 def test_more_windows_than_planned(ctx, graph):
     """Heavy rows that met B rows of 3 entries meet B rows of 2000 instead:
-    their windows and items are ten times what the work lists hold, so rows
-    are refused and the lists' counts run past their capacity."""
+    their windows and items are ten times what the work lists hold, so that
+    most rows are refused and what the lists hold must not be used."""
     rng = np.random.default_rng(1)
     ncols, rows, entries = 100000, 64, 400
     b = _rows([np.sort(rng.choice(ncols, 3 if k < entries else 2000, replace=False)) for k in range(2 * entries)],

@@ -972,6 +972,10 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
                 const int32_t ib = atomicAdd(&cnt->items, nitems);
                 if (wb + nwin > win_cap || ib + nitems > item_cap) {
                     atomicOr(&cnt->overflow, 1);
+                    // taken back, so that refused rows, however many, never
+                    // carry a count past 2^31 (an overflowed list is not read)
+                    atomicSub(&cnt->windows, nwin);
+                    atomicSub(&cnt->items, nitems);
                     sh_wbase = -1;
                 } else {
                     sh_wbase = wb;
@@ -1009,8 +1013,8 @@ __global__ __launch_bounds__(NTH, (PB <= 18 || (PB == 19 && NTH == 1024)) ? 8 : 
 
 // Items of the work list.  A list that would not fit (a batch's replay on
 // operands with another sparsity pattern than the planned one) holds none:
-// its count runs on past its capacity, and refused rows leave gaps that were
-// never written.
+// refused rows leave gaps that were never written, and rows that came while
+// another was refused may lie over each other.
 __device__ __forceinline__ int32_t listed_items(const Counters *__restrict__ cnt) {
     return (cnt->overflow & 1) ? 0 : cnt->items;
 }
